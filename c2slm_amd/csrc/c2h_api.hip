@@ -22,7 +22,6 @@ using namespace c2h;
 namespace {
 
 constexpr int kStateRing = 256;
-constexpr int PF_ATT_SUB = 16;  // batch tokens per long-context attention launch
 
 struct Tensor {
   uint8_t* q = nullptr;
@@ -91,9 +90,8 @@ struct c2h_ctx {
   bool use_graphs = true;
   size_t attn_lds = 0;
   int att_split = 0;     // positions attended up to which k_attn_core runs
-  int pfa_max_pos = 0;   // prefill passes ending at or below this many positions run k_pf_attn
   bool long_attn = false;
-  float* att_sc = nullptr;  // [PF_ATT_SUB][n_heads][sc_ld] scores / probabilities
+  float* att_sc = nullptr;  // [n_heads][sc_ld] scores / probabilities
   float* att_bmax = nullptr;
   int att_sc_ld = 0, att_n_blk = 0;
   int32_t seq_len = 0;   // KVCache.SeqLen (engine/kvcache.go:25-47)
@@ -609,15 +607,15 @@ AttnCoreParams attn_params(c2h_ctx* c, int layer) {
   return A;
 }
 
-// Long-context attention of `ntok` query tokens (rows tok0..): scores over
-// every block of the context, softmax, AV.  Blocks past a token's context
-// return at once, so the grid covers max_ctx and graphs replay at any pos.
-void enqueue_attn_long(c2h_ctx* c, const AttnCoreParams& A, int ntok) {
+// Long-context attention of a decode step: scores over every block of the
+// context, softmax, AV.  Blocks past the token's context return at once, so
+// the grid covers max_ctx and graphs replay at any pos.
+void enqueue_attn_long(c2h_ctx* c, const AttnCoreParams& A) {
   const c2h_model_desc& D = c->desc;
-  hipLaunchKernelGGL(k_attn_scores, dim3(c->att_n_blk, D.n_kv_heads, ntok), dim3(256), 0, c->stream, A);
-  hipLaunchKernelGGL(k_attn_softmax, dim3(D.n_heads, ntok), dim3(1024),
+  hipLaunchKernelGGL(k_attn_scores, dim3(c->att_n_blk, D.n_kv_heads), dim3(256), 0, c->stream, A);
+  hipLaunchKernelGGL(k_attn_softmax, dim3(D.n_heads), dim3(1024),
                      (size_t)attn_softmax_lds_floats(D.max_ctx) * 4, c->stream, A);
-  hipLaunchKernelGGL(k_attn_av, dim3(D.n_kv_heads * ATT_AV_SLICES, ntok), dim3(ATT_AV_THREADS),
+  hipLaunchKernelGGL(k_attn_av, dim3(D.n_kv_heads * ATT_AV_SLICES), dim3(ATT_AV_THREADS),
                      (size_t)ATT_AV_LDS_FLOATS * 4, c->stream,
                      A);
 }
@@ -744,7 +742,7 @@ void enqueue_attn(c2h_ctx* c, int l, int form) {
                        c->stream, A);
   }
   else if (form == ATT_FORM_LONG)
-    enqueue_attn_long(c, A, 1);
+    enqueue_attn_long(c, A);
   else {
     A.xcd_map = D.n_kv_heads <= ATT_XCDS ? 1 : 0;
     const dim3 xgrid(ATT_XCDS * (D.n_heads / D.n_kv_heads));
@@ -1431,6 +1429,13 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
   for (const void* k : {(const void*)k_pf_gemm_q6<MODE_BIAS, 2>, (const void*)k_pf_gemm_q6<MODE_RESID, 2>})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, PF_Q6_LDS_MAX) != hipSuccess)
       return bail(fail(c, C2H_ERR_HIP, "prefill Q6_K GEMM LDS attribute"));
+  for (const void* k : {(const void*)k_pf_gemm_f<MODE_BIAS>, (const void*)k_pf_gemm_f<MODE_RESID>,
+                        (const void*)k_pf_gemm_q50<MODE_BIAS>, (const void*)k_pf_gemm_q50<MODE_RESID>})
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, PF_F_LDS_MAX) != hipSuccess)
+      return bail(fail(c, C2H_ERR_HIP, "prefill GEMM LDS attribute"));
+  for (const void* k : {(const void*)k_pf_attn<64>, (const void*)k_pf_attn<128>})
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PFA_LDS_MAX) != hipSuccess)
+      return bail(fail(c, C2H_ERR_HIP, "prefill attention LDS attribute"));
   if (D.head_dim == 128) {  // k_attn_h128 at every T: the scores of max_ctx positions in LDS
     c->attn_lds = (size_t)attn_h128_lds_floats(D.max_ctx) * 4;
     if (c->attn_lds > 152u * 1024)
@@ -1460,17 +1465,6 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
             hipFuncSetAttribute((const void*)attn_block_f_kernel(form), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)std::max(c->attn_lds, (size_t)gemv_f_lds_floats(D.n_embd) * 4)) != hipSuccess)
           return bail(fail(c, C2H_ERR_HIP, "attention LDS attribute"));
-      const void* pff[] = {(const void*)k_pf_gemm_f<MODE_BIAS>, (const void*)k_pf_gemm_f<MODE_RESID>,
-                           (const void*)k_pf_gemm_q50<MODE_BIAS>, (const void*)k_pf_gemm_q50<MODE_RESID>};
-      for (const void* k : pff)
-        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, PF_F_LDS_MAX) != hipSuccess)
-          return bail(fail(c, C2H_ERR_HIP, "prefill GEMM LDS attribute"));
-      // k_pf_attn keeps the scores of up to att_split positions per token in LDS
-      c->pfa_max_pos = c->att_split;
-      while (c->pfa_max_pos > 1 && (size_t)pfa_lds_floats(c->pfa_max_pos - 1) * 4 > 152u * 1024) --c->pfa_max_pos;
-      if (hipFuncSetAttribute((const void*)k_pf_attn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              pfa_lds_floats(c->pfa_max_pos - 1) * 4) != hipSuccess)
-        return bail(fail(c, C2H_ERR_HIP, "prefill attention LDS attribute"));
     }
     if (c->long_attn) {
       if (D.max_ctx > ATT_LONG_MAX_CTX)
@@ -1480,8 +1474,8 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
         return bail(fail(c, C2H_ERR_UNSUPPORTED, "more than %d query heads per KV head", ATT_MAX_QPKV));
       c->att_sc_ld = (D.max_ctx + 3) & ~3;
       c->att_n_blk = (D.max_ctx + ATT_SB - 1) / ATT_SB;
-      if ((rc = dalloc(c, &c->att_sc, (size_t)PF_ATT_SUB * D.n_heads * c->att_sc_ld * 4)) ||
-          (rc = dalloc(c, &c->att_bmax, (size_t)PF_ATT_SUB * D.n_heads * c->att_n_blk * 4)))
+      if ((rc = dalloc(c, &c->att_sc, (size_t)D.n_heads * c->att_sc_ld * 4)) ||
+          (rc = dalloc(c, &c->att_bmax, (size_t)D.n_heads * c->att_n_blk * 4)))
         return bail(rc);
       if (hipFuncSetAttribute((const void*)k_attn_softmax, hipFuncAttributeMaxDynamicSharedMemorySize,
                               attn_softmax_lds_floats(D.max_ctx) * 4) != hipSuccess ||
@@ -1747,14 +1741,49 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
 
 typedef void (*PFNormKernel)(PFNormParams);
 typedef void (*PFQuantKernel)(PFQuantParams);
-PFNormKernel pf_norm_kernel(int nb) { return nb == 3 ? k_pf_norm_quant<3> : k_pf_norm_quant<4>; }
+// The row widths c2h_create accepts (gemv_row_kernel's).
+PFNormKernel pf_norm_kernel(int nb) {
+  switch (nb) {
+    case 3: return k_pf_norm_quant<3>;
+    case 4: return k_pf_norm_quant<4>;
+    case 6: return k_pf_norm_quant<6>;
+    default: return k_pf_norm_quant<8>;
+  }
+}
 PFQuantKernel pf_quant_kernel(int nb) {
   switch (nb) {
     case 3: return k_pf_quant<3>;
     case 4: return k_pf_quant<4>;
+    case 6: return k_pf_quant<6>;
+    case 8: return k_pf_quant<8>;
     case 12: return k_pf_quant<12>;
-    default: return k_pf_quant<19>;
+    case 19: return k_pf_quant<19>;
+    case 24: return k_pf_quant<24>;
+    case 35: return k_pf_quant<35>;
+    default: return k_pf_quant<43>;
   }
+}
+
+// Query tokens per k_pf_attn workgroup: PFA_TB while a block's scores fit
+// the LDS and the blocks fill the GPU (a workgroup's chains are as long
+// with one token as with sixteen, its exps and its LDS grow with them),
+// down to one.
+int pf_attn_tokens(int n_heads, int m, int pmax) {
+  int tb = PFA_TB;
+  while (tb > 4 && n_heads * ((m + tb - 1) / tb) < PFA_MIN_WG) tb /= 2;
+  while (tb > 1 && pfa_lds_bytes(tb, pmax) > PFA_LDS_MAX) tb /= 2;
+  return tb;
+}
+
+// Whether prompts run the batched kernels.  A Q5_0 ffn_down wider than
+// k_pf_gemm_f's workgroup takes (its LDS, one thread per block of a row)
+// leaves one forward per token.
+bool pf_batched(const c2h_ctx* c) {
+  if (c->desc.head_dim == 64) return true;
+  for (const Layer& L : c->layers)
+    if (float_input(L.wd.type) && (pf_gemm_f_lds_bytes(c->desc.n_ff) > PF_F_LDS_MAX || c->desc.n_ff / 32 > 256))
+      return false;
+  return true;
 }
 
 // One pass of up to PF_MAX tokens at positions pos0.. (engine.Forward per
@@ -1793,16 +1822,21 @@ int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
       N.nb = nb_k(E);
       N.out = q8;
       N.xn = p.xn;
-      hipLaunchKernelGGL(pf_norm_kernel(nb_k(E)), dim3(m_pad), dim3(256), norm_lds, c->stream, N);
+      hipLaunchKernelGGL(pf_norm_kernel(nb_k(E)), dim3(m_pad), dim3(pf_norm_threads(nb_k(E))), norm_lds, c->stream, N);
     }
     pf_gemm(c, m, m_pad, nb_k(E), MODE_BIAS, {&L.wq, &L.wk, &L.wv}, {p.q, p.k, p.v}, {L.bq, L.bk, L.bv},
             {E, KV, KV}, p.xn, E, E);
     {
       PFRopeParams R;
       memset(&R, 0, sizeof(R));
+      R.q = p.q;
+      R.q_ld = E;
       R.k = p.k;
       R.v = p.v;
       R.ld = KV;
+      R.q_norm = L.q_norm;
+      R.k_norm = L.k_norm;
+      R.eps = D.rms_eps;
       R.kv = c->kv;
       R.rope_cos = c->rope_cos;
       R.rope_sin = c->rope_sin;
@@ -1811,36 +1845,25 @@ int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
       R.m = m;
       R.layer = l;
       R.n_layers = D.n_layers;
+      R.n_heads = D.n_heads;
       R.n_kv_heads = D.n_kv_heads;
       R.max_ctx = D.max_ctx;
-      hipLaunchKernelGGL(k_pf_rope_store, dim3(m, D.n_kv_heads), dim3(64), 0, c->stream, R);
+      const size_t lds = (L.q_norm || L.k_norm) ? pf_qk_lds_bytes(D.n_heads + D.n_kv_heads, D.head_dim) : 0;
+      hipLaunchKernelGGL(D.head_dim == 64 ? k_pf_qk<64> : k_pf_qk<128>, dim3(m), dim3(256), lds, c->stream, R);
     }
     {  // causal attention of every token (its K/V and the earlier ones are stored)
       AttnCoreParams A = attn_params(c, l);
       A.q = p.q;
-      A.k = p.k;
-      A.v = p.v;
       A.out = p.attn;
       A.q_ld = E;
-      A.kv_ld = KV;
       A.out_ld = E;
-      A.store_kv = 0;
-      if (pos0 + m <= c->att_split && pos0 + m <= c->pfa_max_pos) {
-        // blocks of PFA_TB query tokens per head, longest first, K/V chunks shared by the block
-        A.n_tok = m;
-        A.sc_ld = pfa_sc_ld(pos0 + m - 1);
-        hipLaunchKernelGGL(k_pf_attn, dim3(D.n_heads * ((m + PFA_TB - 1) / PFA_TB)), dim3(256),
-                           (size_t)pfa_lds_floats(pos0 + m - 1) * 4, c->stream, A);
-      } else if (pos0 + m <= c->att_split) {
-        const size_t lds = (size_t)attn_lds_floats(pos0 + m) * 4;
-        hipLaunchKernelGGL(k_attn_core<ATT_TIER_ANY>, dim3(D.n_heads / D.n_kv_heads, D.n_kv_heads, m), dim3(256), lds,
-                           c->stream, A.state, A.kv, A.q, A.k, A.v, attn_dims(A, D.n_heads / D.n_kv_heads), A.max_ctx, A);
-      } else {
-        for (int t0 = 0; t0 < m; t0 += PF_ATT_SUB) {
-          A.tok0 = t0;
-          enqueue_attn_long(c, A, std::min(PF_ATT_SUB, m - t0));
-        }
-      }
+      A.n_tok = m;
+      const int pmax = pos0 + m - 1;
+      A.tok_blk = pf_attn_tokens(D.n_heads, m, pmax);
+      A.sc_ld = pfa_sc_ld(pmax);
+      hipLaunchKernelGGL(D.head_dim == 64 ? k_pf_attn<64> : k_pf_attn<128>,
+                         dim3(D.n_heads * ((m + A.tok_blk - 1) / A.tok_blk)), dim3(4 * D.head_dim),
+                         pfa_lds_bytes(A.tok_blk, pmax), c->stream, A);
     }
     {
       PFQuantParams Q{p.attn, E, m, q8};
@@ -1858,7 +1881,7 @@ int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
       N.nb = nb_k(E);
       N.out = q8;
       N.xn = p.xn;
-      hipLaunchKernelGGL(pf_norm_kernel(nb_k(E)), dim3(m_pad), dim3(256), norm_lds, c->stream, N);
+      hipLaunchKernelGGL(pf_norm_kernel(nb_k(E)), dim3(m_pad), dim3(pf_norm_threads(nb_k(E))), norm_lds, c->stream, N);
     }
     pf_gemm(c, m, m_pad, nb_k(E), MODE_BIAS, {&L.wg, &L.wu}, {p.g, p.u}, {nullptr, nullptr}, {F, F}, p.xn, E, E);
     hipLaunchKernelGGL(k_pf_swiglu, dim3((F + 255) / 256, m), dim3(256), 0, c->stream, p.g, p.u, p.h, F, m);
@@ -1894,9 +1917,9 @@ int c2h_prefill(c2h_ctx* c, const int32_t* tokens, int32_t n, int32_t pos0, floa
   if (pos0 < 0 || (int64_t)pos0 + n > c->desc.max_ctx)
     return fail(c, C2H_ERR_RANGE, "positions [%d, %d) outside [0, %d)", pos0, pos0 + n, c->desc.max_ctx);
   if (n == 0) return C2H_OK;
-  if (c->desc.head_dim != 64) {
-    // no batched prefill kernels at this head_dim: one forward graph per
-    // token, as engine.IngestFrom runs Forward per token (c2slm.go:103-114)
+  if (!pf_batched(c)) {
+    // one forward graph per token, as engine.IngestFrom runs Forward per
+    // token (c2slm.go:103-114)
     if ((rc = build_graphs(c))) return rc;
     for (int i = 0; i < n; ++i) {
       C2hState s;

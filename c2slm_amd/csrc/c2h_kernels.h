@@ -252,7 +252,8 @@ struct AttnCoreParams {
   float* bmax;
   int sc_ld;    // (k_pf_attn: the row stride of its LDS scores, pfa_sc_ld)
   int n_blk;
-  int n_tok;    // k_pf_attn: query tokens of the prefill pass
+  int n_tok;    // k_pf_attn: query tokens of the prefill pass, and of a workgroup
+  int tok_blk;
   // k_attn_core: 1 = the grid is (ATT_XCDS * qpkv, 1, tokens), n_kv_heads
   // <= ATT_XCDS, and workgroup L serves KV head L % ATT_XCDS, query head
   // L / ATT_XCDS, so the workgroups of one KV head share an XCD and its L2
@@ -263,17 +264,17 @@ struct AttnCoreParams {
 constexpr int ATT_XCDS = 8;
 
 // Causal attention of a prefill pass (k_pf_attn): one workgroup per query
-// head and block of PFA_TB query tokens, K and V staged through LDS in
-// chunks of PFA_CH positions shared by the block's tokens.
-constexpr int PFA_TB = 8;
-constexpr int PFA_WAVES_PER_EU = 3;  // occupancy the register budget is sized for (three workgroups per CU)
-constexpr int PFA_CH = 128;
-constexpr int PFA_KPAD = 68;  // floats per staged K row (64 + 4: conflict-free row reads)
-// Row stride (floats) of the block's scores for positions up to pmax.
+// head and block of tok_blk <= PFA_TB query tokens, their scores in LDS.
+constexpr int PFA_TB = 16;
+// fewer tokens per workgroup below this many workgroups (one per CU)
+constexpr int PFA_MIN_WG = 256;
+// Row stride (floats) of the block's scores for positions up to pmax: 4 mod
+// 64, so that 16 rows of four consecutive floats lie in different banks.
 __host__ __device__ inline int pfa_sc_ld(int pmax) { return ((pmax + 1 + 63) & ~63) + 4; }
-// Dynamic LDS of k_pf_attn, in floats: K chunk (V chunk aliases it) | q of
-// the block's tokens | scores.
-__host__ __device__ inline int pfa_lds_floats(int pmax) { return PFA_CH * PFA_KPAD + PFA_TB * 64 + PFA_TB * pfa_sc_ld(pmax); }
+__host__ __device__ inline size_t pfa_lds_bytes(int tok_blk, int pmax) { return (size_t)tok_blk * pfa_sc_ld(pmax) * 4; }
+// one token's scores of the longest context (head_dim 128: up to 38,848
+// positions) fit with the kernel's static LDS
+constexpr size_t PFA_LDS_MAX = 156 * 1024;
 
 // Dynamic LDS of k_attn_h128 (head_dim 128), in floats: the scores of every
 // position up to max_ctx, then (k_attn_h128<H128_VCH>) two chunks of
@@ -378,20 +379,26 @@ struct PFGemmFParams {
   PFJob jobs[3];
 };
 
-// Per token and KV head: RoPE(k), then K/V stored at pos0 + t.
+// Per token: [QK-norm] RoPE of q (in place) and k, K/V stored at pos0 + t.
 struct PFRopeParams {
+  float* q;
+  int q_ld;
   const float* k;
   const float* v;
   int ld;
+  const float* q_norm;  // head_dim floats each, nullptr: none
+  const float* k_norm;
+  float eps;
   float* kv;
   const float* rope_cos;
   const float* rope_sin;
   int rope_len;
   int pos0;
   int m;
-  int layer, n_layers, n_kv_heads, max_ctx;
+  int layer, n_layers, n_heads, n_kv_heads, max_ctx;
 };
-
+// Dynamic LDS of k_pf_qk where the layer has QK-norms, in bytes.
+__host__ __device__ inline size_t pf_qk_lds_bytes(int heads, int hd) { return (size_t)heads * (hd + 2) * 4; }
 
 struct VocabParams {
   WeightRef w;
@@ -477,7 +484,10 @@ __global__ void k_attn_softmax(AttnCoreParams P);
 __global__ void k_attn_av(AttnCoreParams P);
 template <int VCH>
 __global__ void k_attn_h128(AttnCoreParams P);
-__global__ void k_pf_attn(AttnCoreParams P);
+template <int HD>
+__global__ void k_pf_attn(AttnCoreParams P);  // 4 HD threads
+// threads of k_pf_norm_quant: one float4 of the row each
+__host__ __device__ constexpr int pf_norm_threads(int nb) { return nb <= 4 ? 256 : 512; }
 template <int NB>
 __global__ void k_pf_norm_quant(PFNormParams P);
 template <int NB>
@@ -512,7 +522,8 @@ template <int MODE>
 __global__ void k_pf_gemm_f(PFGemmFParams P);
 template <int MODE>
 __global__ void k_pf_gemm_q50(PFGemmFParams P);
-__global__ void k_pf_rope_store(PFRopeParams P);
+template <int HD>
+__global__ void k_pf_qk(PFRopeParams P);
 __global__ void k_pf_swiglu(const float* gate, const float* up, float* h, int n, int m);
 template <int NB8>
 __global__ void k_vocab(const uint8_t* wq, C2hState* st, const float* xb0, const float* xb1, int n_vocab,

@@ -3059,31 +3059,32 @@ __global__ void __launch_bounds__(ATT_AV_THREADS) k_attn_av(AttnCoreParams P) {
 //   k_pf_norm_quant   [embed] RMSNorm -> Q8_K per token
 //   k_pf_gemm         int8 MFMA GEMM (tokens x rows) whose per-sub-block int32
 //                     sums feed the reference's per-row float fold in order
-//   k_pf_rope_store   RoPE(k), K/V stored at their positions
-//   k_attn_core       causal attention per (head, token)
+//   k_pf_qk           QK-norm, RoPE(q, k), K/V stored at their positions
+//   k_pf_attn         causal attention per (head, block of tokens)
 //   k_pf_quant        Q8_K of the attention / SwiGLU rows
 //   k_pf_swiglu       h = SwiGLU(gate, up)
 
 // One token's Q8_K row (LDS form) into the batch buffer.
-template <int NB>
+template <int NB, int NT = 256>
 __device__ __forceinline__ void store_q8_row(const Q8KRow<NB>& s, const PFQ8& o, int t) {
   const int tid = threadIdx.x;
-  for (int i = tid; i < NB * 64; i += 256) {
+  for (int i = tid; i < NB * 64; i += NT) {
     const int b = i >> 6, w = i & 63;
     reinterpret_cast<uint32_t*>(o.q + ((size_t)t * o.nbs + b) * QK_K)[w] = s.q[b][w];
     reinterpret_cast<uint32_t*>(o.qT + (((size_t)b * 8 + (w >> 3)) * PF_MAX + t) * 32)[w & 7] = s.q[b][w];
   }
-  for (int i = tid; i < NB * 16; i += 256) o.bs[((size_t)t * o.nbs + (i >> 4)) * 16 + (i & 15)] = s.bs[i >> 4][i & 15];
+  for (int i = tid; i < NB * 16; i += NT) o.bs[((size_t)t * o.nbs + (i >> 4)) * 16 + (i & 15)] = s.bs[i >> 4][i & 15];
   if (tid < NB) {
     o.d[(size_t)t * o.nbs + tid] = s.d[tid];
     o.dT[(size_t)tid * PF_MAX + t] = s.d[tid];
   }
 }
 
-// Token blockIdx.x (rows past m repeat token m-1; their results are dropped).
+// Token blockIdx.x (rows past m repeat token m-1; their results are
+// dropped), one float4 of the row per thread, wave w quantises block w.
 template <int NB>
-__global__ void __launch_bounds__(256) k_pf_norm_quant(PFNormParams P) {
-  static_assert(NB <= 4, "one float4 per thread");
+__global__ void __launch_bounds__(pf_norm_threads(NB)) k_pf_norm_quant(PFNormParams P) {
+  static_assert(NB <= 8, "one float4 per thread");
   extern __shared__ __align__(16) unsigned char smem[];
   float* sq = reinterpret_cast<float*>(smem);  // [chain_lds_floats(n_x)]
   __shared__ Q8KRow<NB> s;
@@ -3102,7 +3103,7 @@ __global__ void __launch_bounds__(256) k_pf_norm_quant(PFNormParams P) {
   if (P.xn && 4 * tid < P.n_x) reinterpret_cast<float4*>(P.xn + (size_t)t * P.n_x)[tid] = xn;
   if (wave < NB) quantize_wave(xn, wave, s);
   __syncthreads();
-  store_q8_row<NB>(s, P.out, t);
+  store_q8_row<NB, pf_norm_threads(NB)>(s, P.out, t);
 }
 
 template <int NB>
@@ -3306,301 +3307,313 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
 template __global__ void k_pf_gemm_q50<MODE_BIAS>(PFGemmFParams);
 template __global__ void k_pf_gemm_q50<MODE_RESID>(PFGemmFParams);
 
-// RoPE of token t's k (tensor/ops.go:262-286, same expressions as the
-// attention kernel) and the K/V store at pos0 + t (engine/kvcache.go:143-157).
-__global__ void __launch_bounds__(64) k_pf_rope_store(PFRopeParams P) {
-  const int t = blockIdx.x, g = blockIdx.y, d = threadIdx.x;
+// q and k of token blockIdx.x made ready for k_pf_attn, v stored: per head
+// the Qwen3 QK-norm where the layer has the weights (engine/forward.go:80-91
+// -> tensor/ops.go:207-218 over the head's values; the sequential sums of
+// squares run one head per lane), RoPE (tensor/ops.go:262-286, pairs
+// (i, i + HD/2), the attention kernels' expressions), then q back in place
+// and K/V into the cache at pos0 + t (engine/kvcache.go:143-157).  One
+// workgroup per token, a pair per thread and trip: 1 query + KV head per
+// wave was 4.7 us at 512 tokens for K/V alone, this with q 3.9 us.
+template <int HD>
+__global__ void __launch_bounds__(256) k_pf_qk(PFRopeParams P) {
+  constexpr int H2 = HD / 2;
+  extern __shared__ __align__(16) unsigned char smem[];
+  float* sq = reinterpret_cast<float*>(smem);  // QK-norm: [heads][HD + 1] squares, then the heads' scales
+  const int t = blockIdx.x, tid = threadIdx.x;
   const int pos = P.pos0 + t;
-  if (t >= P.m || pos >= P.max_ctx) return;
-  const float* kr = P.k + (size_t)t * P.ld + g * 64;
-  const float* vr = P.v + (size_t)t * P.ld + g * 64;
-  float kv = kr[d];
-  if (pos < P.rope_len) {
-    const int i = d & 31;
-    const float c = P.rope_cos[(size_t)pos * 32 + i], sn = P.rope_sin[(size_t)pos * 32 + i];
-    const float x0 = kr[i], x1 = kr[i + 32];
-    kv = (d < 32) ? (x0 * c) - (x1 * sn) : (x0 * sn) + (x1 * c);
+  if (t >= P.m || pos >= P.max_ctx) return;  // uniform
+  const int nh = P.n_heads + P.n_kv_heads;
+  float* qr = P.q + (size_t)t * P.q_ld;
+  const float* kr = P.k + (size_t)t * P.ld;
+  const float* vr = P.v + (size_t)t * P.ld;
+  const bool norm = P.q_norm || P.k_norm;  // uniform
+  float* inv = sq + nh * (HD + 1);
+  if (norm) {
+    for (int i = tid; i < nh * HD; i += 256) {
+      const int h = i / HD, d = i & (HD - 1);
+      const float x = h < P.n_heads ? qr[i] : kr[i - P.n_heads * HD];
+      sq[h * (HD + 1) + d] = x * x;
+    }
+    __syncthreads();
+    if (tid < nh) {
+      float sum = 0.0f;
+#pragma unroll 16
+      for (int d = 0; d < HD; ++d) sum = sum + sq[tid * (HD + 1) + d];
+      inv[tid] = rms_scale(sum / (float)HD + P.eps);
+    }
+    __syncthreads();
   }
-  const size_t head_stride = (size_t)kv_slot(P.max_ctx) * 64;
-  P.kv[((size_t)P.layer * P.n_kv_heads + g) * head_stride + (size_t)pos * 64 + d] = kv;
-  P.kv[(((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride + vq_index(pos, d)] = vr[d];
-}
-
-// fma(src of lane K of this lane's row of 16 lanes, v, acc) in one
-// instruction: v_fmac_f32 with the DPP operand row_newbcast:K (gfx90a and
-// later), where a broadcast LDS read and an FMA would be two.  Callers keep
-// every lane of the wave active (a disabled source lane reads as 0) and
-// take src straight from an LDS read (a VALU write of src in the two
-// instructions before would need wait states).  Volatile: never moved into
-// a branch.
-template <int K>
-__device__ __forceinline__ float fmac_row_bcast(float acc, float src, float v) {
-  asm volatile("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(src), "v"(v), "n"(K));
-  return acc;
-}
-
-// attn_score with the query broadcast from registers: lane k of each row of
-// 16 holds q[4k .. 4k+3] in qr, every lane its own K row in kk4.  The same
-// two-accumulator FMA order, sum tree and scale.
-__device__ __forceinline__ float attn_score_bc(const f32x4_t& qr, const float4 (&kk4)[16], float scale) {
-  float a0[8], a1[8];
-#pragma unroll
-  for (int l = 0; l < 8; ++l) {
-    a0[l] = 0.0f;
-    a1[l] = 0.0f;
+  const size_t head_stride = (size_t)kv_slot(P.max_ctx) * HD;
+  for (int i = tid; i < nh * H2; i += 256) {
+    const int h = i / H2, d = i & (H2 - 1);
+    const bool is_q = h < P.n_heads;
+    const float* src = is_q ? qr + h * HD : kr + (h - P.n_heads) * HD;
+    float x0 = src[d], x1 = src[d + H2];
+    const float* nw = is_q ? P.q_norm : P.k_norm;
+    if (nw) {
+      x0 = (x0 * inv[h]) * nw[d];
+      x1 = (x1 * inv[h]) * nw[d + H2];
+    }
+    if (pos < P.rope_len) {
+      const float c = P.rope_cos[(size_t)pos * H2 + d], sn = P.rope_sin[(size_t)pos * H2 + d];
+      const float y0 = (x0 * c) - (x1 * sn);
+      x1 = (x0 * sn) + (x1 * c);
+      x0 = y0;
+    }
+    float* dst = is_q ? qr + h * HD
+                      : P.kv + ((size_t)P.layer * P.n_kv_heads + h - P.n_heads) * head_stride + (size_t)pos * HD;
+    dst[d] = x0;
+    dst[d + H2] = x1;
   }
-  static_for<4>([&](auto dd) {
-    constexpr int d = 16 * (int)dd;
-    const float kk[16] = {kk4[d / 4].x,     kk4[d / 4].y,     kk4[d / 4].z,     kk4[d / 4].w,
-                          kk4[d / 4 + 1].x, kk4[d / 4 + 1].y, kk4[d / 4 + 1].z, kk4[d / 4 + 1].w,
-                          kk4[d / 4 + 2].x, kk4[d / 4 + 2].y, kk4[d / 4 + 2].z, kk4[d / 4 + 2].w,
-                          kk4[d / 4 + 3].x, kk4[d / 4 + 3].y, kk4[d / 4 + 3].z, kk4[d / 4 + 3].w};
-    static_for<8>([&](auto l) {
-      constexpr int i0 = d + (int)l, i1 = d + 8 + (int)l;
-      a0[l] = fmac_row_bcast<i0 / 4>(a0[l], qr[i0 % 4], kk[l]);
-      a1[l] = fmac_row_bcast<i1 / 4>(a1[l], qr[i1 % 4], kk[8 + l]);
-    });
-  });
-  float v[8];
-#pragma unroll
-  for (int l = 0; l < 8; ++l) v[l] = a0[l] + a1[l];
-  const float sco = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-  return sco * scale;
+  for (int i = tid; i < P.n_kv_heads * HD; i += 256) {
+    const int g = i / HD, d = i & (HD - 1);
+    P.kv[(((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride + vq_index(pos, d, HD)] = vr[i];
+  }
+}
+template __global__ void k_pf_qk<64>(PFRopeParams);
+template __global__ void k_pf_qk<128>(PFRopeParams);
+
+// The maximum over each row of 16 lanes (no NaN among the operands).
+__device__ __forceinline__ float row_max_dpp(float x) {
+  x = fmax_gt(x, dpp_or0<0x128>(x));  // row_ror:8, :4, :2, :1
+  x = fmax_gt(x, dpp_or0<0x124>(x));
+  x = fmax_gt(x, dpp_or0<0x122>(x));
+  return fmax_gt(x, dpp_or0<0x121>(x));
 }
 
 // Causal attention of a prefill pass: workgroup (query head h, block of
-// PFA_TB query tokens), token i at position pos0 + i attending positions
-// 0..pos0+i, all of whose K/V rows are in the cache.  Per (token, head) the
-// arithmetic is k_attn_core's, bit for bit:
-//   RoPE of q (tensor/ops.go:262-286);
-//   scores in the two-accumulator FMA order (attn_score), times scale;
-//   softmax (tensor/ops.go:317-339): the max of the non-NaN scores (NaN
-//     when score 0 is NaN), f32(exp(f64(s - max))), the exact sequential
-//     f32 sum, times f32(1/sum);
-//   per output dim one FMA chain over positions 0..pos in order
-//     (c2_tensor_attn_gen.go:85-117).
-// Sharing: the K rows of a PFA_CH-position chunk are read from the cache
-// once per block (coalesced, into LDS rows padded to PFA_KPAD floats) and
-// serve the block's tokens; likewise the V quads.  Thread roles (TB =
-// PFA_TB):
-//   scores     position c0 + (t % 128) of the chunk, tokens (TB/2)*(t/128)
-//              .. +TB/2, the query broadcast from registers (every lane
-//              computes, lanes past the token's last position drop theirs);
-//   sums       wave w the tokens w, w+4, ..: each the exact sequential sum
-//              spread over the wave's 64 lanes (seq_sum_wave / _n);
-//   AV         dim t % 64 of tokens (TB/4)*(t/64) .. +TB/4: independent
-//              chains, the probabilities of 64 positions at a time
-//              broadcast from registers.
+// P.tok_blk <= 16 query tokens), token i at position pos0 + i attending
+// positions 0..pos0+i, all of whose K/V rows are in the cache (k_pf_qk), q
+// rotated in place.  Per (token, head) the arithmetic is k_attn_core's, bit
+// for bit, on the FP32 matrix instruction: v_mfma_f32_16x16x4_f32 is, for
+// each of its 16 x 16 results, the chain fma(a3, b3, fma(a2, b2, fma(a1, b1,
+// fma(a0, b0, c)))) with one rounding each, subnormals, infinities and NaNs
+// as v_fma_f32 has them (tests/test_gpu_prefill.py compares the two).
+//   scores   the reference's accumulator a0[l] (a1[l]) of a (token,
+//     position) is the chain over the elements 16 s + l (16 s + 8 + l),
+//     s = 0, 1, ..: one instruction (two at HD = 128) gives it for 16 tokens
+//     x 16 positions; then the tree of sums and the scale;
+//   softmax  (tensor/ops.go:317-339) the max of the non-NaN scores (NaN when
+//     score 0 is NaN), f32(exp(f64(s - max))), the sequential f32 sum as an
+//     fma chain with ones (e * 1 + sum rounds once, as the add does), times
+//     f32(1/sum);
+//   AV       per output dim one fma chain over positions 0..pos in order
+//     (c2_tensor_attn_gen.go:85-117), four positions per instruction, for
+//     16 tokens x 16 dims per wave; the positions from the block's first
+//     token on, which not every token attends, in VALU fmas.
+// What bounds it: per (token, position) the matrix unit needs HD/32 clk for
+// scores and HD/32 for AV (half of the VALU's rate for the same FMAs, and
+// with no broadcast reads: K and q in registers, V from L2), the f64 exp
+// ~10 clk.  A chain of T positions takes 8 T clk, so every dim and head has
+// a wave of its own (HD/16 waves).  Scores of the block's tokens sit in LDS:
+// 16 tokens up to ~2,300 positions, fewer beyond (the host's rule).
+// 512 tokens, 14 heads of 64: 31.9 us with the same FMAs on the VALU.
 // Block order: a block's work grows with its last position, so the grid is
 // one-dimensional and runs the blocks from the last (longest) to the first;
-// the dispatcher hands each freed slot the next block, which evens out the
-// CUs' loads (the longest block sets the kernel's length).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PFA_WAVES_PER_EU, PFA_WAVES_PER_EU))) k_pf_attn(AttnCoreParams P) {
-  constexpr int HD = 64;
-  constexpr int TB = PFA_TB;
-  constexpr int TPT = TB / 2;                 // score tokens per thread
-  constexpr int TPW = TB / 4;                 // AV tokens per wave
-  static_assert(TB % 4 == 0 && TB <= 16, "roles assume 4..16 tokens per block");
-  constexpr int KP = PFA_KPAD;
-  constexpr int KL = PFA_CH * 16 / 256;       // 16-byte K loads per thread and chunk
-  constexpr int VL = PFA_CH / 4 * 64 / 256;   // V quads per thread and chunk
+// the dispatcher hands each freed slot the next block.
+template <int HD>
+__global__ void __launch_bounds__(4 * HD) k_pf_attn(AttnCoreParams P) {
+  constexpr int NW = HD / 16;  // waves
+  constexpr int NT = 4 * HD;   // threads
+  constexpr int NG = HD / 64;  // groups of four chain steps of a score
   extern __shared__ __align__(16) unsigned char smem[];
-  float* kbuf = reinterpret_cast<float*>(smem);        // [PFA_CH][KP]   (scores phase)
-  f32x4_t* vbuf = reinterpret_cast<f32x4_t*>(smem);    // [PFA_CH/4][64] (AV phase)
-  float* q_s = kbuf + PFA_CH * KP;                     // [TB][64]
-  float* sc = q_s + TB * HD;                           // [TB][P.sc_ld]
-  __shared__ float red_m[4][TPT];
-  __shared__ float mx_s[TB], inv_s[TB];
+  float* sc = reinterpret_cast<float*>(smem);  // [tok_blk][P.sc_ld]
+  __shared__ float red_m[NW][16];
+  __shared__ float mx_s[16], inv_s[16];
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the AV loops run with every lane on
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, kg = lane >> 4;
   const int nblk = (int)gridDim.x / P.n_heads;
   const int h = (int)blockIdx.x % P.n_heads;
   const int g = h / (P.n_heads / P.n_kv_heads);
-  const int t0 = (nblk - 1 - (int)blockIdx.x / P.n_heads) * TB;
-  const int nt = min(TB, P.n_tok - t0);      // tokens of this block
+  const int t0 = (nblk - 1 - (int)blockIdx.x / P.n_heads) * P.tok_blk;
+  const int nt = min(P.tok_blk, P.n_tok - t0);  // tokens of this block
   const int ld = P.sc_ld;
-  const int pos0 = P.state->pos;
-  const int pmax = pos0 + t0 + nt - 1;       // last position the block attends
+  const int pfirst = P.state->pos + t0;  // the first token's position: every token attends [0, pfirst]
+  const int pmax = pfirst + nt - 1;      // last position the block attends
   const size_t head_stride = (size_t)kv_slot(P.max_ctx) * HD;
   const float* kcache = P.kv + ((size_t)P.layer * P.n_kv_heads + g) * head_stride;
-  const f32x4_t* vcache =
-      reinterpret_cast<const f32x4_t*>(P.kv + (((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride);
-  // A chunk's K rows / V quads are read 16 bytes per thread and load,
-  // coalesced; rows past pmax repeat row pmax (read, never used), so the
-  // loads of the chunk after the last are harmless and need no branch.
+  const float* vcache = P.kv + (((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride;
 
-  // ---- loads: q of the block's tokens, K chunk 0
-  float4 qv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  // ---- scores: tiles of 16 positions, wave w the tiles w, w + NW, ..
+  // Operands: lane (col, kg) holds of its row (A: token col; B: position
+  // col) the elements 64 G + 16 kg .. +16 of group G, so component c is
+  // step s = 4 G + kg of accumulator c.  Rows past the block's tokens and
+  // positions repeat the last one (finite or not, they touch no other row).
   {
-    const int tk = tid >> 4, c = tid & 15;
-    if (tk < nt) qv = reinterpret_cast<const float4*>(P.q + (size_t)(t0 + tk) * P.q_ld + h * HD)[c];
-  }
-  f32x4_t kn[KL];  // native vectors: a float4 array copied whole is kept in scratch
-  static_for<KL>([&](auto k) {
-    const int i = tid + 256 * k;
-    kn[k] = reinterpret_cast<const f32x4_t*>(kcache + (size_t)min(i >> 4, pmax) * HD)[i & 15];
-  });
-  if (tid < TB * 16) reinterpret_cast<float4*>(q_s)[tid] = qv;
-  __syncthreads();
-  {  // RoPE (pairs i, i+32) at each token's position
-    const int tk = tid >> 4;
-    const int pos = pos0 + t0 + tk;
-    if (tk < nt && pos >= 0 && pos < P.rope_len) {
+    auto load_row = [&](f32x4_t(&r)[NG][4], const float* row) {
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int i = (tid & 15) * 2 + e;
-        const float rc = P.rope_cos[(size_t)pos * (HD / 2) + i], rs = P.rope_sin[(size_t)pos * (HD / 2) + i];
-        float* qr = q_s + tk * HD;
-        const float x0 = qr[i], x1 = qr[i + 32];
-        qr[i] = (x0 * rc) - (x1 * rs);
-        qr[i + 32] = (x0 * rs) + (x1 * rc);
+      for (int G = 0; G < NG; ++G)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[G][i] = reinterpret_cast<const f32x4_t*>(row + 64 * G + 16 * kg)[i];
+    };
+    f32x4_t q[NG][4], kc[NG][4], kn[NG][4];
+    load_row(q, P.q + (size_t)(t0 + min(col, nt - 1)) * P.q_ld + h * HD);
+    const int ntile = (pmax >> 4) + 1;
+    float lmax[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lmax[i] = -__builtin_inff();
+    auto load_tile = [&](f32x4_t(&r)[NG][4], int tile) {
+      load_row(r, kcache + (size_t)min(16 * min(tile, ntile - 1) + col, pmax) * HD);
+    };
+    auto run_tile = [&](const f32x4_t(&k)[NG][4], int tile) {
+      f32x4_t u[4];  // pair sums (v0+v1), (v2+v3), (v4+v5), (v6+v7)
+      static_for<4>([&](auto pr) {
+        f32x4_t d[4];  // accumulators 2 pr, 2 pr + 8, 2 pr + 1, 2 pr + 9
+        static_for<NG>([&](auto G) {
+          static_for<4>([&](auto x) {
+            constexpr int c = 2 * (int)pr + ((int)x >> 1) + 8 * ((int)x & 1);
+            const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            d[(int)x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[(int)G][c / 4][c % 4], k[(int)G][c / 4][c % 4],
+                                                             (int)G == 0 ? zero : d[(int)x], 0, 0, 0);
+          });
+        });
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[(int)pr][i] = (d[0][i] + d[1][i]) + (d[2][i] + d[3][i]);
+      });
+      const int p = 16 * tile + col;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * kg + i;
+        const float s = ((u[0][i] + u[1][i]) + (u[2][i] + u[3][i])) * P.scale;
+        if (r < nt && p <= pfirst + r) {
+          sc[r * ld + p] = s;
+          lmax[i] = (s > lmax[i]) ? s : lmax[i];
+        }
       }
+    };
+    // two register sets in turn, the next tile's K in flight
+    load_tile(kc, wave);
+    for (int tile = wave; tile < ntile; tile += 2 * NW) {
+      load_tile(kn, tile + NW);
+      run_tile(kc, tile);
+      if (tile + NW >= ntile) break;  // uniform
+      load_tile(kc, tile + 2 * NW);
+      run_tile(kn, tile + NW);
     }
-  }
-
-  // ---- scores, chunk by chunk of K rows; the next chunk loads meanwhile
-  const int th = tid >> 7, pl = tid & 127;
-  __syncthreads();  // q is turned
-  f32x4_t qr[TPT];  // lane k of each row: q[4k .. 4k+3] of token th*TPT + j
-  static_for<TPT>([&](auto j) { qr[j] = reinterpret_cast<const f32x4_t*>(q_s + (th * TPT + (int)j) * HD)[lane & 15]; });
-  float lmax[TPT];
 #pragma unroll
-  for (int j = 0; j < TPT; ++j) lmax[j] = -__builtin_inff();
-  for (int c0 = 0; c0 <= pmax; c0 += PFA_CH) {
-    __syncthreads();  // the previous chunk's rows are read (and, first time, q is turned)
-    static_for<KL>([&](auto k) {
-      const int i = tid + 256 * k;
-      reinterpret_cast<f32x4_t*>(kbuf + (i >> 4) * KP)[i & 15] = kn[k];
-    });
-    static_for<KL>([&](auto k) {  // the next chunk
-      const int i = tid + 256 * k;
-      kn[k] = reinterpret_cast<const f32x4_t*>(kcache + (size_t)min(c0 + PFA_CH + (i >> 4), pmax) * HD)[i & 15];
-    });
-    __syncthreads();
-    const int p = c0 + pl;
-    float4 kk4[16];  // rows past pmax repeat row pmax: finite, computed, dropped
-#pragma unroll
-    for (int i = 0; i < 16; ++i) kk4[i] = reinterpret_cast<const float4*>(kbuf + pl * KP)[i];
-    static_for<TPT>([&](auto j) {
-      const int tk = th * TPT + (int)j;
-      const float sco = attn_score_bc(qr[j], kk4, P.scale);
-      if (tk < nt && p <= pos0 + t0 + tk) {
-        sc[tk * ld + p] = sco;
-        lmax[j] = (sco > lmax[j]) ? sco : lmax[j];
-      }
-    });
-  }
-  // ---- max per token: waves 2th, 2th+1 hold tokens TPT*th .. +TPT
-#pragma unroll
-  for (int j = 0; j < TPT; ++j) {
-    const float m = wave_max_dpp(lmax[j]);
-    if (lane == 0) red_m[wave][j] = m;
+    for (int i = 0; i < 4; ++i) {
+      const float m = row_max_dpp(lmax[i]);
+      if (col == 0) red_m[wave][4 * kg + i] = m;
+    }
   }
   __syncthreads();
   if (tid < nt) {
-    const int w0 = 2 * (tid / TPT), j = tid % TPT;
-    float m = fmax_gt(red_m[w0][j], red_m[w0 + 1][j]);
+    float m = red_m[0][tid];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m = fmax_gt(m, red_m[w][tid]);
     const float s0 = sc[tid * ld];
     if (s0 != s0) m = s0;
     mx_s[tid] = m;
   }
   __syncthreads();
-  // ---- exps
-  for (int tk = 0; tk < nt; ++tk) {
-    const float m = mx_s[tk];
-    for (int p = tid; p <= pos0 + t0 + tk; p += 256) sc[tk * ld + p] = (float)exp((double)(sc[tk * ld + p] - m));
+  // ---- exps, four positions per thread; 0 past a token's last position
+  // (up to whole quads of the block)
+  const int nq = (pmax >> 2) + 1;
+  for (int i = tid; i < nt * nq; i += NT) {
+    const int r = i / nq, p = 4 * (i - r * nq);
+    const float m = mx_s[r];
+    float4* at = reinterpret_cast<float4*>(sc + r * ld + p);
+    const float4 s = *at;
+    const int last = pfirst + r;
+    float4 e;
+    e.x = (p + 0 <= last) ? (float)exp((double)(s.x - m)) : 0.0f;
+    e.y = (p + 1 <= last) ? (float)exp((double)(s.y - m)) : 0.0f;
+    e.z = (p + 2 <= last) ? (float)exp((double)(s.z - m)) : 0.0f;
+    e.w = (p + 3 <= last) ? (float)exp((double)(s.w - m)) : 0.0f;
+    *at = e;
   }
-  f32x4_t vn[VL];  // V chunk 0 lands under the sums
-  static_for<VL>([&](auto k) {
-    const int i = tid + 256 * k;
-    vn[k] = vcache[(size_t)min(i >> 6, pmax >> 2) * 64 + (i & 63)];
-  });
+  // ---- AV operands: B lane (col, kg) dim 16 wave + col of position 4 quad
+  // + kg; the first batch of V and the quads from pfirst's on land under
+  // the sums
+  constexpr int VB = 16;                       // quads per batch
+  const int nfull = (pfirst + 1) >> 2;         // quads every token attends whole
+  const unsigned vl = (unsigned)(16 * wave + col) * 4 + kg;
+  const int qlast = nq - 1;
+  float va[VB], vb[VB];
+  auto load_v = [&](float(&v)[VB], int q0) {
+#pragma unroll
+    for (int k = 0; k < VB; ++k) v[k] = (vcache + (size_t)min(q0 + k, qlast) * (4 * HD))[vl];
+  };
+  load_v(va, 0);
+  constexpr int TQ = 5;  // the tail: positions 4 nfull .. pmax, at most 3 + 16
+  f32x4_t vt[TQ];
+#pragma unroll
+  for (int k = 0; k < TQ; ++k)
+    vt[k] = reinterpret_cast<const f32x4_t*>(vcache)[(size_t)min(nfull + k, qlast) * HD + 16 * wave + col];
   __syncthreads();
-  // ---- sequential sums: wave w the tokens w, w+4, .. over its 64 lanes
-  for (int tk = wave; tk < nt; tk += 4) {
-    const int n = pos0 + t0 + tk + 1;
-    const float s = (n <= 64 * SPEC_C) ? seq_sum_wave(sc + tk * ld, n) : seq_sum_wave_n(sc + tk * ld, n);
-    if (lane == 0) inv_s[tk] = 1.0f / s;
+  const float* arow = sc + min(col, nt - 1) * ld + kg;  // A: token col, position 4 quad + kg
+  // ---- sums: wave 0, all of the block's tokens at once
+  if (wave == 0) {
+    f32x4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+    int q = 0;
+    for (; q + VB <= nq; q += VB) {
+      float a[VB];
+#pragma unroll
+      for (int k = 0; k < VB; ++k) a[k] = arow[4 * (q + k)];
+#pragma unroll
+      for (int k = 0; k < VB; ++k) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], 1.0f, s, 0, 0, 0);
+    }
+    for (; q < nq; ++q) s = __builtin_amdgcn_mfma_f32_16x16x4f32(arow[4 * q], 1.0f, s, 0, 0, 0);
+    if (col == 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) inv_s[4 * kg + i] = 1.0f / s[i];
   }
   __syncthreads();
-  for (int tk = 0; tk < nt; ++tk) {
-    const float iv = inv_s[tk];
-    for (int p = tid; p <= pos0 + t0 + tk; p += 256) sc[tk * ld + p] = sc[tk * ld + p] * iv;
-  }
 
-  // ---- AV: TPW chains per thread (dim lane, tokens TPW*wave .. +TPW), V quads by chunk
-  const float4* sc4[TPW];
+  // ---- AV: the probabilities are e * (1/sum), formed as they are read
+  const float ainv = inv_s[min(col, nt - 1)];
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto run_v = [&](const float(&v)[VB], int q0, int n) {
+    float a[VB];
 #pragma unroll
-  for (int j = 0; j < TPW; ++j) sc4[j] = reinterpret_cast<const float4*>(sc + min(wave * TPW + j, TB - 1) * ld);
-  const int last0 = pos0 + t0 + wave * TPW;  // every token of the wave attends [0, last0]
-  float acc[TPW];
+    for (int k = 0; k < VB; ++k) a[k] = arow[4 * min(q0 + k, qlast)] * ainv;
+    if (n >= VB) {  // uniform
 #pragma unroll
-  for (int j = 0; j < TPW; ++j) acc[j] = 0.0f;
-  for (int c0 = 0; c0 <= pmax; c0 += PFA_CH) {
-    __syncthreads();  // K rows (first time) / the previous V chunk are read
-    static_for<VL>([&](auto k) { vbuf[tid + 256 * k] = vn[k]; });
-    static_for<VL>([&](auto k) {  // the next chunk
-      const int i = tid + 256 * k;
-      vn[k] = vcache[(size_t)min(((c0 + PFA_CH) >> 2) + (i >> 6), pmax >> 2) * 64 + (i & 63)];
-    });
-    __syncthreads();
-    const int nq = min(PFA_CH, pmax + 1 - c0 + 3) >> 2;               // quads of the chunk up to pmax
-    const int nfull = max(min((last0 + 1 - c0) >> 2, nq), 0);          // quads all the wave's tokens use whole
-    int qd = 0;
-    for (; qd + 16 <= nfull; qd += 16) {  // 64 positions: p of c0 + 4(qd+k) + c is component c of lane k
-      f32x4_t pq[TPW];
+      for (int k = 0; k < VB; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], v[k], acc, 0, 0, 0);
+    } else {
 #pragma unroll
-      for (int j = 0; j < TPW; ++j) pq[j] = reinterpret_cast<const f32x4_t*>(sc4[j])[(c0 >> 2) + qd + (lane & 15)];
-      static_for<2>([&](auto hf) {  // two halves of eight quads
-        f32x4_t v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = vbuf[(qd + 8 * (int)hf + k) * 64 + lane];
-        static_for<8>([&](auto k) {
-          static_for<4>([&](auto c) {
-#pragma unroll
-            for (int j = 0; j < TPW; ++j)
-              acc[j] = fmac_row_bcast<8 * (int)hf + (int)k>(acc[j], pq[j][(int)c], v[k][(int)c]);
-          });
-        });
-      });
+      for (int k = 0; k < VB; ++k)
+        if (k < n) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], v[k], acc, 0, 0, 0);
     }
-    for (; qd + 4 <= nfull; qd += 4) {  // sixteen positions: every read issued before the FMAs
-      f32x4_t v[4];
-      float4 pr[TPW][4];
+  };
+  for (int q0 = 0; q0 < nfull; q0 += 2 * VB) {
+    load_v(vb, q0 + VB);
+    run_v(va, q0, nfull - q0);
+    if (q0 + VB >= nfull) break;  // uniform
+    load_v(va, q0 + 2 * VB);
+    run_v(vb, q0 + VB, nfull - q0 - VB);
+  }
+  // the tail, position by position against each token's last
+  float rinv[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[k] = vbuf[(qd + k) * 64 + lane];
+  for (int i = 0; i < 4; ++i) rinv[i] = inv_s[4 * kg + i];
 #pragma unroll
-        for (int j = 0; j < TPW; ++j) pr[j][k] = sc4[j][(c0 >> 2) + qd + k];
-      }
+  for (int k = 0; k < TQ; ++k) {
+    const int p = 4 * (nfull + k);
+    if (p > pmax) break;  // uniform
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int j = 0; j < TPW; ++j) acc[j] = fma4(acc[j], pr[j][k], v[k]);
-    }
-    for (; qd < nq; ++qd) {  // the rest, position by position against each token's last
-      const f32x4_t v = vbuf[qd * 64 + lane];
-      const int p = c0 + 4 * qd;
-#pragma unroll
-      for (int j = 0; j < TPW; ++j) {
-        const int last = last0 + j;
-        if (p <= last) {
-          const float4 pr = sc4[j][p >> 2];
-          acc[j] = __builtin_fmaf(pr.x, v.x, acc[j]);
-          if (p + 1 <= last) acc[j] = __builtin_fmaf(pr.y, v.y, acc[j]);
-          if (p + 2 <= last) acc[j] = __builtin_fmaf(pr.z, v.z, acc[j]);
-          if (p + 3 <= last) acc[j] = __builtin_fmaf(pr.w, v.w, acc[j]);
-        }
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int r = 4 * kg + i, last = pfirst + r;
+      const float4 e = *reinterpret_cast<const float4*>(sc + min(r, nt - 1) * ld + p);
+      float a = acc[i];
+      a = (p + 0 <= last) ? __builtin_fmaf(e.x * rinv[i], vt[k].x, a) : a;
+      a = (p + 1 <= last) ? __builtin_fmaf(e.y * rinv[i], vt[k].y, a) : a;
+      a = (p + 2 <= last) ? __builtin_fmaf(e.z * rinv[i], vt[k].z, a) : a;
+      a = (p + 3 <= last) ? __builtin_fmaf(e.w * rinv[i], vt[k].w, a) : a;
+      acc[i] = a;
     }
   }
 #pragma unroll
-  for (int j = 0; j < TPW; ++j) {
-    const int tk = wave * TPW + j;
-    if (tk < nt) P.out[(size_t)(t0 + tk) * P.out_ld + h * HD + lane] = acc[j];
+  for (int i = 0; i < 4; ++i) {
+    const int r = 4 * kg + i;
+    if (r < nt) P.out[(size_t)(t0 + r) * P.out_ld + h * HD + 16 * wave + col] = acc[i];
   }
 }
+template __global__ void k_pf_attn<64>(AttnCoreParams);
+template __global__ void k_pf_attn<128>(AttnCoreParams);
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x16_t __attribute__((ext_vector_type(16)));
@@ -3960,14 +3973,23 @@ __global__ void __launch_bounds__(256) k_pf_swiglu(const float* gate, const floa
   }
 }
 
-#define C2H_PF(NB_)                                                 \
-  template __global__ void k_pf_norm_quant<NB_>(PFNormParams);      \
-  template __global__ void k_pf_quant<NB_>(PFQuantParams);
+#define C2H_PF(NB_) template __global__ void k_pf_norm_quant<NB_>(PFNormParams);
 C2H_PF(3)
 C2H_PF(4)
+C2H_PF(6)
+C2H_PF(8)
 #undef C2H_PF
-template __global__ void k_pf_quant<12>(PFQuantParams);
-template __global__ void k_pf_quant<19>(PFQuantParams);
+#define C2H_PF(NB_) template __global__ void k_pf_quant<NB_>(PFQuantParams);
+C2H_PF(3)
+C2H_PF(4)
+C2H_PF(6)
+C2H_PF(8)
+C2H_PF(12)
+C2H_PF(19)
+C2H_PF(24)
+C2H_PF(35)
+C2H_PF(43)
+#undef C2H_PF
 template __global__ void k_pf_gemm<T_Q4_K, MODE_BIAS, 4>(PFGemmParams);
 template __global__ void k_pf_gemm<T_Q4_K, MODE_RESID, 4>(PFGemmParams);
 template __global__ void k_pf_gemm<T_Q4_K, MODE_BIAS, 1>(PFGemmParams);
