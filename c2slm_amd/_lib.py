@@ -91,6 +91,7 @@ def lib():
                                                      C.POINTER(C.c_float)]),
             "c2h_check_rms_scale": (C.c_int, [VP, C.c_uint32, C.c_uint64, C.POINTER(C.c_uint64),
                                               C.POINTER(C.c_uint32)]),
+            "c2h_check_exp": (C.c_int, [VP, C.c_uint32, C.c_uint64, C.POINTER(C.c_uint64), C.POINTER(C.c_uint32)]),
             "c2h_time_steps": (C.c_int, [VP, I32, I32, C.c_float, I32, I32, C.POINTER(C.c_float)]),
             "c2h_gemv_f32": (C.c_int, [VP, I32, VP, VP, I32, I32, VP]),
             "c2h_gemv_f32_dev": (C.c_int, [VP, I32, VP, VP, I32, I32, VP]),
@@ -251,6 +252,12 @@ class Ctx:
         scale against the IEEE sqrt and division over patterns [lo, hi)."""
         bad, first = C.c_uint64(), C.c_uint32()
         self._chk(lib().c2h_check_rms_scale(self.h, lo, hi, C.byref(bad), C.byref(first)))
+        return bad.value, first.value
+
+    def check_exp(self, lo: int, hi: int) -> tuple[int, int]:
+        """The same for the softmax's f32(exp(f64(t)))."""
+        bad, first = C.c_uint64(), C.c_uint32()
+        self._chk(lib().c2h_check_exp(self.h, lo, hi, C.byref(bad), C.byref(first)))
         return bad.value, first.value
 
     def time_steps(self, pos: int, iters: int, penalty: float, im_end: int, eos: int) -> float:

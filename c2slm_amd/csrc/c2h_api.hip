@@ -1433,7 +1433,8 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
                         (const void*)k_pf_gemm_q50<MODE_BIAS>, (const void*)k_pf_gemm_q50<MODE_RESID>})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, PF_F_LDS_MAX) != hipSuccess)
       return bail(fail(c, C2H_ERR_HIP, "prefill GEMM LDS attribute"));
-  for (const void* k : {(const void*)k_pf_attn<64>, (const void*)k_pf_attn<128>})
+  for (const void* k : {(const void*)k_pf_attn<64, true>, (const void*)k_pf_attn<64, false>,
+                        (const void*)k_pf_attn<128, true>, (const void*)k_pf_attn<128, false>})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PFA_LDS_MAX) != hipSuccess)
       return bail(fail(c, C2H_ERR_HIP, "prefill attention LDS attribute"));
   if (D.head_dim == 128) {  // k_attn_h128 at every T: the scores of max_ctx positions in LDS
@@ -1771,7 +1772,7 @@ PFQuantKernel pf_quant_kernel(int nb) {
 int pf_attn_tokens(int n_heads, int m, int pmax) {
   int tb = PFA_TB;
   while (tb > 4 && n_heads * ((m + tb - 1) / tb) < PFA_MIN_WG) tb /= 2;
-  while (tb > 1 && pfa_lds_bytes(tb, pmax) > PFA_LDS_MAX) tb /= 2;
+  while (tb > 1 && pfa_lds_bytes(tb, pmax, true) > PFA_LDS_MAX) tb /= 2;
   return tb;
 }
 
@@ -1861,9 +1862,11 @@ int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
       const int pmax = pos0 + m - 1;
       A.tok_blk = pf_attn_tokens(D.n_heads, m, pmax);
       A.sc_ld = pfa_sc_ld(pmax);
-      hipLaunchKernelGGL(D.head_dim == 64 ? k_pf_attn<64> : k_pf_attn<128>,
-                         dim3(D.n_heads * ((m + A.tok_blk - 1) / A.tok_blk)), dim3(4 * D.head_dim),
-                         pfa_lds_bytes(A.tok_blk, pmax), c->stream, A);
+      const bool stage = pfa_lds_bytes(A.tok_blk, pmax, true) <= PFA_LDS_MAX;
+      const auto k = D.head_dim == 64 ? (stage ? k_pf_attn<64, true> : k_pf_attn<64, false>)
+                                      : (stage ? k_pf_attn<128, true> : k_pf_attn<128, false>);
+      hipLaunchKernelGGL(k, dim3(D.n_heads * ((m + A.tok_blk - 1) / A.tok_blk)), dim3(64 * PFA_NW),
+                         pfa_lds_bytes(A.tok_blk, pmax, stage), c->stream, A);
     }
     {
       PFQuantParams Q{p.attn, E, m, q8};
@@ -2462,7 +2465,9 @@ int c2h_copy_bench(c2h_ctx* c, int64_t bytes, int32_t reps, float* ms) {
   return C2H_OK;
 }
 
-int c2h_check_rms_scale(c2h_ctx* c, uint32_t lo, uint64_t hi, uint64_t* mismatches, uint32_t* first_bits) {
+// A sweep kernel over the bit patterns [lo, hi).
+static int check_sweep(c2h_ctx* c, decltype(&k_check_exp) k, const char* what, uint32_t lo, uint64_t hi,
+                       uint64_t* mismatches, uint32_t* first_bits) {
   if (!c || !mismatches || !first_bits || hi > (1ull << 32) || hi < lo) return C2H_ERR_INVALID;
   HIPCHK(c, hipSetDevice(c->device));
   unsigned long long* bad = nullptr;
@@ -2473,7 +2478,7 @@ int c2h_check_rms_scale(c2h_ctx* c, uint32_t lo, uint64_t hi, uint64_t* mismatch
   constexpr uint64_t kChunk = 1ull << 28;  // patterns per launch (2^20 workgroups)
   for (uint64_t b = lo; e == hipSuccess && b < hi; b += kChunk) {
     const uint32_t n = (uint32_t)std::min<uint64_t>(kChunk, hi - b);
-    hipLaunchKernelGGL(k_check_rms_scale, dim3((n + 255) / 256), dim3(256), 0, c->stream, (uint32_t)b, n, bad, first);
+    hipLaunchKernelGGL(k, dim3((n + 255) / 256), dim3(256), 0, c->stream, (uint32_t)b, n, bad, first);
     e = hipGetLastError();
   }
   unsigned long long nb = 0;
@@ -2482,10 +2487,16 @@ int c2h_check_rms_scale(c2h_ctx* c, uint32_t lo, uint64_t hi, uint64_t* mismatch
   if (e == hipSuccess) e = hipMemcpyAsync(&fb, first, 4, hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (bad) (void)hipFree(bad);
-  if (e != hipSuccess) return fail(c, C2H_ERR_HIP, "rms scale check: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return fail(c, C2H_ERR_HIP, "%s check: %s", what, hipGetErrorString(e));
   *mismatches = nb;
   *first_bits = fb;
   return C2H_OK;
+}
+int c2h_check_rms_scale(c2h_ctx* c, uint32_t lo, uint64_t hi, uint64_t* mismatches, uint32_t* first_bits) {
+  return check_sweep(c, k_check_rms_scale, "rms scale", lo, hi, mismatches, first_bits);
+}
+int c2h_check_exp(c2h_ctx* c, uint32_t lo, uint64_t hi, uint64_t* mismatches, uint32_t* first_bits) {
+  return check_sweep(c, k_check_exp, "exp", lo, hi, mismatches, first_bits);
 }
 
 int c2h_launch_floor(c2h_ctx* c, int32_t n, int32_t grid, int32_t reps, float* us) {

@@ -268,12 +268,17 @@ constexpr int ATT_XCDS = 8;
 constexpr int PFA_TB = 16;
 // fewer tokens per workgroup below this many workgroups (one per CU)
 constexpr int PFA_MIN_WG = 256;
+constexpr int PFA_NW = 8;   // waves of a workgroup
+constexpr int PFA_KP = 68;  // floats per staged K row (64 + 4: conflict-free row reads)
 // Row stride (floats) of the block's scores for positions up to pmax: 4 mod
 // 64, so that 16 rows of four consecutive floats lie in different banks.
 __host__ __device__ inline int pfa_sc_ld(int pmax) { return ((pmax + 1 + 63) & ~63) + 4; }
-__host__ __device__ inline size_t pfa_lds_bytes(int tok_blk, int pmax) { return (size_t)tok_blk * pfa_sc_ld(pmax) * 4; }
+// Dynamic LDS: the scores, then (stage) 16 K rows per wave.
+__host__ __device__ inline size_t pfa_lds_bytes(int tok_blk, int pmax, bool stage) {
+  return (size_t)tok_blk * pfa_sc_ld(pmax) * 4 + (stage ? PFA_NW * 16 * PFA_KP * 4 : 0);
+}
 // one token's scores of the longest context (head_dim 128: up to 38,848
-// positions) fit with the kernel's static LDS
+// positions) fit with the kernel's static LDS when K is not staged
 constexpr size_t PFA_LDS_MAX = 156 * 1024;
 
 // Dynamic LDS of k_attn_h128 (head_dim 128), in floats: the scores of every
@@ -484,8 +489,8 @@ __global__ void k_attn_softmax(AttnCoreParams P);
 __global__ void k_attn_av(AttnCoreParams P);
 template <int VCH>
 __global__ void k_attn_h128(AttnCoreParams P);
-template <int HD>
-__global__ void k_pf_attn(AttnCoreParams P);  // 4 HD threads
+template <int HD, bool STAGE>
+__global__ void k_pf_attn(AttnCoreParams P);  // 64 PFA_NW threads
 // threads of k_pf_norm_quant: one float4 of the row each
 __host__ __device__ constexpr int pf_norm_threads(int nb) { return nb <= 4 ? 256 : 512; }
 template <int NB>
@@ -614,5 +619,7 @@ struct PcBenchParams {
 __global__ void k_pc_bench(PcBenchParams P);
 __global__ void k_fill_u32(unsigned* p, int n, unsigned v);
 __global__ void k_check_rms_scale(uint32_t lo, uint32_t n, unsigned long long* bad, uint32_t* first);
+constexpr int EXP_TAB = 32;  // entries of exp_f32's table
+__global__ void k_check_exp(uint32_t lo, uint32_t n, unsigned long long* bad, uint32_t* first);
 
 }  // namespace c2h

@@ -515,6 +515,61 @@ __global__ void __launch_bounds__(256) k_check_rms_scale(uint32_t lo, uint32_t n
   }
 }
 
+// 2^(j/32), each the nearest double.
+__device__ const double kExp2Frac[EXP_TAB] = {
+    0x1.0000000000000p+0, 0x1.059b0d3158574p+0, 0x1.0b5586cf9890fp+0, 0x1.11301d0125b51p+0, 0x1.172b83c7d517bp+0,
+    0x1.1d4873168b9aap+0, 0x1.2387a6e756238p+0, 0x1.29e9df51fdee1p+0, 0x1.306fe0a31b715p+0, 0x1.371a7373aa9cbp+0,
+    0x1.3dea64c123422p+0, 0x1.44e086061892dp+0, 0x1.4bfdad5362a27p+0, 0x1.5342b569d4f82p+0, 0x1.5ab07dd485429p+0,
+    0x1.6247eb03a5585p+0, 0x1.6a09e667f3bcdp+0, 0x1.71f75e8ec5f74p+0, 0x1.7a11473eb0187p+0, 0x1.82589994cce13p+0,
+    0x1.8ace5422aa0dbp+0, 0x1.93737b0cdc5e5p+0, 0x1.9c49182a3f090p+0, 0x1.a5503b23e255dp+0, 0x1.ae89f995ad3adp+0,
+    0x1.b7f76f2fb5e47p+0, 0x1.c199bdd85529cp+0, 0x1.cb720dcef9069p+0, 0x1.d5818dcfba487p+0, 0x1.dfc97337b9b5fp+0,
+    0x1.ea4afa2a490dap+0, 0x1.f50765b6e4540p+0};
+
+// f32(exp(f64(t))) of the softmax (tensor/ops.go:327-330) for t <= 0 or NaN:
+// exp(t) = 2^e 2^(j/32) e^r with n = round(32 t / ln 2) = 32 e + j and
+// |r| <= ln 2 / 64, in f64 (the two-part ln 2 / 32 keeps r exact to a final
+// rounding; the Taylor sum to r^6 is off by 2^-58), rounded once to f32.
+// Equal to the f32 of the library's f64 exp for every such float (swept by
+// c2h_check_exp); ~20 instructions instead of ~45.  tab: kExp2Frac in LDS.
+__device__ __forceinline__ float exp_f32(float t, const double* tab) {
+  const double x = (double)t;
+  const double k = __builtin_fma(x, 0x1.71547652b82fep+5, 0x1.8p+52);
+  const double nd = k - 0x1.8p+52;
+  const int n = __double2loint(k);
+  double r = __builtin_fma(nd, -0x1.62e42fefa0000p-6, x);
+  r = __builtin_fma(nd, -0x1.cf79abc9e3b3ap-45, r);
+  double p = __builtin_fma(r, 1.0 / 720.0, 1.0 / 120.0);
+  p = __builtin_fma(r, p, 1.0 / 24.0);
+  p = __builtin_fma(r, p, 1.0 / 6.0);
+  p = __builtin_fma(r, p, 0.5);
+  p = __builtin_fma(r, p, 1.0);
+  const double f = tab[n & (EXP_TAB - 1)];
+  const double v = __builtin_fma(f * r, p, f);
+  const double y = __hiloint2double(__double2hiint(v) + ((n & ~(EXP_TAB - 1)) << 15), __double2loint(v));
+  return t < -200.0f ? 0.0f : (float)y;  // (2^e stays a normal double down to there)
+}
+__device__ __forceinline__ void load_exp_tab(double* tab) {
+  if (threadIdx.x < EXP_TAB) tab[threadIdx.x] = kExp2Frac[threadIdx.x];
+}
+
+// exp_f32 against the library's f64 exp over the bit patterns [lo, lo + n);
+// mismatches as k_check_rms_scale counts them.
+__global__ void __launch_bounds__(256) k_check_exp(uint32_t lo, uint32_t n, unsigned long long* bad, uint32_t* first) {
+  __shared__ double tab[EXP_TAB];
+  load_exp_tab(tab);
+  __syncthreads();
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t bits = lo + i;
+  const float t = __uint_as_float(bits);
+  const float want = (float)exp((double)t);
+  const float got = exp_f32(t, tab);
+  if (__float_as_uint(want) != __float_as_uint(got) && !(want != want && got != got)) {
+    atomicAdd(bad, 1ull);
+    atomicMin(first, bits);
+  }
+}
+
 // 1/rms of n values (n <= 4*blockDim.x, a multiple of 4) held as elements
 // 4t..4t+3 by thread t < n/4, tensor/ops.go:207-218: sequential f32 sum of
 // x*x, inv = f32(1/sqrt(f64(sum/n + eps))).  sq: LDS scratch of
@@ -3389,7 +3444,7 @@ __device__ __forceinline__ float row_max_dpp(float x) {
 // for bit, on the FP32 matrix instruction: v_mfma_f32_16x16x4_f32 is, for
 // each of its 16 x 16 results, the chain fma(a3, b3, fma(a2, b2, fma(a1, b1,
 // fma(a0, b0, c)))) with one rounding each, subnormals, infinities and NaNs
-// as v_fma_f32 has them (tests/test_gpu_prefill.py compares the two).
+// as v_fma_f32 has them (tests/test_gpu_prefill_attn.py compares the two).
 //   scores   the reference's accumulator a0[l] (a1[l]) of a (token,
 //     position) is the chain over the elements 16 s + l (16 s + 8 + l),
 //     s = 0, 1, ..: one instruction (two at HD = 128) gives it for 16 tokens
@@ -3400,25 +3455,31 @@ __device__ __forceinline__ float row_max_dpp(float x) {
 //     f32(1/sum);
 //   AV       per output dim one fma chain over positions 0..pos in order
 //     (c2_tensor_attn_gen.go:85-117), four positions per instruction, for
-//     16 tokens x 16 dims per wave; the positions from the block's first
-//     token on, which not every token attends, in VALU fmas.
-// What bounds it: per (token, position) the matrix unit needs HD/32 clk for
-// scores and HD/32 for AV (half of the VALU's rate for the same FMAs, and
-// with no broadcast reads: K and q in registers, V from L2), the f64 exp
-// ~10 clk.  A chain of T positions takes 8 T clk, so every dim and head has
-// a wave of its own (HD/16 waves).  Scores of the block's tokens sit in LDS:
-// 16 tokens up to ~2,300 positions, fewer beyond (the host's rule).
-// 512 tokens, 14 heads of 64: 31.9 us with the same FMAs on the VALU.
+//     16 tokens x 16 dims per wave (HD/16 of the waves); the positions from
+//     the block's first token on, which not every token attends, in VALU
+//     fmas.
+// What bounds it: per 16 tokens and position the matrix unit needs HD/2 clk
+// for scores and HD/2 for AV (half of the VALU's time for the same FMAs, and
+// no broadcast reads), the exps ~40 VALU clk; a chain over T positions is
+// 8 T clk long.  Every global load is 16 bytes per lane, each four lanes on
+// 64 contiguous bytes: with the operands' own lane order (a row per lane)
+// the loads took four times the address cycles and set the pace.  K goes
+// through the wave's own 16 rows of LDS (STAGE; without it, where a long
+// context's scores leave no room, in the operands' order), V quads turn into
+// operands with lane-row swaps.  Scores of the block's tokens sit in LDS: 16
+// tokens up to ~1,900 positions, fewer beyond (pf_attn_tokens).
 // Block order: a block's work grows with its last position, so the grid is
 // one-dimensional and runs the blocks from the last (longest) to the first;
 // the dispatcher hands each freed slot the next block.
-template <int HD>
-__global__ void __launch_bounds__(4 * HD) k_pf_attn(AttnCoreParams P) {
-  constexpr int NW = HD / 16;  // waves
-  constexpr int NT = 4 * HD;   // threads
+template <int HD, bool STAGE>
+__global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
+  constexpr int NW = PFA_NW;
+  constexpr int NT = 64 * NW;
   constexpr int NG = HD / 64;  // groups of four chain steps of a score
+  constexpr int KP = PFA_KP;
   extern __shared__ __align__(16) unsigned char smem[];
   float* sc = reinterpret_cast<float*>(smem);  // [tok_blk][P.sc_ld]
+  __shared__ double exp_tab[EXP_TAB];
   __shared__ float red_m[NW][16];
   __shared__ float mx_s[16], inv_s[16];
 
@@ -3436,6 +3497,7 @@ __global__ void __launch_bounds__(4 * HD) k_pf_attn(AttnCoreParams P) {
   const size_t head_stride = (size_t)kv_slot(P.max_ctx) * HD;
   const float* kcache = P.kv + ((size_t)P.layer * P.n_kv_heads + g) * head_stride;
   const float* vcache = P.kv + (((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride;
+  load_exp_tab(exp_tab);
 
   // ---- scores: tiles of 16 positions, wave w the tiles w, w + NW, ..
   // Operands: lane (col, kg) holds of its row (A: token col; B: position
@@ -3443,22 +3505,51 @@ __global__ void __launch_bounds__(4 * HD) k_pf_attn(AttnCoreParams P) {
   // step s = 4 G + kg of accumulator c.  Rows past the block's tokens and
   // positions repeat the last one (finite or not, they touch no other row).
   {
-    auto load_row = [&](f32x4_t(&r)[NG][4], const float* row) {
+    float* kst = sc + P.tok_blk * ld + wave * (16 * KP);  // STAGE: this wave's K rows, one group of 64 elements
+    f32x4_t q[NG][4], k[NG][4], kr[NG][4];
+    {
+      const float* row = P.q + (size_t)(t0 + min(col, nt - 1)) * P.q_ld + h * HD + 16 * kg;
 #pragma unroll
       for (int G = 0; G < NG; ++G)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[G][i] = reinterpret_cast<const f32x4_t*>(row + 64 * G + 16 * kg)[i];
-    };
-    f32x4_t q[NG][4], kc[NG][4], kn[NG][4];
-    load_row(q, P.q + (size_t)(t0 + min(col, nt - 1)) * P.q_ld + h * HD);
+        for (int i = 0; i < 4; ++i) q[G][i] = reinterpret_cast<const f32x4_t*>(row + 64 * G)[i];
+    }
     const int ntile = (pmax >> 4) + 1;
     float lmax[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) lmax[i] = -__builtin_inff();
-    auto load_tile = [&](f32x4_t(&r)[NG][4], int tile) {
-      load_row(r, kcache + (size_t)min(16 * min(tile, ntile - 1) + col, pmax) * HD);
+    // a tile's K as it is loaded: STAGE lane l the 16 bytes l % 16 of rows
+    // 4 i + l / 16; else the operand
+    auto load_tile = [&](int tile) {
+      const int p0 = 16 * min(tile, ntile - 1);
+#pragma unroll
+      for (int G = 0; G < NG; ++G)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int p = STAGE ? p0 + 4 * i + kg : p0 + col;
+          const int e = STAGE ? 64 * G + 4 * col : 64 * G + 16 * kg + 4 * i;
+          kr[G][i] = *reinterpret_cast<const f32x4_t*>(kcache + (size_t)min(p, pmax) * HD + e);
+        }
     };
-    auto run_tile = [&](const f32x4_t(&k)[NG][4], int tile) {
+    load_tile(wave);
+    for (int tile = wave; tile < ntile; tile += NW) {
+      if constexpr (STAGE) {
+#pragma unroll
+        for (int G = 0; G < NG; ++G) {
+          __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses run in order)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4_t*>(kst + (4 * i + kg) * KP + 4 * col) = kr[G][i];
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int i = 0; i < 4; ++i) k[G][i] = *reinterpret_cast<const f32x4_t*>(kst + col * KP + 16 * kg + 4 * i);
+        }
+      } else {
+#pragma unroll
+        for (int G = 0; G < NG; ++G)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) k[G][i] = kr[G][i];
+      }
+      load_tile(tile + NW);
       f32x4_t u[4];  // pair sums (v0+v1), (v2+v3), (v4+v5), (v6+v7)
       static_for<4>([&](auto pr) {
         f32x4_t d[4];  // accumulators 2 pr, 2 pr + 8, 2 pr + 1, 2 pr + 9
@@ -3483,15 +3574,6 @@ __global__ void __launch_bounds__(4 * HD) k_pf_attn(AttnCoreParams P) {
           lmax[i] = (s > lmax[i]) ? s : lmax[i];
         }
       }
-    };
-    // two register sets in turn, the next tile's K in flight
-    load_tile(kc, wave);
-    for (int tile = wave; tile < ntile; tile += 2 * NW) {
-      load_tile(kn, tile + NW);
-      run_tile(kc, tile);
-      if (tile + NW >= ntile) break;  // uniform
-      load_tile(kc, tile + 2 * NW);
-      run_tile(kn, tile + NW);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -3499,6 +3581,25 @@ __global__ void __launch_bounds__(4 * HD) k_pf_attn(AttnCoreParams P) {
       if (col == 0) red_m[wave][4 * kg + i] = m;
     }
   }
+  // ---- AV operands: B of quad q is V[4 q + kg][16 wave + col].  A batch of
+  // VB quads is loaded whole: lane (col, kg) the quads q0 + 4 j + kg of its
+  // dim, 16 bytes each; four registers' lane rows then trade places (turn).
+  // The first batch and the quads from pfirst's on land under the softmax.
+  constexpr int VB = 16;
+  const int nq = (pmax >> 2) + 1, qlast = nq - 1;
+  const int nfull = (pfirst + 1) >> 2;  // quads every token attends whole
+  const int dim = 16 * min(wave, HD / 16 - 1) + col;
+  const f32x4_t* vquads = reinterpret_cast<const f32x4_t*>(vcache);
+  auto load_v = [&](f32x4_t(&v)[VB / 4], int q0) {
+#pragma unroll
+    for (int j = 0; j < VB / 4; ++j) v[j] = vquads[(size_t)min(q0 + 4 * j + kg, qlast) * HD + dim];
+  };
+  f32x4_t va[VB / 4], vb[VB / 4];
+  constexpr int TQ = 5;  // the tail: positions 4 nfull .. pmax, at most 3 + 16
+  f32x4_t vt[TQ];
+  load_v(va, 0);
+#pragma unroll
+  for (int k = 0; k < TQ; ++k) vt[k] = vquads[(size_t)min(nfull + k, qlast) * HD + dim];
   __syncthreads();
   if (tid < nt) {
     float m = red_m[0][tid];
@@ -3511,109 +3612,132 @@ __global__ void __launch_bounds__(4 * HD) k_pf_attn(AttnCoreParams P) {
   __syncthreads();
   // ---- exps, four positions per thread; 0 past a token's last position
   // (up to whole quads of the block)
-  const int nq = (pmax >> 2) + 1;
   for (int i = tid; i < nt * nq; i += NT) {
     const int r = i / nq, p = 4 * (i - r * nq);
     const float m = mx_s[r];
-    float4* at = reinterpret_cast<float4*>(sc + r * ld + p);
-    const float4 s = *at;
-    const int last = pfirst + r;
-    float4 e;
-    e.x = (p + 0 <= last) ? (float)exp((double)(s.x - m)) : 0.0f;
-    e.y = (p + 1 <= last) ? (float)exp((double)(s.y - m)) : 0.0f;
-    e.z = (p + 2 <= last) ? (float)exp((double)(s.z - m)) : 0.0f;
-    e.w = (p + 3 <= last) ? (float)exp((double)(s.w - m)) : 0.0f;
+    f32x4_t* at = reinterpret_cast<f32x4_t*>(sc + r * ld + p);
+    const f32x4_t s = *at;
+    f32x4_t e;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float x = exp_f32(s[c] - m, exp_tab);
+      e[c] = (p + c <= pfirst + r) ? x : 0.0f;
+    }
     *at = e;
   }
-  // ---- AV operands: B lane (col, kg) dim 16 wave + col of position 4 quad
-  // + kg; the first batch of V and the quads from pfirst's on land under
-  // the sums
-  constexpr int VB = 16;                       // quads per batch
-  const int nfull = (pfirst + 1) >> 2;         // quads every token attends whole
-  const unsigned vl = (unsigned)(16 * wave + col) * 4 + kg;
-  const int qlast = nq - 1;
-  float va[VB], vb[VB];
-  auto load_v = [&](float(&v)[VB], int q0) {
-#pragma unroll
-    for (int k = 0; k < VB; ++k) v[k] = (vcache + (size_t)min(q0 + k, qlast) * (4 * HD))[vl];
-  };
-  load_v(va, 0);
-  constexpr int TQ = 5;  // the tail: positions 4 nfull .. pmax, at most 3 + 16
-  f32x4_t vt[TQ];
-#pragma unroll
-  for (int k = 0; k < TQ; ++k)
-    vt[k] = reinterpret_cast<const f32x4_t*>(vcache)[(size_t)min(nfull + k, qlast) * HD + 16 * wave + col];
   __syncthreads();
   const float* arow = sc + min(col, nt - 1) * ld + kg;  // A: token col, position 4 quad + kg
+  auto load_a = [&](float(&a)[VB], int q0) {
+#pragma unroll
+    for (int k = 0; k < VB; ++k) a[k] = arow[4 * min(q0 + k, qlast)];
+  };
   // ---- sums: wave 0, all of the block's tokens at once
   if (wave == 0) {
     f32x4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
-    int q = 0;
-    for (; q + VB <= nq; q += VB) {
-      float a[VB];
+    auto run = [&](const float(&a)[VB], int n) {
+      if (n >= VB) {  // uniform
 #pragma unroll
-      for (int k = 0; k < VB; ++k) a[k] = arow[4 * (q + k)];
+        for (int k = 0; k < VB; ++k) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], 1.0f, s, 0, 0, 0);
+      } else {
 #pragma unroll
-      for (int k = 0; k < VB; ++k) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], 1.0f, s, 0, 0, 0);
+        for (int k = 0; k < VB; ++k)
+          if (k < n) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], 1.0f, s, 0, 0, 0);
+      }
+    };
+    float a0[VB], a1[VB];
+    load_a(a0, 0);
+    for (int q0 = 0; q0 < nq; q0 += 2 * VB) {
+      load_a(a1, q0 + VB);
+      issue_fence();
+      run(a0, nq - q0);
+      if (q0 + VB >= nq) break;  // uniform
+      load_a(a0, q0 + 2 * VB);
+      issue_fence();
+      run(a1, nq - q0 - VB);
     }
-    for (; q < nq; ++q) s = __builtin_amdgcn_mfma_f32_16x16x4f32(arow[4 * q], 1.0f, s, 0, 0, 0);
     if (col == 0)
 #pragma unroll
       for (int i = 0; i < 4; ++i) inv_s[4 * kg + i] = 1.0f / s[i];
   }
   __syncthreads();
+  if (wave >= HD / 16) return;  // no barrier follows
 
   // ---- AV: the probabilities are e * (1/sum), formed as they are read
   const float ainv = inv_s[min(col, nt - 1)];
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  auto run_v = [&](const float(&v)[VB], int q0, int n) {
-    float a[VB];
+  auto run_v = [&](f32x4_t(&v)[VB / 4], const float(&a)[VB], int n) {
+    float b[VB];
 #pragma unroll
-    for (int k = 0; k < VB; ++k) a[k] = arow[4 * min(q0 + k, qlast)] * ainv;
+    for (int j = 0; j < VB / 4; ++j) {
+      // lane row kg of v[j][c] holds quad q0 + 4 j + kg, position c: turn to
+      // register k = quad q0 + 4 j + k, lane row kg = position kg
+      uint32_t r0 = __float_as_uint(v[j][0]), r1 = __float_as_uint(v[j][1]), r2 = __float_as_uint(v[j][2]),
+               r3 = __float_as_uint(v[j][3]);
+      auto s02 = __builtin_amdgcn_permlane32_swap(r0, r2, false, false);
+      auto s13 = __builtin_amdgcn_permlane32_swap(r1, r3, false, false);
+      auto x01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+      auto x23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+      b[4 * j + 0] = __uint_as_float(x01[0]);
+      b[4 * j + 1] = __uint_as_float(x01[1]);
+      b[4 * j + 2] = __uint_as_float(x23[0]);
+      b[4 * j + 3] = __uint_as_float(x23[1]);
+    }
     if (n >= VB) {  // uniform
 #pragma unroll
-      for (int k = 0; k < VB; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], v[k], acc, 0, 0, 0);
+      for (int k = 0; k < VB; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k] * ainv, b[k], acc, 0, 0, 0);
     } else {
 #pragma unroll
       for (int k = 0; k < VB; ++k)
-        if (k < n) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], v[k], acc, 0, 0, 0);
+        if (k < n) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k] * ainv, b[k], acc, 0, 0, 0);
     }
   };
+  float a0[VB], a1[VB];
+  load_a(a0, 0);
   for (int q0 = 0; q0 < nfull; q0 += 2 * VB) {
     load_v(vb, q0 + VB);
-    run_v(va, q0, nfull - q0);
+    load_a(a1, q0 + VB);
+    issue_fence();
+    run_v(va, a0, nfull - q0);
     if (q0 + VB >= nfull) break;  // uniform
     load_v(va, q0 + 2 * VB);
-    run_v(vb, q0 + VB, nfull - q0 - VB);
+    load_a(a0, q0 + 2 * VB);
+    issue_fence();
+    run_v(vb, a1, nfull - q0 - VB);
   }
   // the tail, position by position against each token's last
   float rinv[4];
+  f32x4_t et[2][4];  // a quad of each of the lane's tokens, the next one in flight
+  auto load_e = [&](f32x4_t(&e)[4], int k) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      e[i] = *reinterpret_cast<const f32x4_t*>(sc + min(4 * kg + i, nt - 1) * ld + 4 * min(nfull + k, qlast));
+  };
 #pragma unroll
   for (int i = 0; i < 4; ++i) rinv[i] = inv_s[4 * kg + i];
+  load_e(et[0], 0);
 #pragma unroll
   for (int k = 0; k < TQ; ++k) {
     const int p = 4 * (nfull + k);
     if (p > pmax) break;  // uniform
+    load_e(et[(k + 1) & 1], k + 1);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 4 * kg + i, last = pfirst + r;
-      const float4 e = *reinterpret_cast<const float4*>(sc + min(r, nt - 1) * ld + p);
-      float a = acc[i];
-      a = (p + 0 <= last) ? __builtin_fmaf(e.x * rinv[i], vt[k].x, a) : a;
-      a = (p + 1 <= last) ? __builtin_fmaf(e.y * rinv[i], vt[k].y, a) : a;
-      a = (p + 2 <= last) ? __builtin_fmaf(e.z * rinv[i], vt[k].z, a) : a;
-      a = (p + 3 <= last) ? __builtin_fmaf(e.w * rinv[i], vt[k].w, a) : a;
-      acc[i] = a;
-    }
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a = __builtin_fmaf(et[k & 1][i][c] * rinv[i], vt[k][c], acc[i]);
+        acc[i] = (p + c <= pfirst + 4 * kg + i) ? a : acc[i];
+      }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 4 * kg + i;
-    if (r < nt) P.out[(size_t)(t0 + r) * P.out_ld + h * HD + 16 * wave + col] = acc[i];
+    if (r < nt) P.out[(size_t)(t0 + r) * P.out_ld + h * HD + dim] = acc[i];
   }
 }
-template __global__ void k_pf_attn<64>(AttnCoreParams);
-template __global__ void k_pf_attn<128>(AttnCoreParams);
+template __global__ void k_pf_attn<64, true>(AttnCoreParams);
+template __global__ void k_pf_attn<64, false>(AttnCoreParams);
+template __global__ void k_pf_attn<128, true>(AttnCoreParams);
+template __global__ void k_pf_attn<128, false>(AttnCoreParams);
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x16_t __attribute__((ext_vector_type(16)));

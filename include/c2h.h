@@ -311,6 +311,10 @@ int c2h_time_producer_consumer(c2h_ctx* ctx, int32_t n_prod, int32_t n_cons, int
  * pattern (0xffffffff if none). */
 int c2h_check_rms_scale(c2h_ctx* ctx, uint32_t lo, uint64_t hi, uint64_t* mismatches, uint32_t* first_bits);
 
+/* The same for the softmax's f32(exp(f64(t))), t <= 0 or NaN (patterns 0 and
+ * 0x80000000 up), against the library's f64 exp. */
+int c2h_check_exp(c2h_ctx* ctx, uint32_t lo, uint64_t hi, uint64_t* mismatches, uint32_t* first_bits);
+
 /* Kernels of one decoder layer, for c2h_time_layer_kernel. */
 #define C2H_KERNEL_QKV 0        /* RMSNorm + Q8_K + q|k|v GEMV + bias */
 #define C2H_KERNEL_ATTN 1       /* RoPE, KV store, scores, softmax, AV */

@@ -32,6 +32,14 @@ def test_rms_scale_every_float(ctx):
     assert bad == 0, f"{bad} mismatches, first at {first:#010x}"
 
 
+@pytest.mark.parametrize("lo,hi", [(0, 1), (0x7F800001, 1 << 31), (1 << 31, 1 << 32)])
+def test_softmax_exp_every_float(ctx, lo, hi):
+    # f32(exp(f64(t))) of tensor/ops.go:327-330 as the kernels compute it for
+    # t <= 0 (and NaN): +0, the NaNs, every negative float
+    bad, first = ctx.check_exp(lo, hi)
+    assert bad == 0, f"{bad} mismatches, first at {first:#010x}"
+
+
 @pytest.mark.parametrize("cols", [256, 512, 896, 4864, 16384])
 def test_quantize_q8k_bitexact(ctx, cols):
     rng = np.random.default_rng(cols)
