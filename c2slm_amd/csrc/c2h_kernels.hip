@@ -3472,7 +3472,7 @@ __device__ __forceinline__ float row_max_dpp(float x) {
 // one-dimensional and runs the blocks from the last (longest) to the first;
 // the dispatcher hands each freed slot the next block.
 template <int HD, bool STAGE>
-__global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
+__global__ void __launch_bounds__(64 * PFA_NW) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 2))) k_pf_attn(AttnCoreParams P) {
   constexpr int NW = PFA_NW;
   constexpr int NT = 64 * NW;
   constexpr int NG = HD / 64;  // groups of four chain steps of a score
@@ -3506,7 +3506,7 @@ __global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
   // positions repeat the last one (finite or not, they touch no other row).
   {
     float* kst = sc + P.tok_blk * ld + wave * (16 * KP);  // STAGE: this wave's K rows, one group of 64 elements
-    f32x4_t q[NG][4], k[NG][4], kr[NG][4];
+    f32x4_t q[NG][4], kr[NG][4];
     {
       const float* row = P.q + (size_t)(t0 + min(col, nt - 1)) * P.q_ld + h * HD + 16 * kg;
 #pragma unroll
@@ -3519,61 +3519,86 @@ __global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) lmax[i] = -__builtin_inff();
     // a tile's K as it is loaded: STAGE lane l the 16 bytes l % 16 of rows
-    // 4 i + l / 16; else the operand
+    // 4 i + l / 16; else the operand.  Rows past pmax read zeros.
+    const __amdgpu_buffer_rsrc_t krs = cache_rsrc(kcache, (pmax + 1) * HD * 4);
+    const int koff = (STAGE ? kg * HD + 4 * col : col * HD + 16 * kg) * 4;
     auto load_tile = [&](int tile) {
-      const int p0 = 16 * min(tile, ntile - 1);
 #pragma unroll
       for (int G = 0; G < NG; ++G)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int p = STAGE ? p0 + 4 * i + kg : p0 + col;
-          const int e = STAGE ? 64 * G + 4 * col : 64 * G + 16 * kg + 4 * i;
-          kr[G][i] = *reinterpret_cast<const f32x4_t*>(kcache + (size_t)min(p, pmax) * HD + e);
-        }
+        for (int i = 0; i < 4; ++i)
+          kr[G][i] = cache_ld4(krs, tile * (16 * HD * 4) + koff + (64 * G + (STAGE ? 4 * i * HD : 4 * i)) * 4);
     };
-    load_tile(wave);
-    for (int tile = wave; tile < ntile; tile += NW) {
-      if constexpr (STAGE) {
+    // the loaded tile as operands (a wave's LDS accesses run in order)
+    auto operands = [&](f32x4_t(&k)[NG][4]) {
 #pragma unroll
-        for (int G = 0; G < NG; ++G) {
-          __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses run in order)
+      for (int G = 0; G < NG; ++G) {
+        if constexpr (STAGE) {
+          __builtin_amdgcn_wave_barrier();
 #pragma unroll
           for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4_t*>(kst + (4 * i + kg) * KP + 4 * col) = kr[G][i];
           __builtin_amdgcn_wave_barrier();
 #pragma unroll
           for (int i = 0; i < 4; ++i) k[G][i] = *reinterpret_cast<const f32x4_t*>(kst + col * KP + 16 * kg + 4 * i);
-        }
-      } else {
-#pragma unroll
-        for (int G = 0; G < NG; ++G)
+        } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i) k[G][i] = kr[G][i];
+        }
       }
-      load_tile(tile + NW);
-      f32x4_t u[4];  // pair sums (v0+v1), (v2+v3), (v4+v5), (v6+v7)
+    };
+    int at[4];  // the lane's rows of the scores (past nt: row nt - 1, whose token they repeat)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) at[i] = min(4 * kg + i, nt - 1) * ld + col;
+    auto run_tile = [&](const f32x4_t(&k)[NG][4], int tile) {
+      // accumulators 2 pr, 2 pr + 8, 2 pr + 1, 2 pr + 9, the sums of the
+      // group before between them
+      f32x4_t d[2][4], u[4];
+      auto sum = [&](auto pr, auto x) {
+        const f32x4_t(&e)[4] = d[(int)pr & 1];
+        u[(int)pr][(int)x] = (e[0][(int)x] + e[1][(int)x]) + (e[2][(int)x] + e[3][(int)x]);
+      };
       static_for<4>([&](auto pr) {
-        f32x4_t d[4];  // accumulators 2 pr, 2 pr + 8, 2 pr + 1, 2 pr + 9
-        static_for<NG>([&](auto G) {
+        static_for<4>([&](auto x) {
+          constexpr int c = 2 * (int)pr + ((int)x >> 1) + 8 * ((int)x & 1);
+          const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+          issue_fence();
+          d[(int)pr & 1][(int)x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[0][c / 4][c % 4], k[0][c / 4][c % 4], zero, 0, 0, 0);
+          if constexpr ((int)pr > 0) sum(std::integral_constant<int, (int)pr - 1>{}, x);
+        });
+        if constexpr (NG > 1)
           static_for<4>([&](auto x) {
             constexpr int c = 2 * (int)pr + ((int)x >> 1) + 8 * ((int)x & 1);
-            const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-            d[(int)x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[(int)G][c / 4][c % 4], k[(int)G][c / 4][c % 4],
-                                                             (int)G == 0 ? zero : d[(int)x], 0, 0, 0);
+            f32x4_t& e = d[(int)pr & 1][(int)x];
+            e = __builtin_amdgcn_mfma_f32_16x16x4f32(q[NG - 1][c / 4][c % 4], k[NG - 1][c / 4][c % 4], e, 0, 0, 0);
           });
-        });
-#pragma unroll
-        for (int i = 0; i < 4; ++i) u[(int)pr][i] = (d[0][i] + d[1][i]) + (d[2][i] + d[3][i]);
       });
+      issue_fence();
+      static_for<4>([&](auto x) { sum(std::integral_constant<int, 3>{}, x); });
       const int p = 16 * tile + col;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 4 * kg + i;
         const float s = ((u[0][i] + u[1][i]) + (u[2][i] + u[3][i])) * P.scale;
-        if (r < nt && p <= pfirst + r) {
-          sc[r * ld + p] = s;
-          lmax[i] = (s > lmax[i]) ? s : lmax[i];
-        }
+        sc[at[i] + 16 * tile] = s;  // (the exps write 0 past a token's last position)
+        const float sm = (p <= pfirst + min(4 * kg + i, nt - 1)) ? s : -__builtin_inff();
+        lmax[i] = (sm > lmax[i]) ? sm : lmax[i];
       }
+    };
+    // the next tile's operands are read from LDS, the one after's loaded,
+    // while a tile's MFMAs run
+    f32x4_t k0[NG][4], k1[NG][4];
+    load_tile(wave);
+    operands(k0);
+    load_tile(wave + NW);
+    for (int tile = wave; tile < ntile; tile += 2 * NW) {
+      operands(k1);
+      load_tile(tile + 2 * NW);
+      issue_fence();
+      run_tile(k0, tile);
+      if (tile + NW >= ntile) break;  // uniform
+      operands(k0);
+      load_tile(tile + 3 * NW);
+      issue_fence();
+      run_tile(k1, tile + NW);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -3585,19 +3610,22 @@ __global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
   // VB quads is loaded whole: lane (col, kg) the quads q0 + 4 j + kg of its
   // dim, 16 bytes each; four registers' lane rows then trade places (turn).
   // The first batch and the quads from pfirst's on land under the softmax.
-  constexpr int VB = 16;
+  constexpr int VB = 8;
   const int nq = (pmax >> 2) + 1, qlast = nq - 1;
   const int nfull = (pfirst + 1) >> 2;  // quads every token attends whole
   const int dim = 16 * min(wave, HD / 16 - 1) + col;
   const f32x4_t* vquads = reinterpret_cast<const f32x4_t*>(vcache);
+  const __amdgpu_buffer_rsrc_t vrs = cache_rsrc(vcache, nq * HD * 16);  // quads past the last read zeros
+  const int voff = (kg * HD + dim) * 16;
   auto load_v = [&](f32x4_t(&v)[VB / 4], int q0) {
 #pragma unroll
-    for (int j = 0; j < VB / 4; ++j) v[j] = vquads[(size_t)min(q0 + 4 * j + kg, qlast) * HD + dim];
+    for (int j = 0; j < VB / 4; ++j) v[j] = cache_ld4(vrs, (q0 + 4 * j) * (HD * 16) + voff);
   };
   f32x4_t va[VB / 4], vb[VB / 4];
   constexpr int TQ = 5;  // the tail: positions 4 nfull .. pmax, at most 3 + 16
   f32x4_t vt[TQ];
   load_v(va, 0);
+  load_v(vb, VB);
 #pragma unroll
   for (int k = 0; k < TQ; ++k) vt[k] = vquads[(size_t)min(nfull + k, qlast) * HD + dim];
   __syncthreads();
@@ -3611,9 +3639,10 @@ __global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
   }
   __syncthreads();
   // ---- exps, four positions per thread; 0 past a token's last position
-  // (up to whole quads of the block)
-  for (int i = tid; i < nt * nq; i += NT) {
-    const int r = i / nq, p = 4 * (i - r * nq);
+  // (up to whole batches of VB quads)
+  const int nqb = (nq + VB - 1) & ~(VB - 1);
+  for (int i = tid; i < nt * nqb; i += NT) {
+    const int r = i / nqb, p = 4 * (i - r * nqb);
     const float m = mx_s[r];
     f32x4_t* at = reinterpret_cast<f32x4_t*>(sc + r * ld + p);
     const f32x4_t s = *at;
@@ -3627,33 +3656,34 @@ __global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
   }
   __syncthreads();
   const float* arow = sc + min(col, nt - 1) * ld + kg;  // A: token col, position 4 quad + kg
-  auto load_a = [&](float(&a)[VB], int q0) {
+  auto load_a = [&](float(&a)[VB], int q0) {  // (batches past the last read it again)
+    const float* at = arow + 4 * min(q0, nqb - VB);
 #pragma unroll
-    for (int k = 0; k < VB; ++k) a[k] = arow[4 * min(q0 + k, qlast)];
+    for (int k = 0; k < VB; ++k) a[k] = at[4 * k];
   };
-  // ---- sums: wave 0, all of the block's tokens at once
+  // ---- sums: wave 0, all of the block's tokens at once; a batch's reads go
+  // out between the dependent MFMAs of the one before
   if (wave == 0) {
     f32x4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto run = [&](const float(&a)[VB], int n) {
-      if (n >= VB) {  // uniform
+    auto run = [&](const float(&a)[VB]) {
 #pragma unroll
-        for (int k = 0; k < VB; ++k) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], 1.0f, s, 0, 0, 0);
-      } else {
+      for (int k = 0; k < VB; ++k) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], 1.0f, s, 0, 0, 0);
 #pragma unroll
-        for (int k = 0; k < VB; ++k)
-          if (k < n) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], 1.0f, s, 0, 0, 0);
+      for (int k = 0; k < VB; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
       }
     };
     float a0[VB], a1[VB];
     load_a(a0, 0);
-    for (int q0 = 0; q0 < nq; q0 += 2 * VB) {
+    for (int q0 = 0; q0 < nqb; q0 += 2 * VB) {
+      issue_fence();
       load_a(a1, q0 + VB);
+      run(a0);
+      if (q0 + VB >= nqb) break;  // uniform
       issue_fence();
-      run(a0, nq - q0);
-      if (q0 + VB >= nq) break;  // uniform
       load_a(a0, q0 + 2 * VB);
-      issue_fence();
-      run(a1, nq - q0 - VB);
+      run(a1);
     }
     if (col == 0)
 #pragma unroll
@@ -3665,45 +3695,64 @@ __global__ void __launch_bounds__(64 * PFA_NW) k_pf_attn(AttnCoreParams P) {
   // ---- AV: the probabilities are e * (1/sum), formed as they are read
   const float ainv = inv_s[min(col, nt - 1)];
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  auto run_v = [&](f32x4_t(&v)[VB / 4], const float(&a)[VB], int n) {
-    float b[VB];
+  // lane row kg of v[c] holds quad Q + kg, position c: turn to b[c'] =
+  // quad Q + c', lane row kg = position kg
+  auto turn = [&](const f32x4_t& v, float* b) {
+    // the swaps work in place: on copies, so that v's registers are free for
+    // the next load (else the loop copied them, waiting for the load)
+    uint32_t r[4];
 #pragma unroll
-    for (int j = 0; j < VB / 4; ++j) {
-      // lane row kg of v[j][c] holds quad q0 + 4 j + kg, position c: turn to
-      // register k = quad q0 + 4 j + k, lane row kg = position kg
-      uint32_t r0 = __float_as_uint(v[j][0]), r1 = __float_as_uint(v[j][1]), r2 = __float_as_uint(v[j][2]),
-               r3 = __float_as_uint(v[j][3]);
-      auto s02 = __builtin_amdgcn_permlane32_swap(r0, r2, false, false);
-      auto s13 = __builtin_amdgcn_permlane32_swap(r1, r3, false, false);
-      auto x01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
-      auto x23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
-      b[4 * j + 0] = __uint_as_float(x01[0]);
-      b[4 * j + 1] = __uint_as_float(x01[1]);
-      b[4 * j + 2] = __uint_as_float(x23[0]);
-      b[4 * j + 3] = __uint_as_float(x23[1]);
-    }
-    if (n >= VB) {  // uniform
-#pragma unroll
-      for (int k = 0; k < VB; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k] * ainv, b[k], acc, 0, 0, 0);
-    } else {
-#pragma unroll
-      for (int k = 0; k < VB; ++k)
-        if (k < n) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k] * ainv, b[k], acc, 0, 0, 0);
-    }
+    for (int c = 0; c < 4; ++c) asm volatile("v_mov_b32 %0, %1" : "=v"(r[c]) : "v"(v[c]));
+    const auto s02 = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
+    const auto s13 = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+    const auto x01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+    const auto x23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+    b[0] = __uint_as_float(x01[0]);
+    b[1] = __uint_as_float(x01[1]);
+    b[2] = __uint_as_float(x23[0]);
+    b[3] = __uint_as_float(x23[1]);
   };
-  float a0[VB], a1[VB];
+  // a batch's MFMAs; between them (each waits 32 clk for the one before) the
+  // next batch's operands are read and turned and the V of the third one
+  // loaded into the registers just turned.  Pinned slot by slot: left alone,
+  // the scheduler put all of it after the MFMAs and loaded V through copies
+  // that waited for it (82 clk per MFMA instead of 35).
+  float a0[VB], a1[VB], b0[VB], b1[VB];
+  auto step = [&](const float(&a)[VB], const float(&b)[VB], float(&an)[VB], float(&bn)[VB], f32x4_t(&v)[VB / 4], int q0) {
+    const float* at = arow + 4 * min(q0 + VB, nqb - VB);
+    float am = a[0] * ainv;
+    static_for<VB>([&](auto kc) {
+      constexpr int k = (int)kc;
+      issue_fence();
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(am, b[k], acc, 0, 0, 0);
+      if constexpr (k + 1 < VB) am = a[k + 1] * ainv;
+      an[k] = at[4 * k];
+      if constexpr (k % 4 == 1) turn(v[k / 4], bn + 4 * (k / 4));
+      if constexpr (k % 4 == 3) v[k / 4] = cache_ld4(vrs, (q0 + 3 * VB + 4 * (k / 4)) * (HD * 16) + voff);
+    });
+    issue_fence();
+  };
   load_a(a0, 0);
-  for (int q0 = 0; q0 < nfull; q0 += 2 * VB) {
-    load_v(vb, q0 + VB);
-    load_a(a1, q0 + VB);
-    issue_fence();
-    run_v(va, a0, nfull - q0);
-    if (q0 + VB >= nfull) break;  // uniform
-    load_v(va, q0 + 2 * VB);
-    load_a(a0, q0 + 2 * VB);
-    issue_fence();
-    run_v(vb, a1, nfull - q0 - VB);
+#pragma unroll
+  for (int j = 0; j < VB / 4; ++j) turn(va[j], b0 + 4 * j);
+  load_v(va, 2 * VB);
+  int q0 = 0;
+  for (; q0 + 2 * VB <= nfull; q0 += 2 * VB) {
+    step(a0, b0, a1, b1, vb, q0);
+    step(a1, b1, a0, b0, va, q0 + VB);
   }
+  if (q0 + VB <= nfull) {  // uniform
+    step(a0, b0, a1, b1, vb, q0);
+    q0 += VB;
+#pragma unroll
+    for (int k = 0; k < VB; ++k) {
+      a0[k] = a1[k];
+      b0[k] = b1[k];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < VB; ++k)
+    if (q0 + k < nfull) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[k] * ainv, b0[k], acc, 0, 0, 0);  // uniform
   // the tail, position by position against each token's last
   float rinv[4];
   f32x4_t et[2][4];  // a quad of each of the lane's tokens, the next one in flight
