@@ -1429,10 +1429,6 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
   for (const void* k : {(const void*)k_pf_gemm_q6<MODE_BIAS, 2>, (const void*)k_pf_gemm_q6<MODE_RESID, 2>})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, PF_Q6_LDS_MAX) != hipSuccess)
       return bail(fail(c, C2H_ERR_HIP, "prefill Q6_K GEMM LDS attribute"));
-  for (const void* k : {(const void*)k_pf_gemm_f<MODE_BIAS>, (const void*)k_pf_gemm_f<MODE_RESID>,
-                        (const void*)k_pf_gemm_q50<MODE_BIAS>, (const void*)k_pf_gemm_q50<MODE_RESID>})
-    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, PF_F_LDS_MAX) != hipSuccess)
-      return bail(fail(c, C2H_ERR_HIP, "prefill GEMM LDS attribute"));
   for (const void* k : {(const void*)k_pf_attn<64, true>, (const void*)k_pf_attn<64, false>,
                         (const void*)k_pf_attn<128, true>, (const void*)k_pf_attn<128, false>})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PFA_LDS_MAX) != hipSuccess)
@@ -1648,10 +1644,28 @@ PFGemmKernel pf_gemm_kernel(int type, int mode, bool small_tile = false, int q6_
 // A Q4_K launch whose 64 x 64 tiles would leave CUs idle runs 64-row x
 // 16-token workgroups instead (four times as many).
 constexpr int PF_SMALL_TILE_WG = 512;
+constexpr int PF_Q50_MIN_WAVES = 2048;
+
+// Tokens per wave of a k_pf_gemm_q50 launch and the waves a tile's blocks
+// are split over: sixteen and none while that gives each SIMD two waves (its
+// VALU's full rate), else eight (the decoding of a block's quants, ~100
+// instructions, is then for 512 products' instead of 1,024) and as many
+// waves as bring it about and leave each four blocks or more.
+void pf_q50_split(int row_tiles, int m, int n_x, int* tok, PFGemmFParams* F) {
+  const int nb8 = n_x / 32;
+  F->ks = 1;
+  *tok = 16;
+  if (row_tiles * ((m + 15) / 16) < PF_Q50_MIN_WAVES) {
+    *tok = PF_Q50_KS_TOK;
+    const int tiles = row_tiles * ((m + *tok - 1) / *tok);
+    while (F->ks < PF_Q50_KS_MAX && tiles * F->ks < PF_Q50_MIN_WAVES && nb8 / (2 * F->ks) >= 4) F->ks *= 2;
+  }
+  F->per = std::min((nb8 + F->ks - 1) / F->ks, PF_Q50_PER_MAX);
+}
 
 // y[t][r] (=|+=) W * x[t] for the given matrices: Q4_K / Q6_K on the
 // Q8_K rows (one MFMA launch per type), Q5_0 / Q8_0 on the f32 rows xf
-// (one k_pf_gemm_f launch), as engine/model.go:250-270 dispatches.
+// (a launch per type), as engine/model.go:250-270 dispatches.
 void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_list<const Tensor*> ws,
              std::initializer_list<float*> ys, std::initializer_list<const float*> biases,
              std::initializer_list<int> ldys, const float* xf, int ldxf, int n_x) {
@@ -1696,27 +1710,23 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
                          c->stream, P);
     }
   }
-  // float-input jobs: Q5_0 rows of up to PF_Q50_MAXB blocks in one
-  // k_pf_gemm_q50 launch, the others (Q8_0, wider Q5_0) in one k_pf_gemm_f
-  const int nb8 = n_x / 32;
-  for (int batched = 1; batched >= 0; --batched) {
+  // float-input jobs: Q5_0 in one k_pf_gemm_q50 launch, Q8_0 in one k_pf_gemm_f
+  for (int type : {(int)C2H_Q5_0, (int)C2H_Q8_0}) {
     PFGemmFParams F;
     memset(&F, 0, sizeof(F));
     F.x = xf;
     F.ldx = ldxf;
     F.n_x = n_x;
     F.m = m;
+    const int R = type == C2H_Q5_0 ? PF_Q50_ROWS : 32;
     int tiles = 0;
     for (size_t i = 0; i < W.size(); ++i) {
-      if (!float_input(W[i]->type)) continue;
-      const bool q50b = W[i]->type == C2H_Q5_0 && nb8 <= PF_Q50_MAXB;
-      if (q50b != (batched == 1)) continue;
+      if (W[i]->type != type) continue;
       PFJob& J = F.jobs[F.n_jobs++];
       J.w = W[i]->ref();
       J.type = W[i]->type;
       J.rows = (int)W[i]->rows;
       J.tile_begin = tiles;
-      const int R = (J.type == C2H_Q5_0) ? std::max(1, 256 / nb8) : 32;
       tiles += (J.rows + R - 1) / R;
       J.mode = mode;
       J.y = Y[i];
@@ -1724,10 +1734,16 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
       J.bias = B[i];
     }
     if (F.n_jobs == 0) continue;
-    if (batched) {
-      auto k = (mode == MODE_RESID) ? k_pf_gemm_q50<MODE_RESID> : k_pf_gemm_q50<MODE_BIAS>;
-      hipLaunchKernelGGL(k, dim3(tiles, (m + PF_FT - 1) / PF_FT), dim3(256), (size_t)pf_gemm_q50_lds_bytes(n_x),
-                         c->stream, F);
+    if (type == C2H_Q5_0) {
+      int tok;
+      pf_q50_split(tiles, m, n_x, &tok, &F);
+      F.n_tiles = tiles;
+      auto k = mode == MODE_RESID ? k_pf_gemm_q50<MODE_RESID, 16, false> : k_pf_gemm_q50<MODE_BIAS, 16, false>;
+      if (tok == 8) k = mode == MODE_RESID ? k_pf_gemm_q50<MODE_RESID, 8, false> : k_pf_gemm_q50<MODE_BIAS, 8, false>;
+      if (F.ks > 1) k = mode == MODE_RESID ? k_pf_gemm_q50<MODE_RESID, 8, true> : k_pf_gemm_q50<MODE_BIAS, 8, true>;
+      const dim3 grid(F.ks > 1 ? tiles : (tiles + PF_Q50_TW - 1) / PF_Q50_TW, (m + tok - 1) / tok);
+      hipLaunchKernelGGL(k, grid, dim3(64 * (F.ks > 1 ? F.ks : PF_Q50_TW)),
+                         (size_t)pf_gemm_q50_lds_bytes(F.ks, F.per), c->stream, F);
     } else {
       // tokens one after another per workgroup: fewer of them when the rows
       // alone would leave CUs idle (the 128 rows of attn_v)
@@ -1774,17 +1790,6 @@ int pf_attn_tokens(int n_heads, int m, int pmax) {
   while (tb > 4 && n_heads * ((m + tb - 1) / tb) < PFA_MIN_WG) tb /= 2;
   while (tb > 1 && pfa_lds_bytes(tb, pmax, true) > PFA_LDS_MAX) tb /= 2;
   return tb;
-}
-
-// Whether prompts run the batched kernels.  A Q5_0 ffn_down wider than
-// k_pf_gemm_f's workgroup takes (its LDS, one thread per block of a row)
-// leaves one forward per token.
-bool pf_batched(const c2h_ctx* c) {
-  if (c->desc.head_dim == 64) return true;
-  for (const Layer& L : c->layers)
-    if (float_input(L.wd.type) && (pf_gemm_f_lds_bytes(c->desc.n_ff) > PF_F_LDS_MAX || c->desc.n_ff / 32 > 256))
-      return false;
-  return true;
 }
 
 // One pass of up to PF_MAX tokens at positions pos0.. (engine.Forward per
@@ -1920,35 +1925,15 @@ int c2h_prefill(c2h_ctx* c, const int32_t* tokens, int32_t n, int32_t pos0, floa
   if (pos0 < 0 || (int64_t)pos0 + n > c->desc.max_ctx)
     return fail(c, C2H_ERR_RANGE, "positions [%d, %d) outside [0, %d)", pos0, pos0 + n, c->desc.max_ctx);
   if (n == 0) return C2H_OK;
-  if (!pf_batched(c)) {
-    // one forward graph per token, as engine.IngestFrom runs Forward per
-    // token (c2slm.go:103-114)
-    if ((rc = build_graphs(c))) return rc;
-    for (int i = 0; i < n; ++i) {
-      C2hState s;
-      memset(&s, 0, sizeof(s));
-      s.pos = pos0 + i;
-      s.token = tokens[i];
-      s.penalty = 1.15f;
-      s.nx_in = c->nx_cur;
-      s.nx_out = c->nx_cur ^ 1;
-      if ((rc = push_state(c, s)) || (rc = run_graph(c, false, pos0 + i))) return rc;
-      c->nx_prev = c->nx_cur;
-      c->nx_cur ^= 1;
-      c->seq_len = pos0 + i + 1;
-    }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-  } else {
-    if ((rc = pf_alloc(c)) || (rc = pf_q6_ready(c))) return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    c->ring_next = 0;
-    for (int done = 0; done < n;) {
-      const int m = std::min(n - done, PF_MAX);
-      if ((rc = pf_pass(c, tokens + done, m, pos0 + done))) return rc;
-      HIPCHK(c, hipStreamSynchronize(c->stream));  // tokens are copied from the caller's buffer
-      done += m;
-      c->seq_len = pos0 + done;
-    }
+  if ((rc = pf_alloc(c)) || (rc = pf_q6_ready(c))) return rc;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->ring_next = 0;
+  for (int done = 0; done < n;) {
+    const int m = std::min(n - done, PF_MAX);
+    if ((rc = pf_pass(c, tokens + done, m, pos0 + done))) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));  // tokens are copied from the caller's buffer
+    done += m;
+    c->seq_len = pos0 + done;
   }
   if (normx_out)
     HIPCHK(c, stream_copy(c->stream, normx_out, c->normx[c->nx_cur], (size_t)c->desc.n_embd * 4,

@@ -369,17 +369,19 @@ struct PFGemmParams {
   PFJob jobs[3];
 };
 
-// Q5_0 / Q8_0 jobs of a batch on f32 rows x[t*ldx .. + n_x); grid (row
-// tiles of the jobs, ceil(m / PF_FT)); tile_begin counts row tiles of
-// max(1, 256/(n_x/32)) rows (Q5_0) or 32 rows (Q8_0).
-constexpr int PF_FT = 16;  // tokens per k_pf_gemm_f workgroup
-constexpr int PF_Q50_MAXB = 32;  // Q5_0 blocks per row of k_pf_gemm_q50 (wider rows run k_pf_gemm_f)
+// Q5_0 (k_pf_gemm_q50) or Q8_0 (k_pf_gemm_f) jobs of a batch on f32 rows
+// x[t*ldx .. + n_x); tile_begin counts row tiles of PF_Q50_ROWS or 32 rows.
+constexpr int PF_FT = 16;        // tokens per k_pf_gemm_f workgroup, at most
+constexpr int PF_Q50_ROWS = 64;  // rows of a k_pf_gemm_q50 wave
+constexpr int PF_Q50_TW = 4;     // row tiles per workgroup (ks = 1)
 struct PFGemmFParams {
   const float* x;
   int ldx;
   int n_x;
   int m;
   int ft;  // k_pf_gemm_f: tokens per workgroup (<= PF_FT)
+  int ks, per;  // k_pf_gemm_q50: waves a tile's blocks are split over, blocks of each and round (ks = 1: none)
+  int n_tiles;  // k_pf_gemm_q50: row tiles of all jobs
   int n_jobs;
   PFJob jobs[3];
 };
@@ -428,16 +430,14 @@ __global__ void k_gemv_row(const float* xp, int n_xp, GemvParams P);  // xp, n_x
 template <int PRO, int MODE>
 __global__ void k_gemv_f(GemvParams P);
 constexpr int GF_XPAD = 36;  // floats per 32-element block of x in LDS (Q5_0 reads, bank spread)
-// Dynamic LDS of k_pf_gemm_f, bytes: x of one token in both layouts.
-__host__ __device__ inline int pf_gemm_f_lds_bytes(int n_x) {
-  const int nb8 = n_x / 32;
-  return (nb8 * GF_XPAD + nb8 * 32) * 4;
+// Dynamic LDS of k_pf_gemm_f, bytes: x of one token.
+__host__ __device__ inline int pf_gemm_f_lds_bytes(int n_x) { return n_x / 32 * 32 * 4; }
+// Dynamic LDS of k_pf_gemm_q50 (KS), bytes: the later waves' terms of a
+// round; at most 48 KB: three workgroups per CU.
+constexpr int PF_Q50_KS_TOK = 8, PF_Q50_KS_MAX = 4, PF_Q50_PER_MAX = 8;
+__host__ __device__ inline int pf_gemm_q50_lds_bytes(int ks, int per) {
+  return (ks - 1) * per * PF_Q50_ROWS * PF_Q50_KS_TOK * 4;
 }
-// Dynamic LDS of k_pf_gemm_q50, bytes: x of half the tokens, the terms.
-__host__ __device__ inline int pf_gemm_q50_lds_bytes(int n_x) {
-  return ((PF_FT / 2) * (n_x / 32) * GF_XPAD + PF_FT * 256) * 4;
-}
-constexpr int PF_F_LDS_MAX = ((PF_FT / 2) * PF_Q50_MAXB * GF_XPAD + PF_FT * 256) * 4;
 // Dynamic LDS of k_gemv_f, in floats: x padded per block | x permuted | norm chain.
 __host__ __device__ inline int gemv_f_lds_floats(int n_x) {
   return (n_x / 32) * GF_XPAD + (n_x / 32) * 32 + chain_lds_floats(n_x);
@@ -525,7 +525,8 @@ constexpr int PF_Q6_LDS_MAX = 128 * 1024;
 
 template <int MODE>
 __global__ void k_pf_gemm_f(PFGemmFParams P);
-template <int MODE>
+// TOK tokens per wave; grid (row tiles / (ks > 1 ? 1 : PF_Q50_TW), token tiles)
+template <int MODE, int TOK, bool KS>
 __global__ void k_pf_gemm_q50(PFGemmFParams P);
 template <int HD>
 __global__ void k_pf_qk(PFRopeParams P);

@@ -3176,39 +3176,26 @@ __global__ void __launch_bounds__(256) k_pf_quant(PFQuantParams P) {
   store_q8_row<NB>(s, P.out, t);
 }
 
-// Q5_0 / Q8_0 projections of a token batch on f32 rows (the decode
-// kernel's per-row arithmetic, k_gemv_f): a workgroup keeps its rows'
-// weights in registers and runs P.ft tokens one after the other.  (Q5_0
-// rows of up to PF_Q50_MAXB blocks run k_pf_gemm_q50.)
+// Q8_0 projections of a token batch on f32 rows (the decode kernel's
+// per-row arithmetic, k_gemv_f): a workgroup keeps its rows' weights in
+// registers and runs P.ft tokens one after the other.
 template <int MODE>
 __global__ void __launch_bounds__(256) k_pf_gemm_f(PFGemmFParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int nb8 = P.n_x / 32;
-  float* xq = reinterpret_cast<float*>(smem);  // [nb8][GF_XPAD]
-  float* xp = xq + nb8 * GF_XPAD;              // [nb8][8][4]
+  float* xp = reinterpret_cast<float*>(smem);  // [nb8][8][4]
   int ji = 0;
 #pragma unroll
   for (int j = 1; j < 3; ++j)
     if (j < P.n_jobs && (int)blockIdx.x >= P.jobs[j].tile_begin) ji = j;
   const PFJob& J = P.jobs[ji];
   const int tid = threadIdx.x;
-  const bool q50 = (J.type == T_Q5_0);
-  const int R = q50 ? max(1, 256 / nb8) : 32;
+  constexpr int R = 32;  // rows, eight lanes each
   const int row0 = ((int)blockIdx.x - J.tile_begin) * R;
-  const int b5 = tid / R, r5 = tid - (tid / R) * R;
-  const int r_local = q50 ? r5 : (tid >> 3);
   const int lane8 = tid & 7;
-  const int row = row0 + r_local;
-  const bool active = q50 ? (b5 < nb8 && row < J.rows) : (row < J.rows);
-  const int row_c = min(row, J.rows - 1);
   const int orow = min(row0 + min(tid, R - 1), J.rows - 1);
-  __shared__ float terms[256];
-  Q50Item w5;
-  Q80Row w8;
-  if (q50)
-    w5 = load_q50(J.w, nb8, row_c, min(b5, nb8 - 1));
-  else
-    w8 = load_q80(J.w, nb8, row_c, lane8);
+  __shared__ float terms[R];
+  const Q80Row w8 = load_q80(J.w, nb8, min(row0 + (tid >> 3), J.rows - 1), lane8);
   const int t0 = blockIdx.y * P.ft;
   const float bias = (MODE == MODE_BIAS && J.bias) ? J.bias[orow] : 0.0f;
   for (int tt = 0; tt < P.ft; ++tt) {
@@ -3216,151 +3203,187 @@ __global__ void __launch_bounds__(256) k_pf_gemm_f(PFGemmFParams P) {
     if (t >= P.m) break;  // uniform
     __syncthreads();      // the previous token's LDS reads are done
     for (int e = tid; e < nb8 * 32; e += 256) {
-      const float v = P.x[(size_t)t * P.ldx + e];
-      const int b = e >> 5, kk = e & 31;
-      xq[b * GF_XPAD + kk] = v;
-      xp[(b * 8 + (kk & 7)) * 4 + (kk >> 3)] = v;
+      const int kk = e & 31;
+      xp[((e >> 5) * 8 + (kk & 7)) * 4 + (kk >> 3)] = P.x[(size_t)t * P.ldx + e];
     }
     __syncthreads();
-    float acc = 0.0f;
-    if (q50) {
-      if (active) terms[r5 * nb8 + b5] = q50_term(w5, xq + b5 * GF_XPAD);
-      __syncthreads();
-      if (tid < R)
-        for (int b = 0; b < nb8; ++b) acc = acc + terms[tid * nb8 + b];
-    } else {
-      acc = q80_row_sum(q80_lane_acc(w8, xp, nb8, lane8));
-      if (lane8 == 0) terms[r_local] = acc;
-      __syncthreads();
-      if (tid < R) acc = terms[tid];
-    }
+    const float acc = q80_row_sum(q80_lane_acc(w8, xp, nb8, lane8));
+    if (lane8 == 0) terms[tid >> 3] = acc;
+    __syncthreads();
     if (tid < R && row0 + tid < J.rows) {
       float* y = J.y + (size_t)t * J.ldy + row0 + tid;
       if (MODE == MODE_RESID)
-        *y = *y + acc;
+        *y = *y + terms[tid];
       else
-        *y = J.bias ? acc + bias : acc;
+        *y = J.bias ? terms[tid] + bias : terms[tid];
     }
   }
 }
 template __global__ void k_pf_gemm_f<MODE_BIAS>(PFGemmFParams);
 template __global__ void k_pf_gemm_f<MODE_RESID>(PFGemmFParams);
 
-// Q5_0 projections of a token batch on f32 rows of up to PF_Q50_MAXB blocks
-// (1,024 columns), each (row, token) in the reference's order
-// (c2_tensor_dot_q5_0: per block sum = ((0 + q0 x0) + q16 x16) + q1 x1 ...
-// as mul-then-add, term = d * sum; the row's terms added in block order).
-// Thread (row r5, block b5) of a workgroup of R = 256 / nb rows decodes its
-// block's 32 quants once into floats.  The workgroup's PF_FT tokens go
-// through in two halves: a half's x is staged in LDS, then each thread
-// runs four tokens' block sums at a time as four interleaved chains and
-// stores the terms; at the end one thread per (token, row) folds the row's
-// terms in block order.  48 KB of LDS and <= 168 registers: three
-// workgroups per CU.
-template <int MODE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) k_pf_gemm_q50(PFGemmFParams P) {
-  constexpr int TH = PF_FT / 2;  // tokens staged at a time
+// Q5_0 projections of a token batch on f32 rows, each (row, token) in the
+// reference's order (DotQ5_0, tensor/ops.go:25-74): per 32-element block
+// sum = ((0 + q0 x0) + q16 x16) + q1 x1 .., every product rounded before it
+// is added, term = d * sum; the row's terms added in block order.
+// Bound by the VALU: a multiply and an add per product, 2.35 clk each on a
+// SIMD with two waves or more (4.7 with one).  So nothing else is done per
+// product: a lane is a row, its block's quants floats in registers, and x
+// comes through scalar loads (a token's x is the same for every lane), the
+// next chunk of 4 tokens x 8 elements in flight under the current one.
+// The form before read x from LDS for every two products, which set its
+// pace; the products as outer products on the FP32 matrix unit, which
+// shares the VALU's time, were slower than the multiplies.  300 tokens, a launch:
+// gate|up 144 us, q|k 24.0, o 24.7 us (226, 26 and 27.7 before).
+// KS (launches whose tiles leave SIMDs idle): the blocks of a tile split
+// over P.ks waves, P.per blocks each and round; the later waves leave their
+// terms in LDS and wave 0 adds them in block order.  Otherwise four waves of a workgroup, the same
+// tokens (a scalar cache line serves them all), consecutive row tiles.
+typedef float f32x8_t __attribute__((ext_vector_type(8)));
+template <int MODE, int TOK, bool KS>
+__global__ void __launch_bounds__(256) k_pf_gemm_q50(PFGemmFParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int nb8 = P.n_x / 32;
-  float* xs = reinterpret_cast<float*>(smem);  // [TH][nb8][GF_XPAD]
-  float* tm = xs + TH * nb8 * GF_XPAD;         // [PF_FT][256]
+  float* tl = reinterpret_cast<float*>(smem);  // KS: [later waves' blocks of a round][TOK][64]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int tile = (int)blockIdx.x * (KS ? 1 : PF_Q50_TW) + (KS ? 0 : wave);
+  if (tile >= P.n_tiles) return;  // (ks = 1: no barrier; else uniform over the workgroup)
   int ji = 0;
 #pragma unroll
   for (int j = 1; j < 3; ++j)
-    if (j < P.n_jobs && (int)blockIdx.x >= P.jobs[j].tile_begin) ji = j;
+    if (j < P.n_jobs && tile >= P.jobs[j].tile_begin) ji = j;
   const PFJob& J = P.jobs[ji];
-  const int tid = threadIdx.x;
-  const int R = max(1, 256 / nb8);
-  const int row0 = ((int)blockIdx.x - J.tile_begin) * R;
-  const int b5 = tid / R, r5 = tid - (tid / R) * R;
-  const bool active = b5 < nb8 && row0 + r5 < J.rows;
-  const int bc = min(b5, nb8 - 1);
-  const Q50Item w5 = load_q50(J.w, nb8, min(row0 + r5, J.rows - 1), bc);
-  const int t0 = blockIdx.y * PF_FT;
-  const int nt = min(PF_FT, P.m - t0);
-  float qf[32];
+  const int nb8 = P.n_x / 32;
+  const int row = (tile - J.tile_begin) * PF_Q50_ROWS + lane;
+  const int t0 = (int)blockIdx.y * TOK;
+  const int per = KS ? P.per : nb8;        // blocks of a wave and round
+  const int round = KS ? P.ks * per : nb8;  // blocks of a round
+  const uint8_t* wrow = J.w.q + (size_t)min(row, J.rows - 1) * nb8 * 24;
+  const uint4* wq = reinterpret_cast<const uint4*>(wrow);
+  const uint2* wh = reinterpret_cast<const uint2*>(wrow + (size_t)nb8 * 16);
+  // x through the scalar cache; rows past the batch hold whatever an earlier
+  // one left (the buffers have PF_MAX rows), their results are dropped
+  typedef const __attribute__((address_space(4))) f32x8_t* sx_t;
+  const float* xt = P.x + (size_t)t0 * P.ldx;
+  // in chunks (token pair, half of a block): elements 8 hf .. +8 and
+  // 16 + 8 hf .. +8 of tokens 2 tp, 2 tp + 1
+  constexpr int NC = TOK;  // TOK / 2 pairs x 2 halves
+  f32x8_t cx[2][2][2];     // [set][token][lo | hi]
+  auto load_chunk = [&](auto cc, int b) {
+    constexpr int c = (int)cc;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int hi = 0; hi < 2; ++hi)
+        cx[c & 1][j][hi] = *(sx_t)(uintptr_t)(xt + 32 * b + (size_t)((c >> 1) * 2 + j) * P.ldx + 16 * hi + 8 * (c & 1));
+  };
+
+  float acc[TOK];
+#pragma unroll
+  for (int t = 0; t < TOK; ++t) acc[t] = 0.0f;
+  uint4 qn = make_uint4(0, 0, 0, 0);  // the next block's weights, in flight
+  uint2 hn = make_uint2(0, 0);
   {
-    const uint32_t qw[4] = {w5.qs.x, w5.qs.y, w5.qs.z, w5.qs.w};
-    const uint32_t qh = w5.hd.x;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const uint32_t byte = (qw[e >> 2] >> (8 * (e & 3))) & 0xffu;
-      qf[e] = (float)((int)((byte & 15u) | (((qh >> e) & 1u) << 4)) - 16);
-      qf[e + 16] = (float)((int)((byte >> 4) | (((qh >> (e + 16)) & 1u) << 4)) - 16);
-    }
+    const int b = KS ? min(wave * per, nb8 - 1) : 0;
+    qn = wq[b];
+    hn = wh[b];
+    load_chunk(std::integral_constant<int, 0>{}, b);
   }
-  const float dq = fp16_tensor(w5.hd.y & 0xffffu);
-  for (int hf = 0; hf < 2; ++hf) {
-    if (hf) __syncthreads();  // the first half's x is read
-    if (tid < nb8 * 8) {      // stage x of tokens t0 + hf*TH .. +TH (zeros past the batch)
-      const int b = tid >> 3, kk = (tid & 7) * 4;
-      float4 v[TH];
+  for (int r0 = 0; r0 < nb8; r0 += round) {
+    const int bb0 = KS ? min(r0 + wave * per, nb8) : 0, bb1 = min(bb0 + per, nb8);
+    for (int b = bb0; b < bb1; ++b) {
+      const int bn = min(b + 1 < bb1 ? b + 1 : b + 1 + round - per, nb8 - 1);  // this wave's next block
+      float qf[32];
+      {
+        const uint32_t w[4] = {qn.x, qn.y, qn.z, qn.w};
 #pragma unroll
-      for (int tt = 0; tt < TH; ++tt) {
-        const int t = hf * TH + tt;
-        v[tt] = (t < nt) ? reinterpret_cast<const float4*>(P.x + (size_t)(t0 + t) * P.ldx)[tid]
-                         : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      }
+        for (int k = 0; k < 8; ++k) {
+          // four bits of qh, one into bit 4 of each byte (the products of the
+          // multiplier's bits 0, 7, 14, 21 do not meet in bits 0, 8, 16, 24);
+          // then q - 16 as bytes
+          const uint32_t h = ((((hn.x >> (4 * k)) & 15u) * 0x00204081u) & 0x01010101u) << 4;
+          const uint32_t q5 = ((k < 4 ? w[k & 3] : w[k & 3] >> 4) & 0x0f0f0f0fu) | h;
+          const uint32_t qb = (q5 + 0x70707070u) ^ 0x80808080u;
 #pragma unroll
-      for (int tt = 0; tt < TH; ++tt) *reinterpret_cast<float4*>(xs + (tt * nb8 + b) * GF_XPAD + kk) = v[tt];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < TH; g += 4) {
-      float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int e4 = 0; e4 < 4; ++e4) {  // elements 4e4..+3 and 16+4e4..+3 of the block
-        float4 lo[4], hi[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float4* xb = reinterpret_cast<const float4*>(xs + ((g + j) * nb8 + bc) * GF_XPAD);
-          lo[j] = xb[e4];
-          hi[j] = xb[4 + e4];
+          for (int c = 0; c < 4; ++c) qf[4 * k + c] = (float)(int8_t)(qb >> (8 * c));
         }
+      }
+      const float dq = fp16_tensor(hn.y & 0xffffu);
+      qn = wq[bn];
+      hn = wh[bn];
+      float sum[2];
+      static_for<NC>([&](auto cc) {
+        constexpr int c = (int)cc, tp = c >> 1, hf = c & 1;
+        // this chunk has come before the next one's loads go out (scalar loads
+        // return out of order: a wait after them would wait for them too)
+        asm volatile("" ::"s"(cx[hf][0][0]), "s"(cx[hf][0][1]), "s"(cx[hf][1][0]), "s"(cx[hf][1][1]));
+        issue_fence();
+        if constexpr (c + 1 < NC)
+          load_chunk(std::integral_constant<int, c + 1>{}, b);
+        else
+          load_chunk(std::integral_constant<int, 0>{}, bn);
+        // step s: elements 8 hf + s and 16 + 8 hf + s; its products ahead of
+        // the adds of the one before, so that no add waits for its product
+        float pr[2][2][2];
+        auto products = [&](auto sc) {
+          constexpr int st = (int)sc;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int e = 4 * e4 + c;
+          for (int hi = 0; hi < 2; ++hi)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float xl = c == 0 ? lo[j].x : c == 1 ? lo[j].y : c == 2 ? lo[j].z : lo[j].w;
-            const float xh = c == 0 ? hi[j].x : c == 1 ? hi[j].y : c == 2 ? hi[j].z : hi[j].w;
-            sum[j] = sum[j] + qf[e] * xl;
-            sum[j] = sum[j] + qf[e + 16] * xh;
+            for (int j = 0; j < 2; ++j) pr[st & 1][hi][j] = cx[hf][j][hi][st] * qf[16 * hi + 8 * hf + st];
+        };
+        products(std::integral_constant<int, 0>{});
+        static_for<8>([&](auto sc) {
+          constexpr int st = (int)sc;
+          issue_fence();
+          if constexpr (st + 1 < 8) products(std::integral_constant<int, st + 1>{});
+          issue_fence();
+#pragma unroll
+          for (int hi = 0; hi < 2; ++hi)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              sum[j] = (hf == 0 && st == 0 && hi == 0) ? 0.0f + pr[0][0][j] : sum[j] + pr[st & 1][hi][j];
+        });
+        if constexpr (hf == 1) {
+          if (!KS || wave == 0) {  // uniform
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[2 * tp + j] = acc[2 * tp + j] + dq * sum[j];
+          } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) tl[((b - r0 - per) * TOK + 2 * tp + j) * 64 + lane] = dq * sum[j];
           }
         }
-      }
-      if (active) {
+      });
+    }
+    if constexpr (KS) {
+      __syncthreads();
+      if (wave == 0)
+        for (int b = min(r0 + per, nb8); b < min(r0 + round, nb8); ++b)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) tm[(hf * TH + g + j) * 256 + r5 * nb8 + b5] = dq * sum[j];
-      }
-      __builtin_amdgcn_sched_barrier(0);  // one group's x in registers at a time
+          for (int t = 0; t < TOK; ++t) acc[t] = acc[t] + tl[((b - r0 - per) * TOK + t) * 64 + lane];
+      __syncthreads();
     }
   }
-  __syncthreads();
-  if (tid < nt * R) {
-    const int tt = tid / R, r = tid - (tid / R) * R;
-    if (row0 + r < J.rows) {
-      const float* tr = tm + tt * 256 + r * nb8;
-      float acc = 0.0f;
+  if (KS && wave != 0) return;
+  if (row < J.rows) {
+    const float bias = (MODE == MODE_BIAS && J.bias) ? J.bias[row] : 0.0f;
 #pragma unroll
-      for (int h = 0; h < PF_Q50_MAXB; h += 16) {  // sixteen terms per LDS round trip
-        float tv[16];
-#pragma unroll
-        for (int b = 0; b < 16; ++b) tv[b] = tr[min(h + b, nb8 - 1)];
-#pragma unroll
-        for (int b = 0; b < 16; ++b)
-          if (h + b < nb8) acc = acc + tv[b];
-      }
-      float* y = J.y + (size_t)(t0 + tt) * J.ldy + row0 + r;
+    for (int t = 0; t < TOK; ++t) {
+      if (t0 + t >= P.m) break;  // uniform
+      float* y = J.y + (size_t)(t0 + t) * J.ldy + row;
       if (MODE == MODE_RESID)
-        *y = *y + acc;
+        *y = *y + acc[t];
       else
-        *y = J.bias ? acc + J.bias[row0 + r] : acc;
+        *y = J.bias ? acc[t] + bias : acc[t];
     }
   }
 }
-template __global__ void k_pf_gemm_q50<MODE_BIAS>(PFGemmFParams);
-template __global__ void k_pf_gemm_q50<MODE_RESID>(PFGemmFParams);
+template __global__ void k_pf_gemm_q50<MODE_BIAS, 16, false>(PFGemmFParams);
+template __global__ void k_pf_gemm_q50<MODE_RESID, 16, false>(PFGemmFParams);
+template __global__ void k_pf_gemm_q50<MODE_BIAS, 8, false>(PFGemmFParams);
+template __global__ void k_pf_gemm_q50<MODE_BIAS, 8, true>(PFGemmFParams);
+template __global__ void k_pf_gemm_q50<MODE_RESID, 8, false>(PFGemmFParams);
+template __global__ void k_pf_gemm_q50<MODE_RESID, 8, true>(PFGemmFParams);
 
 // q and k of token blockIdx.x made ready for k_pf_attn, v stored: per head
 // the Qwen3 QK-norm where the layer has the weights (engine/forward.go:80-91

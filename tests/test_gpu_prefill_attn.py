@@ -128,3 +128,18 @@ def test_non_finite_token_leaves_earlier_tokens(model):
         assert before and own == (s.t_v == G.Q8_0)
     finally:
         ctx.upload(0, "TOKEN_EMBD", G.Q8_0, s.n_vocab, s.n_embd, raw)
+
+
+# k_pf_gemm_q50: 16 tokens per wave; 8, with the blocks of a row whole, in
+# one round of two or four waves, and (4,864 columns) in five rounds
+@pytest.mark.parametrize("down", [G.Q6_K, G.Q5_0])
+@pytest.mark.parametrize("n", [5, 100, 150, 260])
+def test_q5_0_prompts(down, n, tmp_path):
+    s = G.ModelShape(n_layers=2, n_vocab=2048, t_q=G.Q5_0, t_k=G.Q5_0, t_v=G.Q8_0, t_o=G.Q5_0, t_gate=G.Q5_0,
+                     t_up=G.Q5_0, t_down=down)
+    G.write_synthetic_model(str(tmp_path / "m.gguf"), s, seed=92)
+    gf = G.GGUFFile(str(tmp_path / "m.gguf"))
+    with H.Ctx(H.desc_from_gguf(gf, max_ctx=512)) as ctx:
+        H.load_gguf_into(ctx, gf)
+        print("q5_0", down, n, flush=True)
+        compare(ctx, s, np.random.default_rng(n).integers(0, s.n_vocab, n).astype(np.int32), 0)
