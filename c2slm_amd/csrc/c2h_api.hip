@@ -1627,23 +1627,24 @@ int pf_alloc(c2h_ctx* c) {
   return C2H_OK;
 }
 
+typedef void (*PFGemmKernel)(PFGemmParams);
+PFGemmKernel pf_gemm_kernel(int mode, int tt) {  // Q4_K, 16 tt tokens per workgroup
+  if (tt == 1) return mode == MODE_RESID ? k_pf_gemm<T_Q4_K, MODE_RESID, 1> : k_pf_gemm<T_Q4_K, MODE_BIAS, 1>;
+  return mode == MODE_RESID ? k_pf_gemm<T_Q4_K, MODE_RESID, 2> : k_pf_gemm<T_Q4_K, MODE_BIAS, 2>;
+}
 // Waves per Q6_K tile: two, each half of the super-blocks, while the
 // second wave's terms fit PF_Q6_LDS_MAX (rows of up to 65 super-blocks,
 // which covers n_ff up to the 16384 c2h_create accepts); one beyond.
 int pf_q6_split(int nb) { return pf_q6_lds_bytes(nb, 2) <= PF_Q6_LDS_MAX ? 2 : 1; }
-typedef void (*PFGemmKernel)(PFGemmParams);
-PFGemmKernel pf_gemm_kernel(int type, int mode, bool small_tile = false, int q6_split = 1) {
-  if (type == C2H_Q4_K) {
-    if (small_tile)
-      return mode == MODE_RESID ? k_pf_gemm<T_Q4_K, MODE_RESID, 1> : k_pf_gemm<T_Q4_K, MODE_BIAS, 1>;
-    return mode == MODE_RESID ? k_pf_gemm<T_Q4_K, MODE_RESID, 4> : k_pf_gemm<T_Q4_K, MODE_BIAS, 4>;
-  }
-  if (q6_split == 2) return mode == MODE_RESID ? k_pf_gemm_q6<MODE_RESID, 2> : k_pf_gemm_q6<MODE_BIAS, 2>;
+PFGemmKernel pf_gemm_q6_kernel(int mode, int ns) {
+  if (ns == 2) return mode == MODE_RESID ? k_pf_gemm_q6<MODE_RESID, 2> : k_pf_gemm_q6<MODE_BIAS, 2>;
   return mode == MODE_RESID ? k_pf_gemm_q6<MODE_RESID, 1> : k_pf_gemm_q6<MODE_BIAS, 1>;
 }
-// A Q4_K launch whose 64 x 64 tiles would leave CUs idle runs 64-row x
-// 16-token workgroups instead (four times as many).
-constexpr int PF_SMALL_TILE_WG = 512;
+// A Q4_K launch of fewer 64-row x 32-token workgroups than this runs
+// 64 x 16 ones: at 416 workgroups (2,048 rows, 400 tokens, eight blocks) 28 us
+// against 34 with the small ones, at 304 (9,728 rows, 37 tokens, three
+// blocks) 12.1 against 10.0, at 256 (1,024 rows, 512 tokens) 12.0 against 9.8.
+constexpr int PF_SMALL_TILE_WG = 384;
 constexpr int PF_Q50_MIN_WAVES = 2048;
 
 // Tokens per wave of a k_pf_gemm_q50 launch and the waves a tile's blocks
@@ -1702,12 +1703,11 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
     if (type == C2H_Q6_K) {
       const int per_xcd = (tiles * (m_pad / 32) + 7) / 8;
       const int ns = pf_q6_split(nb);
-      hipLaunchKernelGGL(pf_gemm_kernel(type, mode, false, ns), dim3(8 * per_xcd), dim3(64 * ns),
+      hipLaunchKernelGGL(pf_gemm_q6_kernel(mode, ns), dim3(8 * per_xcd), dim3(64 * ns),
                          (size_t)pf_q6_lds_bytes(nb, ns), c->stream, P);
     } else {
-      const bool small = tiles * (m_pad / PF_TILE) < PF_SMALL_TILE_WG;
-      hipLaunchKernelGGL(pf_gemm_kernel(type, mode, small), dim3(tiles, m_pad / (small ? 16 : PF_TILE)), dim3(256), 0,
-                         c->stream, P);
+      const int tt = tiles * ((m + 31) / 32) < PF_SMALL_TILE_WG ? 1 : 2;
+      hipLaunchKernelGGL(pf_gemm_kernel(mode, tt), dim3(tiles, (m + 16 * tt - 1) / (16 * tt)), dim3(256), 0, c->stream, P);
     }
   }
   // float-input jobs: Q5_0 in one k_pf_gemm_q50 launch, Q8_0 in one k_pf_gemm_f

@@ -306,7 +306,7 @@ constexpr int ATT_AV_LDS_FLOATS = 3 * (ATT_AV_CH * ATT_AV_DSL + ATT_MAX_QPKV * A
 
 // ---- batched prefill (a prompt of up to PF_MAX tokens per pass)
 
-constexpr int PF_TILE = 64;   // rows and tokens of one prefill GEMM workgroup
+constexpr int PF_TILE = 64;   // rows of one Q4_K prefill GEMM workgroup; the token rows are padded to it
 constexpr int PF_MAX = 512;   // tokens per prefill pass (buffers are sized for it)
 
 // Q8_K rows of a token batch in global memory: token t, block b at
@@ -497,7 +497,7 @@ template <int NB>
 __global__ void k_pf_norm_quant(PFNormParams P);
 template <int NB>
 __global__ void k_pf_quant(PFQuantParams P);
-template <int TYPE, int MODE, int TT>  // TT: 16-token sub-tiles per wave (64 or 16 tokens per workgroup)
+template <int TYPE, int MODE, int TT>  // TT: 16-token sub-tiles per wave (32 or 16 tokens per workgroup)
 __global__ void k_pf_gemm(PFGemmParams P);
 // Q6_K jobs of a prefill: the reference's integer super-block sum
 // isum = sum over sub-blocks of sc * sum(q8 * (q6 - 32)) is, element by

@@ -3813,6 +3813,7 @@ template __global__ void k_pf_attn<128, false>(AttnCoreParams);
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 // One Q4_K super-block of one weight row as the MFMA A operand needs it:
 // lane (r = lane%16, k-group lk = lane/16) holds qs[32p + 8lk .. +8) of
@@ -3826,41 +3827,46 @@ struct PFA {
 
 __device__ __forceinline__ long as_long(u32x2_t v) { return (long)((uint64_t)v.x | ((uint64_t)v.y << 32)); }
 
-// Row parameters a row's lanes publish for the lanes that fold its outputs:
-// Q4_K d, dmin, sc[8], m[8] (c2_tensor_dot_q4_k_q8_k_gen.go:38-61), the
-// 6-bit scales and mins already as floats (exact).
-constexpr int PF_RP = 20;
-__device__ __forceinline__ void pf_row_params_q4k(const PFA& A, float* rp) {
-  rp[0] = fp16_simd_nb(A.hdr.x & 0xffffu);
-  rp[1] = fp16_simd_nb(A.hdr.x >> 16);
-  const uint4 h = make_uint4(A.hdr.x, A.hdr.y, A.hdr.z, A.hdr.w);
-  auto s = [&](int i) { return (int)byte_of(h, 4 + i); };
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    rp[2 + j] = (float)(s(j) & 63);
-    rp[10 + j] = (float)(s(j + 4) & 63);
-    rp[2 + 4 + j] = (float)((s(j + 8) & 15) | ((s(j) >> 6) << 4));
-    rp[10 + 4 + j] = (float)((s(j + 8) >> 4) | ((s(j + 4) >> 6) << 4));
-  }
+// What lane (row lr, pair lk) of a row publishes for the lanes that fold its
+// outputs: the 6-bit scales and mins of sub-blocks 2 lk, 2 lk + 1 as floats
+// (exact; c2_tensor_dot_q4_k_q8_k_gen.go:38-61): sc0, sc1, m0, m1.
+__device__ __forceinline__ f32x4_t pf_pair_params_q4k(const PFA& A, int lk) {
+  // scale bytes 0..3, 4..7, 8..11; pairs 0, 1: sub-blocks 0..3, pairs 2, 3: 4..7
+  const uint32_t s0 = A.hdr.y, s1 = A.hdr.z, s2 = A.hdr.w;
+  const bool up = lk >= 2;
+  const int sh = 16 * (lk & 1);
+  const uint32_t sc = (up ? (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u) : s0 & 0x3f3f3f3fu) >> sh;
+  const uint32_t m = (up ? ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u) : s1 & 0x3f3f3f3fu) >> sh;
+  const f32x4_t r = {(float)(sc & 0xffu), (float)((sc >> 8) & 0xffu), (float)(m & 0xffu), (float)((m >> 8) & 0xffu)};
+  return r;
 }
 
 // tokens x rows GEMM of one Q4_K prefill projection: workgroup tile = 64
-// rows x 64 tokens; wave w owns rows [16w, 16w+16) against all 64 tokens
-// (four 16x16 MFMA tiles).  Per super-block the token tile's Q8_K block is
+// rows x 16 TT tokens; wave w owns rows [16w, 16w+16) against all the tokens
+// (TT 16x16 MFMA tiles).  Per super-block the token tile's Q8_K block is
 // staged in LDS and the next block's weights are loaded while this one
 // runs.  Per pair p two v_mfma_i32_16x16x32_i8 (low nibbles x
 // q8[64p..+32), high nibbles x q8[64p+32..+32)) give s_lo, s_hi; the lane
 // then adds the pair term of c2_tensor_dot_q4_k_q8_k_gen.go:85 for its 4
 // rows x 1 token.  (Q6_K projections run k_pf_gemm_q6.)
+// Bound by the VALU: 14 instructions per (row, token, pair) of the fold in
+// the reference's order and ~4.5 around them; the SIMDs issue one per 4.3
+// clk (91 % busy).  Four waves per SIMD and conflict-free strides of the
+// parameters get it there: with 64-token tiles, 167 registers and every
+// other LDS cycle a conflict it was one per 5.9 clk.  512 tokens, gate|up of
+// the 0.5B shape 42.4 -> 39 us; 400 tokens of the 1.7B shape: gate|up 113 ->
+// 89, q|k 51 -> 38, o 34.7 -> 28 us.
 template <int TYPE, int MODE, int TT>
-__global__ void __launch_bounds__(256) k_pf_gemm(PFGemmParams P) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_pf_gemm(PFGemmParams P) {
   static_assert(TYPE == T_Q4_K, "Q6_K prefill projections run k_pf_gemm_q6");
-  static_assert(TT == 1 || TT == 4, "16 or 64 tokens per workgroup");
+  static_assert(TT == 1 || TT == 2, "16 or 32 tokens per workgroup");
   constexpr int TOK = 16 * TT;  // tokens of the workgroup's tile
   __shared__ __align__(16) uint32_t sq[TOK][68];  // Q8_K quants of the token tile (4-dword pad per row)
   __shared__ float sd[TOK];
-  __shared__ __align__(8) float sbp[TOK][8];     // f32(bsum[2i] + bsum[2i+1]) per token, i = 0..7
-  __shared__ float rp[4][16][PF_RP];
+  // (strides that spread a wave's reads over the banks)
+  __shared__ __align__(8) float sbp[TOK][10];  // f32(bsum[2i] + bsum[2i+1]) per token, i = 0..7
+  __shared__ f32x4_t rp[4][4][16];             // per wave, pair and row: scales and mins
+  __shared__ __align__(8) float rd[4][16][2]; // d, dmin
 
   int ji = 0;
 #pragma unroll
@@ -3904,6 +3910,14 @@ __global__ void __launch_bounds__(256) k_pf_gemm(PFGemmParams P) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) acc[tt][v] = 0.0f;
 
+  // f32(s) of an integer |s| < 2^22 without a conversion (which runs at half
+  // the rate): the MFMA adds s to the bits of 1.5 * 2^23, the subtraction of
+  // 1.5 * 2^23 is exact.  In vector registers: with a scalar operand the
+  // subtractions would lose the rate again.
+  float magic = 12582912.0f;
+  asm("" : "+v"(magic));
+  const int mi = __float_as_int(magic);
+  const i32x4_t magic4 = {mi, mi, mi, mi};
   PFA cur;
   load_a(cur, 0);
   for (int b = 0; b < nb; ++b) {
@@ -3927,36 +3941,48 @@ __global__ void __launch_bounds__(256) k_pf_gemm(PFGemmParams P) {
       if ((w4 & 1) == 0) sbp[tq + 16 * i][w4 >> 1] = (float)(bsv[i] + other);
     }
     if (tid < TOK) sd[tid] = dv;
-    if (lk == 0) pf_row_params_q4k(cur, rp[wave][lr]);
+    rp[wave][lk][lr] = pf_pair_params_q4k(cur, lk);
+    if (lk == 0) {
+      rd[wave][lr][0] = fp16_simd_nb(cur.hdr.x & 0xffffu);
+      rd[wave][lr][1] = fp16_simd_nb(cur.hdr.x >> 16);
+    }
     __syncthreads();
 
-    {
+    float dW[TT][4], mW[TT][4];  // d q8d, dmin q8d of the lane's rows and tokens
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const u32x2_t qs = cur.a[p];
-        const long a_lo = as_long(qs & 0x0f0f0f0fu);
-        const long a_hi = as_long((qs >> 4) & 0x0f0f0f0fu);
+    for (int v = 0; v < 4; ++v) {
+      const float d = rd[wave][4 * lk + v][0], dm = rd[wave][4 * lk + v][1];
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        dW[tt][v] = d * sd[tt * 16 + lr];
+        mW[tt][v] = dm * sd[tt * 16 + lr];
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const u32x2_t qs = cur.a[p];
+      const long a_lo = as_long(qs & 0x0f0f0f0fu);
+      const long a_hi = as_long((qs >> 4) & 0x0f0f0f0fu);
+      i32x4_t slo[TT], shi[TT];
+      f32x2_t bs[TT];
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        const int t = tt * 16 + lr;
+        const long b_lo = as_long(*reinterpret_cast<const u32x2_t*>(&sq[t][16 * p + 2 * lk]));
+        const long b_hi = as_long(*reinterpret_cast<const u32x2_t*>(&sq[t][16 * p + 8 + 2 * lk]));
+        slo[tt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, b_lo, magic4, 0, 0, 0);
+        shi[tt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, b_hi, magic4, 0, 0, 0);
+        bs[tt] = *reinterpret_cast<const f32x2_t*>(&sbp[t][2 * p]);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const f32x4_t r = rp[wave][p][4 * lk + v];
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt) {
-          const int t = tt * 16 + lr;
-          const long b_lo = as_long(*reinterpret_cast<const u32x2_t*>(&sq[t][16 * p + 2 * lk]));
-          const long b_hi = as_long(*reinterpret_cast<const u32x2_t*>(&sq[t][16 * p + 8 + 2 * lk]));
-          const i32x4_t zero = {0, 0, 0, 0};
-          const i32x4_t slo = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, b_lo, zero, 0, 0, 0);
-          const i32x4_t shi = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, b_hi, zero, 0, 0, 0);
-          const float q8d = sd[t];
-          const float bA = sbp[t][2 * p], bB = sbp[t][2 * p + 1];
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float* r = rp[wave][4 * lk + v];
-            const float dW = r[0] * q8d;
-            const float mW = r[1] * q8d;
-            const float sc0 = r[2 + 2 * p], sc1 = r[3 + 2 * p];
-            const float m0 = r[10 + 2 * p], m1 = r[11 + 2 * p];
-            const float term = (((float)slo[v] * (dW * sc0)) - (bA * (mW * m0))) +
-                               (((float)shi[v] * (dW * sc1)) - (bB * (mW * m1)));
-            acc[tt][v] = acc[tt][v] + term;
-          }
+          const float lo = __int_as_float(slo[tt][v]) - magic, hi = __int_as_float(shi[tt][v]) - magic;
+          const float term = ((lo * (dW[tt][v] * r.x)) - (bs[tt].x * (mW[tt][v] * r.z))) +
+                             ((hi * (dW[tt][v] * r.y)) - (bs[tt].y * (mW[tt][v] * r.w)));
+          acc[tt][v] = acc[tt][v] + term;
         }
       }
     }
@@ -4186,8 +4212,8 @@ C2H_PF(24)
 C2H_PF(35)
 C2H_PF(43)
 #undef C2H_PF
-template __global__ void k_pf_gemm<T_Q4_K, MODE_BIAS, 4>(PFGemmParams);
-template __global__ void k_pf_gemm<T_Q4_K, MODE_RESID, 4>(PFGemmParams);
+template __global__ void k_pf_gemm<T_Q4_K, MODE_BIAS, 2>(PFGemmParams);
+template __global__ void k_pf_gemm<T_Q4_K, MODE_RESID, 2>(PFGemmParams);
 template __global__ void k_pf_gemm<T_Q4_K, MODE_BIAS, 1>(PFGemmParams);
 template __global__ void k_pf_gemm<T_Q4_K, MODE_RESID, 1>(PFGemmParams);
 
