@@ -1769,15 +1769,23 @@ PFNormKernel pf_norm_kernel(int nb) {
 }
 PFQuantKernel pf_quant_kernel(int nb) {
   switch (nb) {
-    case 3: return k_pf_quant<3>;
-    case 4: return k_pf_quant<4>;
-    case 6: return k_pf_quant<6>;
-    case 8: return k_pf_quant<8>;
-    case 12: return k_pf_quant<12>;
-    case 19: return k_pf_quant<19>;
-    case 24: return k_pf_quant<24>;
-    case 35: return k_pf_quant<35>;
-    default: return k_pf_quant<43>;
+    case 3: return k_pf_quant<3, false>;
+    case 4: return k_pf_quant<4, false>;
+    case 6: return k_pf_quant<6, false>;
+    default: return k_pf_quant<8, false>;
+  }
+}
+PFQuantKernel pf_swiglu_quant_kernel(int nb) {
+  switch (nb) {
+    case 3: return k_pf_quant<3, true>;
+    case 4: return k_pf_quant<4, true>;
+    case 6: return k_pf_quant<6, true>;
+    case 8: return k_pf_quant<8, true>;
+    case 12: return k_pf_quant<12, true>;
+    case 19: return k_pf_quant<19, true>;
+    case 24: return k_pf_quant<24, true>;
+    case 35: return k_pf_quant<35, true>;
+    default: return k_pf_quant<43, true>;
   }
 }
 
@@ -1873,8 +1881,8 @@ int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
       hipLaunchKernelGGL(k, dim3(D.n_heads * ((m + A.tok_blk - 1) / A.tok_blk)), dim3(64 * PFA_NW),
                          pfa_lds_bytes(A.tok_blk, pmax, stage), c->stream, A);
     }
-    {
-      PFQuantParams Q{p.attn, E, m, q8};
+    if (!float_input(L.wo.type)) {  // (a float-input o-projection reads the f32 rows)
+      PFQuantParams Q{p.attn, nullptr, E, m, q8};
       hipLaunchKernelGGL(pf_quant_kernel(nb_k(E)), dim3(m_pad), dim3(256), 0, c->stream, Q);
     }
     pf_gemm(c, m, m_pad, nb_k(E), MODE_RESID, {&L.wo}, {p.X}, {nullptr}, {E}, p.attn, E, E);
@@ -1892,10 +1900,11 @@ int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
       hipLaunchKernelGGL(pf_norm_kernel(nb_k(E)), dim3(m_pad), dim3(pf_norm_threads(nb_k(E))), norm_lds, c->stream, N);
     }
     pf_gemm(c, m, m_pad, nb_k(E), MODE_BIAS, {&L.wg, &L.wu}, {p.g, p.u}, {nullptr, nullptr}, {F, F}, p.xn, E, E);
-    hipLaunchKernelGGL(k_pf_swiglu, dim3((F + 255) / 256, m), dim3(256), 0, c->stream, p.g, p.u, p.h, F, m);
-    {
-      PFQuantParams Q{p.h, F, m, q8};
-      hipLaunchKernelGGL(pf_quant_kernel(nb_k(F)), dim3(m_pad), dim3(256), 0, c->stream, Q);
+    if (float_input(L.wd.type)) {
+      hipLaunchKernelGGL(k_pf_swiglu, dim3((F + 255) / 256, m), dim3(256), 0, c->stream, p.g, p.u, p.h, F, m);
+    } else {
+      PFQuantParams Q{p.g, p.u, F, m, q8};
+      hipLaunchKernelGGL(pf_swiglu_quant_kernel(nb_k(F)), dim3(m_pad), dim3(256), 0, c->stream, Q);
     }
     pf_gemm(c, m, m_pad, nb_k(F), MODE_RESID, {&L.wd}, {p.X}, {nullptr}, {E}, p.h, F, F);
   }

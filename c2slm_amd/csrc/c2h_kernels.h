@@ -339,9 +339,10 @@ struct PFNormParams {
   float* xn;  // optional: the normalised rows [m_pad][n_x] as f32
 };
 
-// Per token: Q8_K of x[t][0 .. nb*256).
+// Per token: Q8_K of x[t][0 .. nb*256), or of SwiGLU(x, up).
 struct PFQuantParams {
   const float* x;
+  const float* up;
   int ld;
   int m;
   PFQ8 out;
@@ -495,7 +496,7 @@ __global__ void k_pf_attn(AttnCoreParams P);  // 64 PFA_NW threads
 __host__ __device__ constexpr int pf_norm_threads(int nb) { return nb <= 4 ? 256 : 512; }
 template <int NB>
 __global__ void k_pf_norm_quant(PFNormParams P);
-template <int NB>
+template <int NB, bool GLU>
 __global__ void k_pf_quant(PFQuantParams P);
 template <int TYPE, int MODE, int TT>  // TT: 16-token sub-tiles per wave (32 or 16 tokens per workgroup)
 __global__ void k_pf_gemm(PFGemmParams P);

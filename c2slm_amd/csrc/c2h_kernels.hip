@@ -3116,8 +3116,8 @@ __global__ void __launch_bounds__(ATT_AV_THREADS) k_attn_av(AttnCoreParams P) {
 //                     sums feed the reference's per-row float fold in order
 //   k_pf_qk           QK-norm, RoPE(q, k), K/V stored at their positions
 //   k_pf_attn         causal attention per (head, block of tokens)
-//   k_pf_quant        Q8_K of the attention / SwiGLU rows
-//   k_pf_swiglu       h = SwiGLU(gate, up)
+//   k_pf_quant        Q8_K of the attention rows / of SwiGLU(gate, up)
+//   k_pf_swiglu       h = SwiGLU(gate, up), where ffn_down reads f32 rows
 
 // One token's Q8_K row (LDS form) into the batch buffer.
 template <int NB, int NT = 256>
@@ -3161,7 +3161,11 @@ __global__ void __launch_bounds__(pf_norm_threads(NB)) k_pf_norm_quant(PFNormPar
   store_q8_row<NB, pf_norm_threads(NB)>(s, P.out, t);
 }
 
-template <int NB>
+// Q8_K of a token's row; GLU: of SwiGLU(x, up) (c2_tensor_swiglu_gen.go; whole
+// super-blocks end before the row's n % 8 last elements, which alone take
+// the scalar path), formed here: as a kernel of its own the SwiGLU wrote and
+// this one read 10 MB at 512 tokens (7.6 + 6.0 us, 9.3 together).
+template <int NB, bool GLU>
 __global__ void __launch_bounds__(256) k_pf_quant(PFQuantParams P) {
   constexpr int BPW = (NB + 3) / 4;
   __shared__ Q8KRow<NB> s;
@@ -3172,6 +3176,16 @@ __global__ void __launch_bounds__(256) k_pf_quant(PFQuantParams P) {
 #pragma unroll
   for (int i = 0; i < BPW; ++i)
     xa[i] = reinterpret_cast<const float4*>(P.x + (size_t)tc * P.ld + min(wave + 4 * i, NB - 1) * QK_K)[lane];
+  if constexpr (GLU) {
+    float4 ua[BPW];
+#pragma unroll
+    for (int i = 0; i < BPW; ++i)
+      ua[i] = reinterpret_cast<const float4*>(P.up + (size_t)tc * P.ld + min(wave + 4 * i, NB - 1) * QK_K)[lane];
+#pragma unroll
+    for (int i = 0; i < BPW; ++i)
+      xa[i] = make_float4(swiglu_poly(xa[i].x, ua[i].x), swiglu_poly(xa[i].y, ua[i].y), swiglu_poly(xa[i].z, ua[i].z),
+                          swiglu_poly(xa[i].w, ua[i].w));
+  }
   quantize_row_waves<NB>(xa, s);
   store_q8_row<NB>(s, P.out, t);
 }
@@ -4201,16 +4215,20 @@ C2H_PF(4)
 C2H_PF(6)
 C2H_PF(8)
 #undef C2H_PF
-#define C2H_PF(NB_) template __global__ void k_pf_quant<NB_>(PFQuantParams);
-C2H_PF(3)
-C2H_PF(4)
-C2H_PF(6)
-C2H_PF(8)
-C2H_PF(12)
-C2H_PF(19)
-C2H_PF(24)
-C2H_PF(35)
-C2H_PF(43)
+#define C2H_PF(NB_, GLU_) template __global__ void k_pf_quant<NB_, GLU_>(PFQuantParams);
+C2H_PF(3, false)
+C2H_PF(4, false)
+C2H_PF(6, false)
+C2H_PF(8, false)
+C2H_PF(3, true)
+C2H_PF(4, true)
+C2H_PF(6, true)
+C2H_PF(8, true)
+C2H_PF(12, true)
+C2H_PF(19, true)
+C2H_PF(24, true)
+C2H_PF(35, true)
+C2H_PF(43, true)
 #undef C2H_PF
 template __global__ void k_pf_gemm<T_Q4_K, MODE_BIAS, 2>(PFGemmParams);
 template __global__ void k_pf_gemm<T_Q4_K, MODE_RESID, 2>(PFGemmParams);
