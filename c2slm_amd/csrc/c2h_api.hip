@@ -94,6 +94,7 @@ struct c2h_ctx {
   float* att_sc = nullptr;  // [n_heads][sc_ld] scores / probabilities
   float* att_bmax = nullptr;
   int att_sc_ld = 0, att_n_blk = 0;
+  int sav_hpw = 1;  // query heads per k_attn_h128_sav workgroup
   int32_t seq_len = 0;   // KVCache.SeqLen (engine/kvcache.go:25-47)
 
   // batched prefill buffers (allocated by the first c2h_prefill)
@@ -610,14 +611,21 @@ AttnCoreParams attn_params(c2h_ctx* c, int layer) {
 // Long-context attention of a decode step: scores over every block of the
 // context, softmax, AV.  Blocks past the token's context return at once, so
 // the grid covers max_ctx and graphs replay at any pos.
-void enqueue_attn_long(c2h_ctx* c, const AttnCoreParams& A) {
+void enqueue_attn_long(c2h_ctx* c, AttnCoreParams A) {
   const c2h_model_desc& D = c->desc;
+  if (D.head_dim == 128) {
+    A.hpw = c->sav_hpw;
+    A.sav_ld = pfa_sc_ld(D.max_ctx - 1);
+    hipLaunchKernelGGL(k_attn_h128_scores, dim3(c->att_n_blk, D.n_kv_heads), dim3(256), 0, c->stream, A);
+    hipLaunchKernelGGL(k_attn_h128_sav, dim3(128 / 16, (D.n_heads / D.n_kv_heads + A.hpw - 1) / A.hpw, D.n_kv_heads),
+                       dim3(ATT_SAV_THREADS), (size_t)A.hpw * A.sav_ld * 4, c->stream, A);
+    return;
+  }
   hipLaunchKernelGGL(k_attn_scores, dim3(c->att_n_blk, D.n_kv_heads), dim3(256), 0, c->stream, A);
   hipLaunchKernelGGL(k_attn_softmax, dim3(D.n_heads), dim3(1024),
                      (size_t)attn_softmax_lds_floats(D.max_ctx) * 4, c->stream, A);
   hipLaunchKernelGGL(k_attn_av, dim3(D.n_kv_heads * ATT_AV_SLICES), dim3(ATT_AV_THREADS),
-                     (size_t)ATT_AV_LDS_FLOATS * 4, c->stream,
-                     A);
+                     (size_t)ATT_AV_LDS_FLOATS * 4, c->stream, A);
 }
 
 // Attention forms of a decode step by the positions T it attends to:
@@ -630,8 +638,8 @@ constexpr int kFormTier[ATT_FORM_CORE] = {ATT_TIER_32, ATT_TIER_64, ATT_TIER_96,
 static_assert(sizeof(c2h_ctx::g_step) / sizeof(hipGraphExec_t) == ATT_FORMS, "one graph per attention form");
 
 int attn_form(const c2h_ctx* c, int T) {
-  if (c->desc.head_dim == 128) return ATT_FORM_32;  // k_attn_h128 serves every T
   if (c->long_attn && T > c->att_split) return ATT_FORM_LONG;
+  if (c->desc.head_dim == 128) return ATT_FORM_32;  // k_attn_h128 serves every T up to the split
   for (int f = 0; f < ATT_FORM_CORE; ++f)
     if (T <= kFormTier[f]) return f;
   return ATT_FORM_CORE;
@@ -639,7 +647,7 @@ int attn_form(const c2h_ctx* c, int T) {
 
 // Whether some decode position of this context runs the form.
 bool form_used(const c2h_ctx* c, int form) {
-  if (c->desc.head_dim == 128) return form == ATT_FORM_32;
+  if (c->desc.head_dim == 128) return form == ATT_FORM_32 || (form == ATT_FORM_LONG && c->long_attn);
   const int tmax = c->long_attn ? c->att_split : c->desc.max_ctx;  // largest T of the core forms
   if (form == ATT_FORM_LONG) return c->long_attn;
   return form == 0 || tmax > kFormTier[form - 1];
@@ -736,14 +744,13 @@ void enqueue_attn(c2h_ctx* c, int l, int form) {
   A.out = c->attn;
   A.store_kv = 1;
   const dim3 grid(D.n_heads / D.n_kv_heads, D.n_kv_heads);
-  if (D.head_dim == 128) {
-    A.sc_ld = attn_h128_lds_floats(D.max_ctx);  // the V chunks follow the scores
+  if (form == ATT_FORM_LONG) {
+    enqueue_attn_long(c, A);
+  } else if (D.head_dim == 128) {
+    A.sc_ld = attn_h128_lds_floats(c->att_split);  // the V chunks follow the scores
     hipLaunchKernelGGL(c->h128_staged ? k_attn_h128<H128_VCH> : k_attn_h128<0>, grid, dim3(256), c->attn_lds,
                        c->stream, A);
-  }
-  else if (form == ATT_FORM_LONG)
-    enqueue_attn_long(c, A);
-  else {
+  } else {
     A.xcd_map = D.n_kv_heads <= ATT_XCDS ? 1 : 0;
     const dim3 xgrid(ATT_XCDS * (D.n_heads / D.n_kv_heads));
     hipLaunchKernelGGL(attn_core_kernel(form), A.xcd_map ? xgrid : grid, dim3(256), c->attn_lds, c->stream, A.state,
@@ -1433,17 +1440,26 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
                         (const void*)k_pf_attn<128, true>, (const void*)k_pf_attn<128, false>})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PFA_LDS_MAX) != hipSuccess)
       return bail(fail(c, C2H_ERR_HIP, "prefill attention LDS attribute"));
-  if (D.head_dim == 128) {  // k_attn_h128 at every T: the scores of max_ctx positions in LDS
-    c->attn_lds = (size_t)attn_h128_lds_floats(D.max_ctx) * 4;
-    if (c->attn_lds > 152u * 1024)
+  const int qpkv = D.n_heads / D.n_kv_heads;
+  if (D.head_dim == 128) {
+    if ((size_t)attn_h128_lds_floats(D.max_ctx) * 4 > 152u * 1024)
       return bail(fail(c, C2H_ERR_UNSUPPORTED, "head_dim 128 runs up to %d positions", 152 * 256 - 64));
+    // k_attn_h128 up to the split length (every T with more query heads per
+    // KV head than the long-context kernels take), its scores in LDS
+    c->att_split = D.max_ctx;
+    if (qpkv <= ATT_MAX_QPKV) {
+      int split = ATT_SPLIT_T_H128;
+      if (const char* sp = getenv("C2H_ATT_SPLIT")) split = std::max(1, atoi(sp));
+      c->att_split = std::min(split, D.max_ctx);
+    }
+    c->long_attn = D.max_ctx > c->att_split;
+    c->attn_lds = (size_t)attn_h128_lds_floats(c->att_split) * 4;
     // V staged through LDS where its two chunks fit beside the scores
     c->h128_staged = c->attn_lds + (size_t)attn_h128_v_lds_floats() * 4 <= 152u * 1024;
     if (c->h128_staged) c->attn_lds += (size_t)attn_h128_v_lds_floats() * 4;
     if (hipFuncSetAttribute(c->h128_staged ? (const void*)k_attn_h128<H128_VCH> : (const void*)k_attn_h128<0>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->attn_lds) != hipSuccess)
       return bail(fail(c, C2H_ERR_HIP, "attention LDS attribute"));
-    c->att_split = D.max_ctx;
   } else {
     c->att_split = ATT_SPLIT_T;
     if (const char* sp = getenv("C2H_ATT_SPLIT")) c->att_split = std::max(1, atoi(sp));
@@ -1467,19 +1483,27 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
       if (D.max_ctx > ATT_LONG_MAX_CTX)
         return bail(fail(c, C2H_ERR_UNSUPPORTED, "max_ctx %d above the %d positions of the exact attention kernels",
                          D.max_ctx, ATT_LONG_MAX_CTX));
-      if (D.n_heads / D.n_kv_heads > ATT_MAX_QPKV)
+      if (qpkv > ATT_MAX_QPKV)
         return bail(fail(c, C2H_ERR_UNSUPPORTED, "more than %d query heads per KV head", ATT_MAX_QPKV));
-      c->att_sc_ld = (D.max_ctx + 3) & ~3;
-      c->att_n_blk = (D.max_ctx + ATT_SB - 1) / ATT_SB;
-      if ((rc = dalloc(c, &c->att_sc, (size_t)D.n_heads * c->att_sc_ld * 4)) ||
-          (rc = dalloc(c, &c->att_bmax, (size_t)D.n_heads * c->att_n_blk * 4)))
-        return bail(rc);
-      if (hipFuncSetAttribute((const void*)k_attn_softmax, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              attn_softmax_lds_floats(D.max_ctx) * 4) != hipSuccess ||
-          hipFuncSetAttribute((const void*)k_attn_av, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              ATT_AV_LDS_FLOATS * 4) != hipSuccess)
-        return bail(fail(c, C2H_ERR_HIP, "long attention LDS attribute"));
     }
+  }
+  if (c->long_attn) {
+    const int sb = D.head_dim == 128 ? H128_SB : ATT_SB;
+    c->att_sc_ld = (D.max_ctx + 3) & ~3;
+    c->att_n_blk = (D.max_ctx + sb - 1) / sb;
+    if ((rc = dalloc(c, &c->att_sc, (size_t)D.n_heads * c->att_sc_ld * 4)) ||
+        (rc = dalloc(c, &c->att_bmax, (size_t)D.n_heads * c->att_n_blk * 4)))
+      return bail(rc);
+    const size_t row = (size_t)pfa_sc_ld(D.max_ctx - 1) * 4;
+    c->sav_hpw = std::max(1, std::min(qpkv, (int)(PFA_LDS_MAX / row)));
+    if (D.head_dim == 128
+            ? hipFuncSetAttribute((const void*)k_attn_h128_sav, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(c->sav_hpw * row)) != hipSuccess
+            : hipFuncSetAttribute((const void*)k_attn_softmax, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  attn_softmax_lds_floats(D.max_ctx) * 4) != hipSuccess ||
+                  hipFuncSetAttribute((const void*)k_attn_av, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      ATT_AV_LDS_FLOATS * 4) != hipSuccess)
+      return bail(fail(c, C2H_ERR_HIP, "long attention LDS attribute"));
   }
   C2hState s0;
   memset(&s0, 0, sizeof(s0));
@@ -1640,6 +1664,10 @@ PFGemmKernel pf_gemm_q6_kernel(int mode, int ns) {
   if (ns == 2) return mode == MODE_RESID ? k_pf_gemm_q6<MODE_RESID, 2> : k_pf_gemm_q6<MODE_BIAS, 2>;
   return mode == MODE_RESID ? k_pf_gemm_q6<MODE_RESID, 1> : k_pf_gemm_q6<MODE_BIAS, 1>;
 }
+// Prompts of a head_dim-128 model up to this long run the decode forward per
+// token: one costs 40..55 us a layer at a few hundred positions, a batched
+// pass ~110 however few its tokens (1 token, a few layers: 184 against 457 us).
+constexpr int PF_H128_FORWARDS = 2;
 // A Q4_K launch of fewer 64-row x 32-token workgroups than this runs
 // 64 x 16 ones: at 416 workgroups (2,048 rows, 400 tokens, eight blocks) 28 us
 // against 34 with the small ones, at 304 (9,728 rows, 37 tokens, three
@@ -1934,15 +1962,35 @@ int c2h_prefill(c2h_ctx* c, const int32_t* tokens, int32_t n, int32_t pos0, floa
   if (pos0 < 0 || (int64_t)pos0 + n > c->desc.max_ctx)
     return fail(c, C2H_ERR_RANGE, "positions [%d, %d) outside [0, %d)", pos0, pos0 + n, c->desc.max_ctx);
   if (n == 0) return C2H_OK;
-  if ((rc = pf_alloc(c)) || (rc = pf_q6_ready(c))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  c->ring_next = 0;
-  for (int done = 0; done < n;) {
-    const int m = std::min(n - done, PF_MAX);
-    if ((rc = pf_pass(c, tokens + done, m, pos0 + done))) return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));  // tokens are copied from the caller's buffer
-    done += m;
-    c->seq_len = pos0 + done;
+  if (c->desc.head_dim == 128 && n <= PF_H128_FORWARDS) {
+    // a forward graph per token, as engine.IngestFrom runs Forward per token
+    // (c2slm.go:103-114)
+    if ((rc = build_graphs(c))) return rc;
+    for (int i = 0; i < n; ++i) {
+      C2hState s;
+      memset(&s, 0, sizeof(s));
+      s.pos = pos0 + i;
+      s.token = tokens[i];
+      s.penalty = 1.15f;
+      s.nx_in = c->nx_cur;
+      s.nx_out = c->nx_cur ^ 1;
+      if ((rc = push_state(c, s)) || (rc = run_graph(c, false, pos0 + i))) return rc;
+      c->nx_prev = c->nx_cur;
+      c->nx_cur ^= 1;
+      c->seq_len = pos0 + i + 1;
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  } else {
+    if ((rc = pf_alloc(c)) || (rc = pf_q6_ready(c))) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->ring_next = 0;
+    for (int done = 0; done < n;) {
+      const int m = std::min(n - done, PF_MAX);
+      if ((rc = pf_pass(c, tokens + done, m, pos0 + done))) return rc;
+      HIPCHK(c, hipStreamSynchronize(c->stream));  // tokens are copied from the caller's buffer
+      done += m;
+      c->seq_len = pos0 + done;
+    }
   }
   if (normx_out)
     HIPCHK(c, stream_copy(c->stream, normx_out, c->normx[c->nx_cur], (size_t)c->desc.n_embd * 4,

@@ -191,6 +191,9 @@ __host__ __device__ inline size_t vq_index(int p, int d, int hd = 64) {
 //     workgroup per head, exps in LDS) -> k_attn_av (one workgroup per KV
 //     head and 16-dim slice: two waves run the FMA chains of all the group's
 //     query heads, the others stage the V slice through LDS).
+// At head_dim 128 the forms are k_attn_h128, and k_attn_h128_scores ->
+// k_attn_h128_sav (workgroups over 16 output dims of a group's query heads:
+// softmax, FMA chains).
 constexpr int ATT_CH = 128;   // V positions staged in LDS per pass (chunk 0 prefetched)
 constexpr int ATT_KPF = 256;  // K rows per LDS chunk of the scores (one per thread)
 constexpr int ATT_KPAD = 68;  // floats per staged K row (64 + 4: conflict-free row reads)
@@ -210,6 +213,9 @@ __host__ __device__ inline int attn_tier(int T) {
          : T <= 256 ? ATT_TIER_256 : ATT_TIER_ANY;
 }
 constexpr int ATT_SPLIT_T = 1024;  // default split length (positions attended)
+constexpr int ATT_SPLIT_T_H128 = 512;
+constexpr int H128_SB = 64;           // positions per k_attn_h128_scores workgroup (16 per wave)
+constexpr int ATT_SAV_THREADS = 512;  // k_attn_h128_sav: the softmax on eight waves, the chain on one
 constexpr int ATT_SB = 256;        // positions per k_attn_scores workgroup
 constexpr int ATT_AV_CH = 256;     // positions per k_attn_av LDS chunk
 constexpr int ATT_AV_THREADS = 256;  // k_attn_av: one chain wave, three staging waves
@@ -246,20 +252,21 @@ struct AttnCoreParams {
   float scale;
   C2hState* state;
   int tok0;  // first query token of this launch within the q/k/v/out rows
-  // long form: scores / probabilities sc[(i*n_heads + h)*sc_ld + p] of
-  // launch token i, block maxima bmax[(i*n_heads + h)*n_blk + b]
+  // long forms: scores / probabilities sc[h*sc_ld + p], block maxima
+  // bmax[h*n_blk + b]
   float* sc;
   float* bmax;
   int sc_ld;    // (k_pf_attn: the row stride of its LDS scores, pfa_sc_ld)
   int n_blk;
-  int n_tok;    // k_pf_attn: query tokens of the prefill pass, and of a workgroup
-  int tok_blk;
+  int n_tok;    // k_pf_attn: query tokens of the prefill pass
   // k_attn_core: 1 = the grid is (ATT_XCDS * qpkv, 1, tokens), n_kv_heads
   // <= ATT_XCDS, and workgroup L serves KV head L % ATT_XCDS, query head
   // L / ATT_XCDS, so the workgroups of one KV head share an XCD and its L2
   // (workgroups go to the XCDs round robin); the workgroups left over exit
   // at once.  0 = the grid is (qpkv, n_kv_heads, tokens).
   int xcd_map;
+  int tok_blk;      // k_pf_attn: query tokens of a workgroup
+  int hpw, sav_ld;  // k_attn_h128_sav: query heads per workgroup, its LDS row stride (pfa_sc_ld)
 };
 constexpr int ATT_XCDS = 8;
 
@@ -488,6 +495,8 @@ inline int attn_dims(const AttnCoreParams& A, int qpkv) {
 __global__ void k_attn_scores(AttnCoreParams P);
 __global__ void k_attn_softmax(AttnCoreParams P);
 __global__ void k_attn_av(AttnCoreParams P);
+__global__ void k_attn_h128_scores(AttnCoreParams P);
+__global__ void k_attn_h128_sav(AttnCoreParams P);
 template <int VCH>
 __global__ void k_attn_h128(AttnCoreParams P);
 template <int HD, bool STAGE>

@@ -3474,6 +3474,307 @@ __device__ __forceinline__ float row_max_dpp(float x) {
   return fmax_gt(x, dpp_or0<0x121>(x));
 }
 
+// ----------------------------- attention, head_dim 128, longer contexts
+//
+// The arithmetic of k_attn_h128 for one token, in two launches on the FP32
+// matrix instruction (its chains are the reference's, see k_pf_attn), the
+// query heads of a KV head as the rows of the tiles; k_attn_h128's one
+// workgroup per query head leaves the GPU to 12 or 16 of them:
+//   k_attn_h128_scores  per block of H128_SB positions: QK-norm, RoPE, K/V
+//                  store, scores of the KV head's query heads (each K row
+//                  read once), block maxima per head;
+//   k_attn_h128_sav     per 16 output dims and group of query heads: max, f64
+//                  exp, the sequential f32 sum (exact speculative form),
+//                  p = e * (1/sum), the FMA chain over p = 0..pos in order.
+// The chain is what bounds k_attn_h128_sav (50 clk per four positions); its
+// workgroups repeat the softmax of their heads, which costs less than a
+// launch and a trip of the probabilities through memory.  1,500 positions,
+// 12 heads: 6.1 + 16.2 us against k_attn_h128's 34.1; the same at ~512, where
+// the split lies (a decode step of four layers at 384, 512, 768 positions:
+// 182, 193, 212 us with one launch, 188, 193, 199 with two).  At head_dim 64
+// k_attn_softmax and k_attn_av stay: their chain runs on VALU fmas at 8.0 clk
+// per position, and at 4,096 positions the pair took 31 us against 40.
+
+__global__ void __launch_bounds__(256) k_attn_h128_scores(AttnCoreParams P) {
+  constexpr int HD = 128, NG = HD / 64, H2 = HD / 2;
+  __shared__ __align__(16) float qs[ATT_MAX_QPKV + 1][HD + 4];  // the group's query heads, then k
+  __shared__ float inv[ATT_MAX_QPKV + 1];
+  __shared__ float bm[4][16];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = blockIdx.y;
+  const int qpkv = P.n_heads / P.n_kv_heads;
+  const int pos = P.state->pos;
+  const int T = pos + 1;
+  const int p0 = blockIdx.x * H128_SB;
+  if (p0 >= T) return;  // uniform: blocks past the context do nothing
+  const size_t head_stride = (size_t)kv_slot(P.max_ctx) * HD;
+  float* kcache = P.kv + ((size_t)P.layer * P.n_kv_heads + g) * head_stride;
+  float* vcache = P.kv + (((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride;
+  const int p = p0 + 16 * wave + col;
+
+  // ---- loads: the heads' rows (pairs i, i + HD/2), k's and v's, the wave's 16 K rows
+  const int nh = qpkv + 1;
+  constexpr int PT = ((ATT_MAX_QPKV + 1) * H2 + 255) / 256;  // pairs per thread
+  float x0[PT], x1[PT];
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {
+    const int i = min(tid + 256 * k, nh * H2 - 1), h = i / H2, d = i & (H2 - 1);
+    const float* src = h < qpkv ? P.q + (g * qpkv + h) * HD : P.k + g * HD;
+    x0[k] = src[d];
+    x1[k] = src[d + H2];
+  }
+  const float vn = P.v[g * HD + (tid & (HD - 1))];
+  const int rp = min(max(pos, 0), P.rope_len - 1);
+  const float rcos = P.rope_cos[(size_t)rp * H2 + (tid & (H2 - 1))];  // (256 k + tid: the same pair index)
+  const float rsin = P.rope_sin[(size_t)rp * H2 + (tid & (H2 - 1))];
+  f32x4_t kr[NG][4];
+  {
+    const float* row = kcache + (size_t)min(p, max(pos - 1, 0)) * HD + 16 * kg;  // rows before pos are stored
+#pragma unroll
+    for (int G = 0; G < NG; ++G)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kr[G][i] = reinterpret_cast<const f32x4_t*>(row + 64 * G)[i];
+  }
+  issue_fence();
+  if (P.q_norm || P.k_norm) {  // uniform; sequential sums of squares, a head per lane
+#pragma unroll
+    for (int k = 0; k < PT; ++k) {
+      const int i = tid + 256 * k;
+      if (i < nh * H2) {
+        qs[i / H2][i & (H2 - 1)] = x0[k] * x0[k];
+        qs[i / H2][(i & (H2 - 1)) + H2] = x1[k] * x1[k];
+      }
+    }
+    __syncthreads();
+    if (tid < nh) {
+      float sum = 0.0f;
+#pragma unroll 16
+      for (int d = 0; d < HD; ++d) sum = sum + qs[tid][d];
+      inv[tid] = rms_scale(sum / (float)HD + P.eps);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PT; ++k) {
+      const int i = min(tid + 256 * k, nh * H2 - 1), h = i / H2, d = i & (H2 - 1);
+      const float* nw = h < qpkv ? P.q_norm : P.k_norm;
+      if (nw) {
+        x0[k] = (x0[k] * inv[h]) * nw[d];
+        x1[k] = (x1[k] * inv[h]) * nw[d + H2];
+      }
+    }
+  }
+  const bool rope = pos >= 0 && pos < P.rope_len;
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {
+    const int i = tid + 256 * k;
+    if (i < nh * H2) {
+      const float y0 = rope ? (x0[k] * rcos) - (x1[k] * rsin) : x0[k];
+      const float y1 = rope ? (x0[k] * rsin) + (x1[k] * rcos) : x1[k];
+      qs[i / H2][i & (H2 - 1)] = y0;
+      qs[i / H2][(i & (H2 - 1)) + H2] = y1;
+    }
+  }
+  __syncthreads();
+  if (tid < HD && pos >= p0 && pos < p0 + H128_SB && pos < P.max_ctx) {
+    kcache[(size_t)pos * HD + tid] = qs[qpkv][tid];
+    vcache[vq_index(pos, tid, HD)] = vn;
+  }
+  // ---- operands: lane (col, kg), A row col = query head (past the group's
+  // its last), B column col = position p; k of pos from this launch
+  f32x4_t q[NG][4];
+#pragma unroll
+  for (int G = 0; G < NG; ++G)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      q[G][i] = *reinterpret_cast<const f32x4_t*>(&qs[min(col, qpkv - 1)][64 * G + 16 * kg + 4 * i]);
+      const f32x4_t kp = *reinterpret_cast<const f32x4_t*>(&qs[qpkv][64 * G + 16 * kg + 4 * i]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) kr[G][i][c] = (p == pos) ? kp[c] : kr[G][i][c];
+    }
+  f32x4_t u[4];
+  static_for<4>([&](auto pr) {
+    f32x4_t d[4];  // accumulators 2 pr, 2 pr + 8, 2 pr + 1, 2 pr + 9
+    static_for<NG>([&](auto G) {
+      static_for<4>([&](auto x) {
+        constexpr int c = 2 * (int)pr + ((int)x >> 1) + 8 * ((int)x & 1);
+        const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        d[(int)x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[(int)G][c / 4][c % 4], kr[(int)G][c / 4][c % 4],
+                                                         (int)G == 0 ? zero : d[(int)x], 0, 0, 0);
+      });
+    });
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[(int)pr][i] = (d[0][i] + d[1][i]) + (d[2][i] + d[3][i]);
+  });
+  float* srow = P.sc + (size_t)g * qpkv * P.sc_ld;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 4 * kg + i;
+    const float s = ((u[0][i] + u[1][i]) + (u[2][i] + u[3][i])) * P.scale;
+    if (r < qpkv && p < T) srow[(size_t)r * P.sc_ld + p] = s;
+    const float m = row_max_dpp((p < T && s > -__builtin_inff()) ? s : -__builtin_inff());  // NaN never wins
+    if (col == 0) bm[wave][r] = m;
+  }
+  __syncthreads();
+  if (tid < qpkv) {
+    const float m = fmax_gt(fmax_gt(fmax_gt(bm[0][tid], bm[1][tid]), bm[2][tid]), bm[3][tid]);
+    P.bmax[((size_t)g * qpkv + tid) * P.n_blk + blockIdx.x] = m;
+  }
+}
+
+// Exps to probabilities in MFMA operand order, in place: rows of ld floats,
+// each times its 1/sum, the 16 positions of a group transposed as a 4 x 4
+// block (position 4 c + k at slot 4 k + c), so that lane row k reads the
+// operands of four consecutive instructions as 16 bytes.  Position p is then
+// at prob_slot(p).  A thread per row and group; the caller's barriers around.
+__device__ __forceinline__ int prob_slot(int p) { return (p & ~15) + 4 * (p & 3) + ((p >> 2) & 3); }
+__device__ __forceinline__ void probs_in_order(float* e, int rows, int ld, int groups, const float* inv, int nthr) {
+  for (int i = threadIdx.x; i < rows * groups; i += nthr) {
+    const int r = i / groups;
+    f32x4_t* g = reinterpret_cast<f32x4_t*>(e + r * ld + 16 * (i - r * groups));
+    const float iv = inv[r];
+    f32x4_t x[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) x[c] = g[c];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const f32x4_t y = {x[0][k] * iv, x[1][k] * iv, x[2][k] * iv, x[3][k] * iv};
+      g[k] = y;
+    }
+  }
+}
+
+// Grid (HD / 16 slices of dims, head groups, KV heads), P.hpw query heads
+// per workgroup; dynamic LDS [P.hpw][P.sav_ld] exps.
+__global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParams P) {
+  constexpr int HD = 128;
+  constexpr int NT = ATT_SAV_THREADS;
+  extern __shared__ __align__(16) unsigned char smem[];
+  float* e = reinterpret_cast<float*>(smem);
+  __shared__ double exp_tab[EXP_TAB];
+  __shared__ float mx_s[8], inv_s[8];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = blockIdx.z;
+  const int qpkv = P.n_heads / P.n_kv_heads;
+  const int h0 = blockIdx.y * P.hpw, nh = min(P.hpw, qpkv - h0);
+  const int ld = P.sav_ld;
+  const int T = P.state->pos + 1;
+  const size_t head_stride = (size_t)kv_slot(P.max_ctx) * HD;
+  const float* vcache = P.kv + (((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride;
+  const float* srow = P.sc + ((size_t)g * qpkv + h0) * P.sc_ld;
+  load_exp_tab(exp_tab);
+
+  // V as B operands, a dword each (lane (col, kg): position 4 quad + kg of
+  // its dim): the first batches land under the softmax (wave 0 runs the chain)
+  constexpr int VB = 16, NV = 4;  // quads per batch, batches in flight
+  const int nq = (T + 3) >> 2, nfull = T >> 2, nbat = nfull / VB;
+  const int dim = 16 * (int)blockIdx.x + col;
+  const unsigned vl = (unsigned)dim * 4 + kg;
+  float v[NV][VB], vr[VB];  // vr: the quads past the whole batches
+  f32x4_t vt = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (wave == 0) {
+#pragma unroll
+    for (int s = 0; s < NV; ++s)
+#pragma unroll
+      for (int k = 0; k < VB; ++k) v[s][k] = (vcache + (size_t)min(s * VB + k, nq - 1) * (4 * HD))[vl];
+#pragma unroll
+    for (int k = 0; k < VB; ++k) vr[k] = (vcache + (size_t)min(nbat * VB + k, nq - 1) * (4 * HD))[vl];
+    vt = reinterpret_cast<const f32x4_t*>(vcache)[(size_t)(nq - 1) * HD + dim];
+  }
+  // ---- max: wave w head w, over its block maxima (never NaN); NaN when score 0 is
+  if (wave < nh) {
+    const int nb = (T + H128_SB - 1) / H128_SB;
+    const float* bmx = P.bmax + ((size_t)g * qpkv + h0 + wave) * P.n_blk;
+    float lm = -__builtin_inff();
+    for (int b = lane; b < nb; b += 64) lm = fmax_gt(lm, bmx[b]);
+    lm = wave_max_dpp(lm);
+    const float s0 = srow[(size_t)wave * P.sc_ld];
+    if (lane == 0) mx_s[wave] = s0 != s0 ? s0 : lm;
+  }
+  __syncthreads();
+  // ---- exps (eight loads of four positions in flight)
+  for (int r = 0; r < nh; ++r) {
+    const float m = mx_s[r];
+    const f32x4_t* s4 = reinterpret_cast<const f32x4_t*>(srow + (size_t)r * P.sc_ld);
+    f32x4_t* e4 = reinterpret_cast<f32x4_t*>(e + r * ld);
+    for (int i0 = tid; i0 < nq; i0 += 8 * NT) {
+      f32x4_t s[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s[k] = s4[min(i0 + k * NT, nq - 1)];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (i0 + k * NT >= nq) break;
+        f32x4_t x;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[c] = exp_f32(s[k][c] - m, exp_tab);  // (past pos: never used)
+        e4[i0 + k * NT] = x;
+      }
+    }
+  }
+  __syncthreads();
+  // the sequential sums, wave w head w
+  if (wave < nh) {
+    const float* a = e + wave * ld;
+    const float s = (T <= 64 * SPEC_C)    ? seq_sum_wave(a, T)
+                    : (T <= 128 * SPEC_C) ? seq_sum_wave<2 * SPEC_C>(a, T)
+                                          : seq_sum_wave_n(a, T);
+    if (lane == 0) inv_s[wave] = 1.0f / s;
+  }
+  __syncthreads();
+  probs_in_order(e, nh, ld, (nq + 3) >> 2, inv_s, NT);
+  __syncthreads();
+  if (wave != 0) return;  // no barrier follows
+
+  // ---- AV: A row col = head, four positions per instruction.  An FP32 MFMA
+  // holds up its own wave's VALU for its 32 clk, so the chain's loop has
+  // none: the probabilities come four instructions' at a time from LDS, V as
+  // operands, NV batches ahead (with a multiply, lane swaps and copies per
+  // instruction it ran at 75 clk instead of 50).
+  const f32x4_t* arow = reinterpret_cast<const f32x4_t*>(e + min(col, nh - 1) * ld + 4 * kg);
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_t a[2][VB / 4];
+#pragma unroll
+  for (int j = 0; j < VB / 4; ++j) a[0][j] = arow[4 * j];
+  // batch bi, in set S of V and S % 2 of the probabilities
+  auto step = [&](auto S, int bi) {
+    constexpr int st = (int)S;
+    const f32x4_t* an = arow + VB * min(bi + 1, max(nbat - 1, 0));
+    const float* vn = vcache + (size_t)min(bi + NV, nbat - 1) * (VB * 4 * HD);
+    static_for<VB>([&](auto kc) {
+      constexpr int k = (int)kc;
+      issue_fence();
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st & 1][k / 4][k % 4], v[st][k], acc, 0, 0, 0);
+      if constexpr (k % 4 == 0) a[(st & 1) ^ 1][k / 4] = an[k];
+      v[st][k] = (vn + k * (4 * HD))[vl];
+    });
+    issue_fence();
+  };
+  int bi = 0;
+  for (; bi + NV <= nbat; bi += NV) static_for<NV>([&](auto i) { step(i, bi + (int)i); });
+  static_for<NV - 1>([&](auto i) {
+    if (bi < nbat) {  // uniform
+      step(i, bi);
+      ++bi;
+    }
+  });
+#pragma unroll
+  for (int k = 0; k < VB; ++k)
+    if (nbat * VB + k < nfull)  // uniform
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float*>(arow + VB * nbat + 4 * (k / 4))[k % 4],
+                                                 vr[k], acc, 0, 0, 0);
+  // the last one to three positions
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = min(4 * kg + i, nh - 1);
+    float x = acc[i];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      if (4 * nfull + c < T) x = __builtin_fmaf(e[r * ld + prob_slot(4 * nfull + c)], vt[c], x);
+    if (4 * kg + i < nh) P.out[((size_t)g * qpkv + h0 + r) * HD + dim] = x;
+  }
+}
+
 // Causal attention of a prefill pass: workgroup (query head h, block of
 // P.tok_blk <= 16 query tokens), token i at position pos0 + i attending
 // positions 0..pos0+i, all of whose K/V rows are in the cache (k_pf_qk), q

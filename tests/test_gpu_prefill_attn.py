@@ -65,7 +65,7 @@ def compare(ctx, s, toks, pos0):
     n = pos0 + len(toks)
     nx = ctx.prefill(toks, pos0)
     kv = all_kv(ctx, s, n)
-    for p, t in enumerate(toks):
+    for p, t in enumerate(toks):  # (two-launch attention past 512 positions at head_dim 128)
         want = ctx.forward(int(t), pos0 + p)
     for got, ref in zip(kv, all_kv(ctx, s, n)):
         ok = same(got, ref)
@@ -76,7 +76,8 @@ def compare(ctx, s, toks, pos0):
 # blocks of 16 tokens, tiles of 16 positions, quads of 4, batches of 64
 # (AV and sums); 2,340 positions is past 16 tokens' scores in LDS, 4,700
 # past eight's
-@pytest.mark.parametrize("pos0,n", [(0, 1), (0, 2), (0, 16), (0, 17), (3, 33), (63, 1), (62, 37), (127, 20), (300, 75),
+@pytest.mark.parametrize("pos0,n", [(0, 1), (0, 2), (0, 3), (0, 16), (0, 17), (3, 33), (63, 1), (62, 37), (127, 20), (300, 75),
+                                    (505, 12),
                                     (1000, 30), (2340, 18), (4700, 9)])
 def test_prefill_equals_forwards(model, pos0, n):
     s, _, ctx = model
