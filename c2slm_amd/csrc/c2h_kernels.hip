@@ -3405,8 +3405,9 @@ template __global__ void k_pf_gemm_q50<MODE_RESID, 8, true>(PFGemmFParams);
 // squares run one head per lane), RoPE (tensor/ops.go:262-286, pairs
 // (i, i + HD/2), the attention kernels' expressions), then q back in place
 // and K/V into the cache at pos0 + t (engine/kvcache.go:143-157).  One
-// workgroup per token, a pair per thread and trip: 1 query + KV head per
-// wave was 4.7 us at 512 tokens for K/V alone, this with q 3.9 us.
+// workgroup per token, a pair per thread and trip: 5.0 us at 512 tokens of 14
+// + 2 heads of 64 (a wave per KV head took 4.7 us for K and V alone, and the
+// attention turned q once per block).
 template <int HD>
 __global__ void __launch_bounds__(256) k_pf_qk(PFRopeParams P) {
   constexpr int H2 = HD / 2;
@@ -3805,7 +3806,10 @@ __global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParam
 // through the wave's own 16 rows of LDS (STAGE; without it, where a long
 // context's scores leave no room, in the operands' order), V quads turn into
 // operands with lane-row swaps.  Scores of the block's tokens sit in LDS: 16
-// tokens up to ~1,900 positions, fewer beyond (pf_attn_tokens).
+// tokens up to ~1,900 positions, fewer beyond (pf_attn_tokens).  512 tokens,
+// 14 heads of 64: 20.2 us (31.9 with the same FMAs on the VALU); 400 tokens, 16
+// heads of 128: 25 us; 512 tokens ending at 3,000 positions: 160 us (1,340 in
+// three launches per 16 tokens).
 // Block order: a block's work grows with its last position, so the grid is
 // one-dimensional and runs the blocks from the last (longest) to the first;
 // the dispatcher hands each freed slot the next block.
