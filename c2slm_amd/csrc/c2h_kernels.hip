@@ -3808,8 +3808,8 @@ __global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParam
 // operands with lane-row swaps.  Scores of the block's tokens sit in LDS: 16
 // tokens up to ~1,900 positions, fewer beyond (pf_attn_tokens).  512 tokens,
 // 14 heads of 64: 20.2 us (31.9 with the same FMAs on the VALU); 400 tokens, 16
-// heads of 128: 25 us; 512 tokens ending at 3,000 positions: 160 us (1,340 in
-// three launches per 16 tokens).
+// heads of 128: 25 us; the six passes of a 3,000-token prompt 121 us on
+// average (beyond 1,024 positions three launches per 16 tokens took 42 us).
 // Block order: a block's work grows with its last position, so the grid is
 // one-dimensional and runs the blocks from the last (longest) to the first;
 // the dispatcher hands each freed slot the next block.
