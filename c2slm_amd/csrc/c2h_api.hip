@@ -22,6 +22,7 @@ using namespace c2h;
 namespace {
 
 constexpr int kStateRing = 256;
+constexpr int PF_ATT_SUB = 16;  // prompt tokens per launch of the long-context attention kernels
 
 struct Tensor {
   uint8_t* q = nullptr;
@@ -91,7 +92,7 @@ struct c2h_ctx {
   size_t attn_lds = 0;
   int att_split = 0;     // positions attended up to which k_attn_core runs
   bool long_attn = false;
-  float* att_sc = nullptr;  // [n_heads][sc_ld] scores / probabilities
+  float* att_sc = nullptr;  // [tokens of a launch][n_heads][sc_ld] scores / probabilities
   float* att_bmax = nullptr;
   int att_sc_ld = 0, att_n_blk = 0;
   int sav_hpw = 1;  // query heads per k_attn_h128_sav workgroup
@@ -608,10 +609,11 @@ AttnCoreParams attn_params(c2h_ctx* c, int layer) {
   return A;
 }
 
-// Long-context attention of a decode step: scores over every block of the
-// context, softmax, AV.  Blocks past the token's context return at once, so
-// the grid covers max_ctx and graphs replay at any pos.
-void enqueue_attn_long(c2h_ctx* c, AttnCoreParams A) {
+// Long-context attention of a decode step, or at head_dim 64 of `ntok` query
+// tokens of a prompt (rows tok0..): scores over every block of the context,
+// softmax, AV.  Blocks past a token's context return at once, so the grid
+// covers max_ctx and graphs replay at any pos.
+void enqueue_attn_long(c2h_ctx* c, AttnCoreParams A, int ntok) {
   const c2h_model_desc& D = c->desc;
   if (D.head_dim == 128) {
     A.hpw = c->sav_hpw;
@@ -621,10 +623,10 @@ void enqueue_attn_long(c2h_ctx* c, AttnCoreParams A) {
                        dim3(ATT_SAV_THREADS), (size_t)A.hpw * A.sav_ld * 4, c->stream, A);
     return;
   }
-  hipLaunchKernelGGL(k_attn_scores, dim3(c->att_n_blk, D.n_kv_heads), dim3(256), 0, c->stream, A);
-  hipLaunchKernelGGL(k_attn_softmax, dim3(D.n_heads), dim3(1024),
+  hipLaunchKernelGGL(k_attn_scores, dim3(c->att_n_blk, D.n_kv_heads, ntok), dim3(256), 0, c->stream, A);
+  hipLaunchKernelGGL(k_attn_softmax, dim3(D.n_heads, ntok), dim3(1024),
                      (size_t)attn_softmax_lds_floats(D.max_ctx) * 4, c->stream, A);
-  hipLaunchKernelGGL(k_attn_av, dim3(D.n_kv_heads * ATT_AV_SLICES), dim3(ATT_AV_THREADS),
+  hipLaunchKernelGGL(k_attn_av, dim3(D.n_kv_heads * ATT_AV_SLICES, ntok), dim3(ATT_AV_THREADS),
                      (size_t)ATT_AV_LDS_FLOATS * 4, c->stream, A);
 }
 
@@ -745,7 +747,7 @@ void enqueue_attn(c2h_ctx* c, int l, int form) {
   A.store_kv = 1;
   const dim3 grid(D.n_heads / D.n_kv_heads, D.n_kv_heads);
   if (form == ATT_FORM_LONG) {
-    enqueue_attn_long(c, A);
+    enqueue_attn_long(c, A, 1);
   } else if (D.head_dim == 128) {
     A.sc_ld = attn_h128_lds_floats(c->att_split);  // the V chunks follow the scores
     hipLaunchKernelGGL(c->h128_staged ? k_attn_h128<H128_VCH> : k_attn_h128<0>, grid, dim3(256), c->attn_lds,
@@ -1491,8 +1493,9 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
     const int sb = D.head_dim == 128 ? H128_SB : ATT_SB;
     c->att_sc_ld = (D.max_ctx + 3) & ~3;
     c->att_n_blk = (D.max_ctx + sb - 1) / sb;
-    if ((rc = dalloc(c, &c->att_sc, (size_t)D.n_heads * c->att_sc_ld * 4)) ||
-        (rc = dalloc(c, &c->att_bmax, (size_t)D.n_heads * c->att_n_blk * 4)))
+    const size_t rows = (size_t)D.n_heads * (D.head_dim == 64 ? PF_ATT_SUB : 1);
+    if ((rc = dalloc(c, &c->att_sc, rows * c->att_sc_ld * 4)) ||
+        (rc = dalloc(c, &c->att_bmax, rows * c->att_n_blk * 4)))
       return bail(rc);
     const size_t row = (size_t)pfa_sc_ld(D.max_ctx - 1) * 4;
     c->sav_hpw = std::max(1, std::min(qpkv, (int)(PFA_LDS_MAX / row)));
@@ -1828,6 +1831,27 @@ int pf_attn_tokens(int n_heads, int m, int pmax) {
   return tb;
 }
 
+// Whether the attention of m prompt tokens up to position pmax runs as the
+// three long-context launches per PF_ATT_SUB tokens (head_dim 64) instead of
+// k_pf_attn, whose workgroups each run all of a head's positions in order:
+// by the time of either, in ns for T = pmax + 1 positions, fitted to passes of
+// 14 / 2, 16 / 8 and 24 / 4 (KV) heads at 1,100..36,000 positions, 1..512
+// tokens.  k_pf_attn: 18 per position and round of one workgroup per CU (what
+// fits past ~2,900 positions; below, it wins from 17 tokens on either way).
+// The three launches: 18,000 + 4.8 per position, and 220 + 0.07 per position
+// for each token and KV head.  They run where that saves 5 %: 14 / 2 heads,
+// a layer of 1 token at 8,192 positions 152 against 240 us, of 16 at 4,096
+// 147 / 177, of 512 at 15,700 (one token per k_pf_attn workgroup) 4.90 / 8.45
+// ms; not for 32 tokens at 4,096 (204 / 181), or 512 at 8,192 (3.03 / 2.39 ms).
+bool pf_attn_split(int n_heads, int n_kv_heads, int m, int pmax, int tok_blk) {
+  const double T = pmax + 1;
+  const int rounds = (n_heads * ((m + tok_blk - 1) / tok_blk) + PFA_MIN_WG - 1) / PFA_MIN_WG;
+  const double whole = 8000.0 + rounds * 18.2 * T;
+  const int launches = (m + PF_ATT_SUB - 1) / PF_ATT_SUB;
+  const double split = launches * (18000.0 + 4.8 * T) + (double)m * n_kv_heads * (220.0 + 0.07 * T);
+  return split < 0.95 * whole;
+}
+
 // One pass of up to PF_MAX tokens at positions pos0.. (engine.Forward per
 // token, batched layer by layer).
 int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
@@ -1899,15 +1923,27 @@ int pf_pass(c2h_ctx* c, const int32_t* tokens, int m, int pos0) {
       A.out = p.attn;
       A.q_ld = E;
       A.out_ld = E;
-      A.n_tok = m;
       const int pmax = pos0 + m - 1;
       A.tok_blk = pf_attn_tokens(D.n_heads, m, pmax);
-      A.sc_ld = pfa_sc_ld(pmax);
-      const bool stage = pfa_lds_bytes(A.tok_blk, pmax, true) <= PFA_LDS_MAX;
-      const auto k = D.head_dim == 64 ? (stage ? k_pf_attn<64, true> : k_pf_attn<64, false>)
-                                      : (stage ? k_pf_attn<128, true> : k_pf_attn<128, false>);
-      hipLaunchKernelGGL(k, dim3(D.n_heads * ((m + A.tok_blk - 1) / A.tok_blk)), dim3(64 * PFA_NW),
-                         pfa_lds_bytes(A.tok_blk, pmax, stage), c->stream, A);
+      if (D.head_dim == 64 && c->long_attn && pmax >= c->att_split &&
+          pf_attn_split(D.n_heads, D.n_kv_heads, m, pmax, A.tok_blk)) {
+        A.k = p.k;
+        A.v = p.v;
+        A.kv_ld = KV;
+        A.store_kv = 0;
+        for (int t0 = 0; t0 < m; t0 += PF_ATT_SUB) {
+          A.tok0 = t0;
+          enqueue_attn_long(c, A, std::min(PF_ATT_SUB, m - t0));
+        }
+      } else {
+        A.n_tok = m;
+        A.sc_ld = pfa_sc_ld(pmax);
+        const bool stage = pfa_lds_bytes(A.tok_blk, pmax, true) <= PFA_LDS_MAX;
+        const auto k = D.head_dim == 64 ? (stage ? k_pf_attn<64, true> : k_pf_attn<64, false>)
+                                        : (stage ? k_pf_attn<128, true> : k_pf_attn<128, false>);
+        hipLaunchKernelGGL(k, dim3(D.n_heads * ((m + A.tok_blk - 1) / A.tok_blk)), dim3(64 * PFA_NW),
+                           pfa_lds_bytes(A.tok_blk, pmax, stage), c->stream, A);
+      }
     }
     if (!float_input(L.wo.type)) {  // (a float-input o-projection reads the f32 rows)
       PFQuantParams Q{p.attn, nullptr, E, m, q8};

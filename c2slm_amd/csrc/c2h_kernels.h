@@ -252,8 +252,8 @@ struct AttnCoreParams {
   float scale;
   C2hState* state;
   int tok0;  // first query token of this launch within the q/k/v/out rows
-  // long forms: scores / probabilities sc[h*sc_ld + p], block maxima
-  // bmax[h*n_blk + b]
+  // long forms: scores / probabilities sc[(i*n_heads + h)*sc_ld + p] of
+  // launch token i, block maxima bmax[(i*n_heads + h)*n_blk + b]
   float* sc;
   float* bmax;
   int sc_ld;    // (k_pf_attn: the row stride of its LDS scores, pfa_sc_ld)

@@ -2803,7 +2803,8 @@ template __global__ void k_attn_h128<H128_VCH>(AttnCoreParams);
 //                   probabilities through two LDS chunks.
 
 // In decode (store_kv) the workgroup whose block holds pos stores RoPE(k)
-// and v at pos; a batch has stored its K/V before the launch.
+// and v at pos; a batch has its K/V stored and its q rotated (k_pf_qk)
+// before the launch.
 __global__ void __launch_bounds__(256) k_attn_scores(AttnCoreParams P) {
   constexpr int HD = 64;
   __shared__ __align__(16) float qs[ATT_MAX_QPKV][HD];
@@ -2842,8 +2843,9 @@ __global__ void __launch_bounds__(256) k_attn_scores(AttnCoreParams P) {
   if (tid < nq4) reinterpret_cast<float4*>(&qs[0][0])[tid] = qv;
   if (tid < HD) ks[tid] = kn;
   __syncthreads();
-  // RoPE (tensor/ops.go:262-286) of the group's query heads and of k
-  if (pos >= 0 && pos < P.rope_len) {
+  // RoPE (tensor/ops.go:262-286) of the group's query heads and of k (a
+  // batch's q comes rotated)
+  if (P.store_kv && pos >= 0 && pos < P.rope_len) {
     for (int i = tid; i < (qpkv + 1) * 32; i += 256) {  // i & 31 == tid & 31
       float* x = (i < qpkv * 32) ? qs[i >> 5] : ks;
       const int j = i & 31;

@@ -140,6 +140,25 @@ def test_long_kernels_prefill(tiny_model_path):
     orc.close()
 
 
+@pytest.mark.parametrize("pos0,n", [(2500, 16), (7000, 17)])
+def test_long_kernels_late_prompt(tiny_model_path, pos0, n):
+    # few prompt tokens late in a session run the long-context kernels, in
+    # launches of 16 tokens: KV and normX equal to sequential ingest
+    gf, ctx, orc, im_end, eos = open_pair(tiny_model_path, max_ctx=8192)
+    fill_cache(ctx, orc, pos0, seed=n)
+    toks = np.random.default_rng(n).integers(0, 4096, n).astype(np.int32)
+    got = ctx.prefill(toks, pos0)
+    want = orc.ingest_from(pos0, toks)
+    assert np.array_equal(bits(got), bits(want))
+    kv = orc.kv()
+    for which in (0, 1):
+        for layer in (0, 1):
+            for h in (0, 1):
+                assert np.array_equal(bits(ctx.kv(which, layer, h, pos0 + n)), bits(kv[which, layer, h, :pos0 + n]))
+    ctx.close()
+    orc.close()
+
+
 def test_long_kernels_nan_score_zero(tiny_model_path):
     # a NaN in K row 0 makes score[0] NaN for every head of its group: the
     # max is NaN (tensor/ops.go:320-326) and so is every probability; the

@@ -1,0 +1,87 @@
+"""Prompts take, at each size, the kernels that suit it: the time of one
+against that of work the other route would not keep up with, with a wide
+margin on both sides, and bit for bit what one forward per token leaves."""
+import time
+
+import numpy as np
+import pytest
+
+from c2slm_amd import _lib as H
+from c2slm_amd import gguf as G
+
+pytestmark = pytest.mark.gpu
+
+
+def best_us(f, reps=7):
+    t = []
+    for _ in range(reps):
+        t0 = time.perf_counter()
+        f()
+        t.append(time.perf_counter() - t0)
+    return min(t) * 1e6
+
+
+def open_model(path, shape, max_ctx, seed=71):
+    G.write_synthetic_model(str(path), shape, seed=seed)
+    gf = G.GGUFFile(str(path))
+    ctx = H.Ctx(H.desc_from_gguf(gf, max_ctx=max_ctx))
+    H.load_gguf_into(ctx, gf)
+    return ctx
+
+
+def fill(ctx, s, n, seed=72):
+    kv = np.random.default_rng(seed).standard_normal((n, s.head_dim)).astype(np.float32)
+    for which in range(2):
+        for layer in range(s.n_layers):
+            for h in range(s.n_kv_heads):
+                ctx.set_kv(which, layer, h, 0, np.roll(kv, 17 * (which + 2 * layer + 5 * h), 0))
+
+
+def check_prompt(ctx, s, toks, pos0):
+    """normX, and K and V of every layer from pos0 on, as one forward per token leaves them."""
+    n = pos0 + len(toks)
+    got = ctx.prefill(toks, pos0)
+    kv = [ctx.kv(w, layer, h, n)[pos0:] for w in (0, 1) for layer in range(s.n_layers) for h in range(s.n_kv_heads)]
+    for i, t in enumerate(toks):
+        want = ctx.forward(int(t), pos0 + i)
+    ref = [ctx.kv(w, layer, h, n)[pos0:] for w in (0, 1) for layer in range(s.n_layers) for h in range(s.n_kv_heads)]
+    for a, b in zip([got, *kv], [want, *ref]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# Prompts late in a session: few tokens, and any number once a workgroup's
+# LDS holds one token's scores, run the decode's long-context kernels.
+
+LATE = 15700
+
+
+@pytest.fixture(scope="module")
+def late(tmp_path_factory):
+    s = G.ModelShape(n_layers=2, n_vocab=2048)
+    ctx = open_model(tmp_path_factory.mktemp("late") / "m.gguf", s, 16384)
+    fill(ctx, s, LATE)
+    yield s, ctx
+    ctx.close()
+
+
+# what the context adds to a prompt, in units of what it adds to a forward
+# (whose attention is the same three launches for one token): 0.9, 1.3 and 21
+# measured; with a workgroup per head and block of tokens 3.9, 4.3 and 59
+@pytest.mark.parametrize("n,most", [(1, 2.0), (16, 2.7), (256, 44.0)])
+def test_late_prompts_keep_up_with_decode(late, n, most):
+    s, ctx = late
+    toks = np.random.default_rng(n).integers(0, s.n_vocab, n).astype(np.int32)
+    more = best_us(lambda: ctx.prefill(toks, LATE)) - best_us(lambda: ctx.prefill(toks, 100))
+    one = best_us(lambda: ctx.forward(5, LATE)) - best_us(lambda: ctx.forward(5, 100))
+    print(n, more, one, more / one, flush=True)
+    assert more < most * one
+
+
+# one sub-launch whole and in part, several with a part; an ordinary prompt
+# beside them (37 tokens at 4,000 stay with k_pf_attn)
+@pytest.mark.parametrize("pos0,n", [(1024, 1), (3000, 16), (4000, 5), (4000, 37), (7000, 17), (LATE, 37), (LATE, 1)])
+def test_late_prompts_equal_forwards(late, pos0, n):
+    s, ctx = late
+    print(pos0, n, flush=True)
+    check_prompt(ctx, s, np.random.default_rng(pos0 + n).integers(0, s.n_vocab, n).astype(np.int32), pos0)
+    fill(ctx, s, LATE)
