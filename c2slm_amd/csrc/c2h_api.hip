@@ -1695,6 +1695,24 @@ void pf_q50_split(int row_tiles, int m, int n_x, int* tok, PFGemmFParams* F) {
   F->per = std::min((nb8 + F->ks - 1) / F->ks, PF_Q50_PER_MAX);
 }
 
+// The kernel of a Q5_0 launch of `rows` rows and m tokens: k_pf_gemm_q50 has
+// the higher rate, but its waves wait out a weight load per block and run
+// eight tokens however few there are.  Up to PF_Q50S_WG workgroups
+// k_pf_gemm_q50s takes rows of up to PF_Q50_MAXB blocks (28 blocks at 912
+// workgroups, q|k of 128 tokens: 15.6 us against 16.1; at 1,081, gate|up of 1
+// to 16 tokens, 15.2..18.0 against 15.6..17.2), and k_pf_gemm_f wider ones of
+// a few tokens (152 blocks, 4 and 8 tokens: 44 and 84 us against 71 and 78).
+constexpr int PF_Q50S_WG = 1000;
+constexpr int PF_Q50F_TOK = 7;
+enum Q50Kernel { Q50_TILES, Q50_SMALL, Q50_WIDE };
+Q50Kernel pf_q50_kernel(int64_t rows, int m, int nb8) {
+  if (nb8 <= PF_Q50_MAXB) {
+    const int R = pf_q50_rows(nb8);
+    return (rows + R - 1) / R * ((m + PF_FT - 1) / PF_FT) <= PF_Q50S_WG ? Q50_SMALL : Q50_TILES;
+  }
+  return m <= PF_Q50F_TOK && nb8 <= 256 ? Q50_WIDE : Q50_TILES;
+}
+
 // y[t][r] (=|+=) W * x[t] for the given matrices: Q4_K / Q6_K on the
 // Q8_K rows (one MFMA launch per type), Q5_0 / Q8_0 on the f32 rows xf
 // (a launch per type), as engine/model.go:250-270 dispatches.
@@ -1741,7 +1759,7 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
       hipLaunchKernelGGL(pf_gemm_kernel(mode, tt), dim3(tiles, (m + 16 * tt - 1) / (16 * tt)), dim3(256), 0, c->stream, P);
     }
   }
-  // float-input jobs: Q5_0 in one k_pf_gemm_q50 launch, Q8_0 in one k_pf_gemm_f
+  // float-input jobs: a launch for Q5_0, a launch for Q8_0
   for (int type : {(int)C2H_Q5_0, (int)C2H_Q8_0}) {
     PFGemmFParams F;
     memset(&F, 0, sizeof(F));
@@ -1749,7 +1767,11 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
     F.ldx = ldxf;
     F.n_x = n_x;
     F.m = m;
-    const int R = type == C2H_Q5_0 ? PF_Q50_ROWS : 32;
+    int64_t rows = 0;
+    for (const Tensor* w : W)
+      if (w->type == type) rows += w->rows;
+    const Q50Kernel q50 = pf_q50_kernel(rows, m, n_x / 32);
+    const int R = type != C2H_Q5_0 ? 32 : q50 == Q50_TILES ? PF_Q50_ROWS : pf_q50_rows(n_x / 32);
     int tiles = 0;
     for (size_t i = 0; i < W.size(); ++i) {
       if (W[i]->type != type) continue;
@@ -1765,7 +1787,11 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
       J.bias = B[i];
     }
     if (F.n_jobs == 0) continue;
-    if (type == C2H_Q5_0) {
+    if (type == C2H_Q5_0 && q50 == Q50_SMALL) {
+      auto k = mode == MODE_RESID ? k_pf_gemm_q50s<MODE_RESID> : k_pf_gemm_q50s<MODE_BIAS>;
+      hipLaunchKernelGGL(k, dim3(tiles, (m + PF_FT - 1) / PF_FT), dim3(256), (size_t)pf_gemm_q50s_lds_bytes(n_x),
+                         c->stream, F);
+    } else if (type == C2H_Q5_0 && q50 == Q50_TILES) {
       int tok;
       pf_q50_split(tiles, m, n_x, &tok, &F);
       F.n_tiles = tiles;
@@ -1780,8 +1806,10 @@ void pf_gemm(c2h_ctx* c, int m, int m_pad, int nb, int mode, std::initializer_li
       // alone would leave CUs idle (the 128 rows of attn_v)
       F.ft = PF_FT;
       while (F.ft > 1 && tiles * ((m + F.ft - 1) / F.ft) < 512) F.ft /= 2;
-      auto k = (mode == MODE_RESID) ? k_pf_gemm_f<MODE_RESID> : k_pf_gemm_f<MODE_BIAS>;
-      hipLaunchKernelGGL(k, dim3(tiles, (m + F.ft - 1) / F.ft), dim3(256), (size_t)pf_gemm_f_lds_bytes(n_x),
+      const bool wide = type == C2H_Q5_0;
+      auto k = mode == MODE_RESID ? k_pf_gemm_f<MODE_RESID, false> : k_pf_gemm_f<MODE_BIAS, false>;
+      if (wide) k = mode == MODE_RESID ? k_pf_gemm_f<MODE_RESID, true> : k_pf_gemm_f<MODE_BIAS, true>;
+      hipLaunchKernelGGL(k, dim3(tiles, (m + F.ft - 1) / F.ft), dim3(256), (size_t)pf_gemm_f_lds_bytes(n_x, wide),
                          c->stream, F);
     }
   }

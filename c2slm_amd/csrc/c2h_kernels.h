@@ -377,9 +377,12 @@ struct PFGemmParams {
   PFJob jobs[3];
 };
 
-// Q5_0 (k_pf_gemm_q50) or Q8_0 (k_pf_gemm_f) jobs of a batch on f32 rows
-// x[t*ldx .. + n_x); tile_begin counts row tiles of PF_Q50_ROWS or 32 rows.
-constexpr int PF_FT = 16;        // tokens per k_pf_gemm_f workgroup, at most
+// Q5_0 (k_pf_gemm_q50, _q50s, k_pf_gemm_f<.., true>) or Q8_0 (k_pf_gemm_f)
+// jobs of a batch on f32 rows x[t*ldx .. + n_x); tile_begin counts row tiles
+// of PF_Q50_ROWS, pf_q50_rows or 32 rows.
+constexpr int PF_FT = 16;        // tokens per k_pf_gemm_q50s workgroup; per k_pf_gemm_f one, at most
+constexpr int PF_Q50_MAXB = 32;  // blocks per row of k_pf_gemm_q50s
+__host__ __device__ inline int pf_q50_rows(int nb8) { return nb8 < 256 ? 256 / nb8 : 1; }  // a block per thread
 constexpr int PF_Q50_ROWS = 64;  // rows of a k_pf_gemm_q50 wave
 constexpr int PF_Q50_TW = 4;     // row tiles per workgroup (ks = 1)
 struct PFGemmFParams {
@@ -439,7 +442,11 @@ template <int PRO, int MODE>
 __global__ void k_gemv_f(GemvParams P);
 constexpr int GF_XPAD = 36;  // floats per 32-element block of x in LDS (Q5_0 reads, bank spread)
 // Dynamic LDS of k_pf_gemm_f, bytes: x of one token.
-__host__ __device__ inline int pf_gemm_f_lds_bytes(int n_x) { return n_x / 32 * 32 * 4; }
+__host__ __device__ inline int pf_gemm_f_lds_bytes(int n_x, bool q50) { return n_x / 32 * (q50 ? GF_XPAD : 32) * 4; }
+// Dynamic LDS of k_pf_gemm_q50s, bytes: x of half the tokens, the terms.
+__host__ __device__ inline int pf_gemm_q50s_lds_bytes(int n_x) {
+  return ((PF_FT / 2) * (n_x / 32) * GF_XPAD + PF_FT * 256) * 4;
+}
 // Dynamic LDS of k_pf_gemm_q50 (KS), bytes: the later waves' terms of a
 // round; at most 48 KB: three workgroups per CU.
 constexpr int PF_Q50_KS_TOK = 8, PF_Q50_KS_MAX = 4, PF_Q50_PER_MAX = 8;
@@ -533,8 +540,10 @@ __host__ __device__ inline int pf_q6_lds_bytes(int nb, int ns) {
 }
 constexpr int PF_Q6_LDS_MAX = 128 * 1024;
 
-template <int MODE>
+template <int MODE, bool Q50>
 __global__ void k_pf_gemm_f(PFGemmFParams P);
+template <int MODE>
+__global__ void k_pf_gemm_q50s(PFGemmFParams P);
 // TOK tokens per wave; grid (row tiles / (ks > 1 ? 1 : PF_Q50_TW), token tiles)
 template <int MODE, int TOK, bool KS>
 __global__ void k_pf_gemm_q50(PFGemmFParams P);

@@ -85,3 +85,42 @@ def test_late_prompts_equal_forwards(late, pos0, n):
     print(pos0, n, flush=True)
     check_prompt(ctx, s, np.random.default_rng(pos0 + n).integers(0, s.n_vocab, n).astype(np.int32), pos0)
     fill(ctx, s, LATE)
+
+
+# Q5_0 projections of few tokens: a block per thread (k_pf_gemm_q50s,
+# k_pf_gemm_f) where k_pf_gemm_q50's waves would wait out a load per block.
+
+Q50 = dict(n_layers=2, n_vocab=2048, t_q=G.Q5_0, t_k=G.Q5_0, t_v=G.Q8_0, t_o=G.Q5_0, t_gate=G.Q5_0, t_up=G.Q5_0)
+
+
+# the same prompt with Q5_0 matrices and with others beside them: rows of 28
+# blocks against Q8_0 (a small FFN, so that q|k and o are much of the pass):
+# 1.23 measured, 1.89 with k_pf_gemm_q50 for all; rows of 152 blocks against
+# Q6_K: below 1, 1.52
+@pytest.mark.parametrize("kind,n,most", [("narrow", 8, 1.5), ("wide", 1, 1.2)])
+def test_few_q5_0_tokens_keep_up(kind, n, most, tmp_path):
+    if kind == "narrow":
+        a, b = (dict(Q50, n_ff=768, t_q=t, t_k=t, t_o=t, t_gate=t, t_up=t, t_down=t) for t in (G.Q5_0, G.Q8_0))
+    else:
+        a, b = (dict(Q50, t_down=t) for t in (G.Q5_0, G.Q6_K))
+    us = []
+    for i, kw in enumerate((a, b)):
+        s = G.ModelShape(**dict(kw, n_layers=6))
+        with open_model(tmp_path / f"{i}.gguf", s, 512) as ctx:
+            toks = np.random.default_rng(n).integers(0, s.n_vocab, n).astype(np.int32)
+            us.append(best_us(lambda: ctx.prefill(toks, 0), 9))
+    print(kind, us, us[0] / us[1], flush=True)
+    assert us[0] < most * us[1]
+
+
+# each kernel's tokens and tiles, and the lines between them: 16 tokens per
+# k_pf_gemm_q50s workgroup and 1,000 of those a launch (145 tokens of q|k,
+# 17 of gate|up); 7 tokens of wide rows; ffn_down rows of 24, 32, 33 (a
+# workgroup's 7 rows leave threads over) and 152 blocks
+@pytest.mark.parametrize("n_ff", [768, 1024, 1056, 4864])
+@pytest.mark.parametrize("n", [1, 7, 8, 16, 17, 128, 145])
+def test_q5_0_prompts_equal_forwards(n_ff, n, tmp_path):
+    s = G.ModelShape(**dict(Q50, n_ff=n_ff, t_down=G.Q5_0))
+    with open_model(tmp_path / "m.gguf", s, 256) as ctx:
+        print(n_ff, n, flush=True)
+        check_prompt(ctx, s, np.random.default_rng(n).integers(0, s.n_vocab, n).astype(np.int32), 0)
