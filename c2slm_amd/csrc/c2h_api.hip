@@ -95,7 +95,6 @@ struct c2h_ctx {
   float* att_sc = nullptr;  // [tokens of a launch][n_heads][sc_ld] scores / probabilities
   float* att_bmax = nullptr;
   int att_sc_ld = 0, att_n_blk = 0;
-  int sav_hpw = 1;  // query heads per k_attn_h128_sav workgroup
   int32_t seq_len = 0;   // KVCache.SeqLen (engine/kvcache.go:25-47)
 
   // batched prefill buffers (allocated by the first c2h_prefill)
@@ -616,11 +615,9 @@ AttnCoreParams attn_params(c2h_ctx* c, int layer) {
 void enqueue_attn_long(c2h_ctx* c, AttnCoreParams A, int ntok) {
   const c2h_model_desc& D = c->desc;
   if (D.head_dim == 128) {
-    A.hpw = c->sav_hpw;
-    A.sav_ld = pfa_sc_ld(D.max_ctx - 1);
     hipLaunchKernelGGL(k_attn_h128_scores, dim3(c->att_n_blk, D.n_kv_heads), dim3(256), 0, c->stream, A);
-    hipLaunchKernelGGL(k_attn_h128_sav, dim3(128 / 16, (D.n_heads / D.n_kv_heads + A.hpw - 1) / A.hpw, D.n_kv_heads),
-                       dim3(ATT_SAV_THREADS), (size_t)A.hpw * A.sav_ld * 4, c->stream, A);
+    hipLaunchKernelGGL(k_attn_h128_sav, dim3(128 / 16, D.n_heads), dim3(ATT_SAV_THREADS),
+                       (size_t)pfa_sc_ld(D.max_ctx - 1) * 4, c->stream, A);
     return;
   }
   hipLaunchKernelGGL(k_attn_scores, dim3(c->att_n_blk, D.n_kv_heads, ntok), dim3(256), 0, c->stream, A);
@@ -1497,11 +1494,9 @@ int c2h_create(const c2h_model_desc* desc, int device, c2h_ctx** out) {
     if ((rc = dalloc(c, &c->att_sc, rows * c->att_sc_ld * 4)) ||
         (rc = dalloc(c, &c->att_bmax, rows * c->att_n_blk * 4)))
       return bail(rc);
-    const size_t row = (size_t)pfa_sc_ld(D.max_ctx - 1) * 4;
-    c->sav_hpw = std::max(1, std::min(qpkv, (int)(PFA_LDS_MAX / row)));
     if (D.head_dim == 128
             ? hipFuncSetAttribute((const void*)k_attn_h128_sav, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)(c->sav_hpw * row)) != hipSuccess
+                                  pfa_sc_ld(D.max_ctx - 1) * 4) != hipSuccess
             : hipFuncSetAttribute((const void*)k_attn_softmax, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   attn_softmax_lds_floats(D.max_ctx) * 4) != hipSuccess ||
                   hipFuncSetAttribute((const void*)k_attn_av, hipFuncAttributeMaxDynamicSharedMemorySize,

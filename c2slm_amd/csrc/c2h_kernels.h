@@ -192,8 +192,8 @@ __host__ __device__ inline size_t vq_index(int p, int d, int hd = 64) {
 //     head and 16-dim slice: two waves run the FMA chains of all the group's
 //     query heads, the others stage the V slice through LDS).
 // At head_dim 128 the forms are k_attn_h128, and k_attn_h128_scores ->
-// k_attn_h128_sav (workgroups over 16 output dims of a group's query heads:
-// softmax, FMA chains).
+// k_attn_h128_sav (a workgroup per query head and 16 output dims: softmax, FMA
+// chains).
 constexpr int ATT_CH = 128;   // V positions staged in LDS per pass (chunk 0 prefetched)
 constexpr int ATT_KPF = 256;  // K rows per LDS chunk of the scores (one per thread)
 constexpr int ATT_KPAD = 68;  // floats per staged K row (64 + 4: conflict-free row reads)
@@ -266,7 +266,6 @@ struct AttnCoreParams {
   // at once.  0 = the grid is (qpkv, n_kv_heads, tokens).
   int xcd_map;
   int tok_blk;      // k_pf_attn: query tokens of a workgroup
-  int hpw, sav_ld;  // k_attn_h128_sav: query heads per workgroup, its LDS row stride (pfa_sc_ld)
 };
 constexpr int ATT_XCDS = 8;
 

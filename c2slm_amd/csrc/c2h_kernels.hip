@@ -3626,17 +3626,18 @@ __device__ __forceinline__ float row_max_dpp(float x) {
 //   k_attn_h128_scores  per block of H128_SB positions: QK-norm, RoPE, K/V
 //                  store, scores of the KV head's query heads (each K row
 //                  read once), block maxima per head;
-//   k_attn_h128_sav     per 16 output dims and group of query heads: max, f64
-//                  exp, the sequential f32 sum (exact speculative form),
-//                  p = e * (1/sum), the FMA chain over p = 0..pos in order.
+//   k_attn_h128_sav     per 16 output dims of a query head: max, f64 exp, the
+//                  sequential f32 sum (exact speculative form), p = e *
+//                  (1/sum), the FMA chain over p = 0..pos in order.
 // The chain is what bounds k_attn_h128_sav (50 clk per four positions); its
-// workgroups repeat the softmax of their heads, which costs less than a
-// launch and a trip of the probabilities through memory.  1,500 positions,
-// 12 heads: 6.1 + 16.2 us against k_attn_h128's 34.1; the same at ~512, where
-// the split lies (a decode step of four layers at 384, 512, 768 positions:
-// 182, 193, 212 us with one launch, 188, 193, 199 with two).  At head_dim 64
-// k_attn_softmax and k_attn_av stay: their chain runs on VALU fmas at 8.0 clk
-// per position, and at 4,096 positions the pair took 31 us against 40.
+// workgroups repeat the softmax of their head, which costs less than a launch
+// and a trip of the probabilities through memory.  12 heads, sessions of
+// 2,048: 17.3 us at 512 positions and 28.3 at 1,500, where k_attn_h128 takes
+// 19.3 and 42.9 (16 heads, 16,384: 20.8 and 32.2 against 21.9 and 45.6).  The
+// two are equal at 384 positions, so the split at 512 leaves up to 0.7 us.  At
+// head_dim 64 k_attn_softmax and k_attn_av stay: their chain runs on VALU
+// fmas at 8.0 clk per position, and at 4,096 positions the pair took 31 us
+// against 40.
 
 __global__ void __launch_bounds__(256) k_attn_h128_scores(AttnCoreParams P) {
   constexpr int HD = 128, NG = HD / 64, H2 = HD / 2;
@@ -3765,47 +3766,46 @@ __global__ void __launch_bounds__(256) k_attn_h128_scores(AttnCoreParams P) {
   }
 }
 
-// Exps to probabilities in MFMA operand order, in place: rows of ld floats,
-// each times its 1/sum, the 16 positions of a group transposed as a 4 x 4
-// block (position 4 c + k at slot 4 k + c), so that lane row k reads the
-// operands of four consecutive instructions as 16 bytes.  Position p is then
-// at prob_slot(p).  A thread per row and group; the caller's barriers around.
+// Exps to probabilities in MFMA operand order, in place: each times 1/sum,
+// the 16 positions of a group transposed as a 4 x 4 block (position 4 c + k
+// at slot 4 k + c), so that lane row k reads the operands of four consecutive
+// instructions as 16 bytes.  Position p is then at prob_slot(p).  A thread
+// per group; the caller's barriers around.
 __device__ __forceinline__ int prob_slot(int p) { return (p & ~15) + 4 * (p & 3) + ((p >> 2) & 3); }
-__device__ __forceinline__ void probs_in_order(float* e, int rows, int ld, int groups, const float* inv, int nthr) {
-  for (int i = threadIdx.x; i < rows * groups; i += nthr) {
-    const int r = i / groups;
-    f32x4_t* g = reinterpret_cast<f32x4_t*>(e + r * ld + 16 * (i - r * groups));
-    const float iv = inv[r];
+__device__ __forceinline__ void probs_in_order(float* e, int groups, float inv, int nthr) {
+  for (int i = threadIdx.x; i < groups; i += nthr) {
+    f32x4_t* g = reinterpret_cast<f32x4_t*>(e + 16 * i);
     f32x4_t x[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) x[c] = g[c];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const f32x4_t y = {x[0][k] * iv, x[1][k] * iv, x[2][k] * iv, x[3][k] * iv};
+      const f32x4_t y = {x[0][k] * inv, x[1][k] * inv, x[2][k] * inv, x[3][k] * inv};
       g[k] = y;
     }
   }
 }
 
-// Grid (HD / 16 slices of dims, head groups, KV heads), P.hpw query heads
-// per workgroup; dynamic LDS [P.hpw][P.sav_ld] exps.
+// Grid (HD / 16 slices of dims, query heads), dynamic LDS pfa_sc_ld(max_ctx -
+// 1) exps.  One head per workgroup: the other rows of its tiles repeat it, and
+// a KV head's V comes once per query head, from L2.  With as many heads as
+// the LDS held per workgroup their softmaxes ran one after the other, and the
+// kernel's time followed the session length that the LDS was sized for.
 __global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParams P) {
   constexpr int HD = 128;
   constexpr int NT = ATT_SAV_THREADS;
   extern __shared__ __align__(16) unsigned char smem[];
   float* e = reinterpret_cast<float*>(smem);
   __shared__ double exp_tab[EXP_TAB];
-  __shared__ float mx_s[8], inv_s[8];
+  __shared__ float mx_s, inv_s;
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = blockIdx.z;
-  const int qpkv = P.n_heads / P.n_kv_heads;
-  const int h0 = blockIdx.y * P.hpw, nh = min(P.hpw, qpkv - h0);
-  const int ld = P.sav_ld;
+  const int h = blockIdx.y;
+  const int g = h / (P.n_heads / P.n_kv_heads);
   const int T = P.state->pos + 1;
   const size_t head_stride = (size_t)kv_slot(P.max_ctx) * HD;
   const float* vcache = P.kv + (((size_t)P.n_layers + P.layer) * P.n_kv_heads + g) * head_stride;
-  const float* srow = P.sc + ((size_t)g * qpkv + h0) * P.sc_ld;
+  const float* srow = P.sc + (size_t)h * P.sc_ld;
   load_exp_tab(exp_tab);
 
   // V as B operands, a dword each (lane (col, kg): position 4 quad + kg of
@@ -3825,22 +3825,22 @@ __global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParam
     for (int k = 0; k < VB; ++k) vr[k] = (vcache + (size_t)min(nbat * VB + k, nq - 1) * (4 * HD))[vl];
     vt = reinterpret_cast<const f32x4_t*>(vcache)[(size_t)(nq - 1) * HD + dim];
   }
-  // ---- max: wave w head w, over its block maxima (never NaN); NaN when score 0 is
-  if (wave < nh) {
+  // ---- max over the block maxima (never NaN); NaN when score 0 is
+  if (wave == 1) {
     const int nb = (T + H128_SB - 1) / H128_SB;
-    const float* bmx = P.bmax + ((size_t)g * qpkv + h0 + wave) * P.n_blk;
+    const float* bmx = P.bmax + (size_t)h * P.n_blk;
     float lm = -__builtin_inff();
     for (int b = lane; b < nb; b += 64) lm = fmax_gt(lm, bmx[b]);
     lm = wave_max_dpp(lm);
-    const float s0 = srow[(size_t)wave * P.sc_ld];
-    if (lane == 0) mx_s[wave] = s0 != s0 ? s0 : lm;
+    const float s0 = srow[0];
+    if (lane == 0) mx_s = s0 != s0 ? s0 : lm;
   }
   __syncthreads();
   // ---- exps (eight loads of four positions in flight)
-  for (int r = 0; r < nh; ++r) {
-    const float m = mx_s[r];
-    const f32x4_t* s4 = reinterpret_cast<const f32x4_t*>(srow + (size_t)r * P.sc_ld);
-    f32x4_t* e4 = reinterpret_cast<f32x4_t*>(e + r * ld);
+  {
+    const float m = mx_s;
+    const f32x4_t* s4 = reinterpret_cast<const f32x4_t*>(srow);
+    f32x4_t* e4 = reinterpret_cast<f32x4_t*>(e);
     for (int i0 = tid; i0 < nq; i0 += 8 * NT) {
       f32x4_t s[8];
 #pragma unroll
@@ -3856,25 +3856,24 @@ __global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParam
     }
   }
   __syncthreads();
-  // the sequential sums, wave w head w
-  if (wave < nh) {
-    const float* a = e + wave * ld;
-    const float s = (T <= 64 * SPEC_C)    ? seq_sum_wave(a, T)
-                    : (T <= 128 * SPEC_C) ? seq_sum_wave<2 * SPEC_C>(a, T)
-                                          : seq_sum_wave_n(a, T);
-    if (lane == 0) inv_s[wave] = 1.0f / s;
+  // the sequential sum
+  if (wave == 1) {
+    const float s = (T <= 64 * SPEC_C)    ? seq_sum_wave(e, T)
+                    : (T <= 128 * SPEC_C) ? seq_sum_wave<2 * SPEC_C>(e, T)
+                                          : seq_sum_wave_n(e, T);
+    if (lane == 0) inv_s = 1.0f / s;
   }
   __syncthreads();
-  probs_in_order(e, nh, ld, (nq + 3) >> 2, inv_s, NT);
+  probs_in_order(e, (nq + 3) >> 2, inv_s, NT);
   __syncthreads();
   if (wave != 0) return;  // no barrier follows
 
-  // ---- AV: A row col = head, four positions per instruction.  An FP32 MFMA
+  // ---- AV: A rows the head, four positions per instruction.  An FP32 MFMA
   // holds up its own wave's VALU for its 32 clk, so the chain's loop has
   // none: the probabilities come four instructions' at a time from LDS, V as
   // operands, NV batches ahead (with a multiply, lane swaps and copies per
   // instruction it ran at 75 clk instead of 50).
-  const f32x4_t* arow = reinterpret_cast<const f32x4_t*>(e + min(col, nh - 1) * ld + 4 * kg);
+  const f32x4_t* arow = reinterpret_cast<const f32x4_t*>(e + 4 * kg);
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
   f32x4_t a[2][VB / 4];
 #pragma unroll
@@ -3907,15 +3906,11 @@ __global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParam
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float*>(arow + VB * nbat + 4 * (k / 4))[k % 4],
                                                  vr[k], acc, 0, 0, 0);
   // the last one to three positions
+  float x = acc[0];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = min(4 * kg + i, nh - 1);
-    float x = acc[i];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      if (4 * nfull + c < T) x = __builtin_fmaf(e[r * ld + prob_slot(4 * nfull + c)], vt[c], x);
-    if (4 * kg + i < nh) P.out[((size_t)g * qpkv + h0 + r) * HD + dim] = x;
-  }
+  for (int c = 0; c < 3; ++c)
+    if (4 * nfull + c < T) x = __builtin_fmaf(e[prob_slot(4 * nfull + c)], vt[c], x);
+  if (kg == 0) P.out[(size_t)h * HD + dim] = x;
 }
 
 // Causal attention of a prefill pass: workgroup (query head h, block of

@@ -1,6 +1,6 @@
-"""Prompts take, at each size, the kernels that suit it: the time of one
-against that of work the other route would not keep up with, with a wide
-margin on both sides, and bit for bit what one forward per token leaves."""
+"""Prompts and decode steps take, at each size, the kernels that suit it: the
+time of one against that of work the other route would not keep up with, with
+a wide margin on both sides, and bit for bit what one forward per token leaves."""
 import time
 
 import numpy as np
@@ -124,3 +124,23 @@ def test_q5_0_prompts_equal_forwards(n_ff, n, tmp_path):
     with open_model(tmp_path / "m.gguf", s, 256) as ctx:
         print(n_ff, n, flush=True)
         check_prompt(ctx, s, np.random.default_rng(n).integers(0, s.n_vocab, n).astype(np.int32), 0)
+
+
+# Decode attention at head_dim 128 past the split: no slower than the one
+# launch it replaces there (0.82 measured; with a workgroup per group of heads
+# 1.13).
+
+def test_h128_two_launches_no_slower_than_one(tmp_path, monkeypatch):
+    s = G.ModelShape(n_layers=2, n_embd=1536, n_heads=12, n_kv_heads=2, n_ff=8960, n_vocab=2048)
+    ctxs = []
+    for split in (None, "2047"):
+        if split is not None:
+            monkeypatch.setenv("C2H_ATT_SPLIT", split)
+        ctxs.append(open_model(tmp_path / "m.gguf", s, 2048))
+        fill(ctxs[-1], s, 530)
+        ctxs[-1].set_seq(520)
+    two, one = np.min([[c.time_layer_kernel("attn", 200, True) * 1e3 for c in ctxs] for _ in range(6)], axis=0)
+    print(two, one, two / one, flush=True)
+    for c in ctxs:
+        c.close()
+    assert two < 1.05 * one
