@@ -1706,10 +1706,23 @@ __device__ __forceinline__ void gemv_f_body(const int bx, const int by, const Ge
           if (PAIRED) acc2 = acc2 + tb[PAIRED ? b : 0];
         }
       }
-    } else if (tid < R) {  // wider rows (a Q5_0 ffn_down): one row per workgroup
-      for (int b = 0; b < nb8; ++b) acc = acc + terms[0][tid * nb8 + b];
-      if (PAIRED)
-        for (int b = 0; b < nb8; ++b) acc2 = acc2 + terms[PAIRED ? 1 : 0][tid * nb8 + b];
+    } else {  // wider rows (a Q5_0 ffn_down): R = 256 / nb8 rows, past 256 blocks one
+      const int n0 = min(nb8, 256);
+      if (tid < R) {
+        for (int b = 0; b < n0; ++b) acc = acc + terms[0][tid * nb8 + b];
+        if (PAIRED)
+          for (int b = 0; b < n0; ++b) acc2 = acc2 + terms[PAIRED ? 1 : 0][tid * nb8 + b];
+      }
+      if constexpr (PRO == PRO_QUANT && !TAGX) {  // (the others' x is n_embd long: 32 blocks)
+        for (int b0 = 256; b0 < nb8; b0 += 256) {  // uniform
+          __syncthreads();                         // the terms before are added
+          const int b = b0 + tid;
+          if (b < nb8) terms[0][tid] = q50_term(load_q50(J.w, nb8, row_c, b), xq + b * GF_XPAD);
+          __syncthreads();
+          if (tid == 0)
+            for (int i = 0; i < min(nb8 - b0, 256); ++i) acc = acc + terms[0][i];
+        }
+      }
     }
   } else {
     acc = q80_row_sum(q80_lane_acc(w8a, xp, nb8, lane8));

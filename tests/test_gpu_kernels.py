@@ -213,6 +213,15 @@ def test_gemv_q5_0_bitexact(ctx, rows, cols):
     assert np.array_equal(bits(got), bits(want))
 
 
+# more blocks than a workgroup has threads: 256 exactly, one more, 280, 313
+@pytest.mark.parametrize("rows,cols", [(5, 8192), (5, 8224), (4, 8960), (3, 10016)])
+def test_gemv_q5_0_wide_rows(ctx, rows, cols):
+    rng = np.random.default_rng(cols)
+    w = G.synth_q5_0(rng, rows * (cols // 32))
+    x = rng.normal(size=cols).astype(np.float32)
+    assert np.array_equal(bits(ctx.gemv(H.Q5_0, w, x, rows, cols)), bits(O.gemv(w, G.Q5_0, rows, cols, x=x)))
+
+
 def test_gemv_q5_0_order_known_answers(ctx):
     from tests.test_oracle import q5_0_block
     ones = q5_0_block(0x3C00, 0xFFFFFFFF, [0x11] * 16)

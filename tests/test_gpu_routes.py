@@ -116,8 +116,9 @@ def test_few_q5_0_tokens_keep_up(kind, n, most, tmp_path):
 # each kernel's tokens and tiles, and the lines between them: 16 tokens per
 # k_pf_gemm_q50s workgroup and 1,000 of those a launch (145 tokens of q|k,
 # 17 of gate|up); 7 tokens of wide rows; ffn_down rows of 24, 32, 33 (a
-# workgroup's 7 rows leave threads over) and 152 blocks
-@pytest.mark.parametrize("n_ff", [768, 1024, 1056, 4864])
+# workgroup's 7 rows leave threads over), 152 and 280 blocks (past the 256 of
+# a decode workgroup's threads)
+@pytest.mark.parametrize("n_ff", [768, 1024, 1056, 4864, 8960])
 @pytest.mark.parametrize("n", [1, 7, 8, 16, 17, 128, 145])
 def test_q5_0_prompts_equal_forwards(n_ff, n, tmp_path):
     s = G.ModelShape(**dict(Q50, n_ff=n_ff, t_down=G.Q5_0))
