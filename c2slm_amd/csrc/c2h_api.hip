@@ -819,7 +819,6 @@ AttnCoreParams fused_attn_params(c2h_ctx* c, int l) {
   A.k = c->k;
   A.v = c->v;
   A.out = c->attn;
-  A.store_kv = 1;
   A.xcd_map = 1;
   A.out_tag = c->attn_tag;
   A.n_attn_wg = ATT_XCDS * (D.n_heads / D.n_kv_heads);

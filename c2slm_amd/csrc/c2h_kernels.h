@@ -224,9 +224,9 @@ constexpr int ATT_AV_SLICES = 64 / ATT_AV_DSL;
 constexpr int ATT_AV_ITEMS = 6;      // 16-byte staging items per staging lane and chunk
 constexpr int ATT_MAX_QPKV = 8;    // query heads per KV head the long form handles
 constexpr int ATT_LONG_MAX_CTX = 36864;  // exps of one head in LDS (k_attn_softmax)
-// grid (n_heads, tokens) for k_attn_core / k_attn_softmax / k_attn_av and
-// (blocks, n_kv_heads, tokens) for k_attn_scores: query token i of a launch
-// sits at position state->pos + tok0 + i; decode launches one token.
+// k_attn_scores, k_attn_softmax and k_attn_av take several query tokens of a
+// prompt in their grid's last dimension, token i at position state->pos + tok0
+// + i; the other decode kernels take the one at state->pos.
 struct AttnCoreParams {
   const float* q;  // [tokens][q_ld]: n_heads*hd, bias added, before QK-norm and RoPE
   const float* k;  // [tokens][kv_ld]: n_kv_heads*hd
@@ -239,7 +239,7 @@ struct AttnCoreParams {
   int n_attn_wg;      // k_attn_oproj: workgroups of the attention half
   int* wait_err;      // k_attn_block: the flag a wait for q|k|v that runs out sets
   int q_ld, kv_ld, out_ld;
-  int store_kv;    // 1: K/V of pos come from k/v and are stored by this launch
+  int store_kv;    // k_attn_scores, 1: K/V of pos come from k/v and are stored by this launch
   float* kv;
   const float* rope_cos;
   const float* rope_sin;

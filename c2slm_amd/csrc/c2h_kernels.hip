@@ -2082,7 +2082,7 @@ struct VStage {
   f32x4_t r[PER];
 };
 
-// The body of k_attn_core for workgroup (bx, by, bz) of its grid.  TAG:
+// The body of k_attn_core for workgroup (bx, by) of its grid.  TAG:
 // the output is also stored as 8-byte {value, tag} words in P.out_tag for
 // the consumers of the same launch (k_attn_oproj), tag = the state's epoch
 // * 256 + layer.  TAGIN (with TAG): q|k|v come from producers of the same
@@ -2090,7 +2090,7 @@ struct VStage {
 // at (n_heads + g)*64, v at (n_heads + n_kv + g)*64), polled after the K/V
 // rows and the position have been issued.
 template <int TIER, bool TAG, bool TAGIN = false>
-__device__ __forceinline__ void attn_core_body(const int bx, const int by, const int bz, C2hState* __restrict__ st,
+__device__ __forceinline__ void attn_core_body(const int bx, const int by, C2hState* __restrict__ st,
                                                float* __restrict__ kv, const float* __restrict__ qg,
                                                const float* __restrict__ kg, const float* __restrict__ vg, int dims,
                                                int max_ctx, const AttnCoreParams& P,
@@ -2117,8 +2117,8 @@ __device__ __forceinline__ void attn_core_body(const int bx, const int by, const
   const int tid = threadIdx.x;
   const int layer = dims & 0xff, n_layers = (dims >> 8) & 0xff, n_kv = (dims >> 16) & 0x7f;
   const int qpkv = (dims >> 24) & 0xff;
-  // grid (query heads per KV head, KV heads, query tokens of the batch), or
-  // the XCD-grouped order of xcd_map (at most ATT_XCDS KV heads)
+  // grid (query heads per KV head, KV heads), or the XCD-grouped order of
+  // xcd_map (at most ATT_XCDS KV heads)
   int g = by, hx = bx;
   if ((dims >> 23) & 1) {
     g = bx % ATT_XCDS;
@@ -2126,16 +2126,14 @@ __device__ __forceinline__ void attn_core_body(const int bx, const int by, const
     if (g >= n_kv) return;  // uniform: a spare workgroup of the grid
   }
   const int h = g * qpkv + hx;
-  // query token of the batch (the tiers serve decode: one token, row 0)
-  const int ti = ANY ? P.tok0 + bz : 0;
   // this head's q and the group's k, v: thread t < 192 holds element t%64
   // of q_h (t < 64), k_g, v_g.  Issued before the position is read.
   const int bm = min(tid >> 6, 2);
   float own = 0.0f;
   if constexpr (!TAGIN) {
-    const float* qsrc = qg + (ANY ? (size_t)ti * P.q_ld : 0) + h * HD;
-    const float* ksrc = kg + (ANY ? (size_t)ti * P.kv_ld : 0) + g * HD;
-    const float* vsrc = vg + (ANY ? (size_t)ti * P.kv_ld : 0) + g * HD;
+    const float* qsrc = qg + h * HD;
+    const float* ksrc = kg + g * HD;
+    const float* vsrc = vg + g * HD;
     own = ((bm == 0) ? qsrc : ((bm == 1) ? ksrc : vsrc))[tid & 63];
   }
   // the position, and for a tier its RoPE row from the state: issued now,
@@ -2182,13 +2180,12 @@ __device__ __forceinline__ void attn_core_body(const int bx, const int by, const
   }
   // the other fields in one scalar batch (a scalar load still in flight
   // would make every later LDS wait, which shares its counter, wait too)
-  asm volatile("" ::"s"(P.rope_cos), "s"(P.rope_sin), "s"(P.q_ld), "s"(P.kv_ld), "s"(P.tok0), "s"(P.rope_len),
-               "s"(P.out), "s"(P.out_ld), "s"(P.scale), "s"(P.store_kv));
+  asm volatile("" ::"s"(P.rope_cos), "s"(P.rope_sin), "s"(P.rope_len), "s"(P.out), "s"(P.scale));
   asm volatile("" : "+v"(pos_state));
   // the RoPE row is used here, so its loads stay ahead of the K/V loads
   // (used only under the rotation's branch, they would be sunk behind them)
   if constexpr (!ANY) asm volatile("" ::"v"(rcos), "v"(rsin));
-  const int pos = __builtin_amdgcn_readfirstlane(pos_state) + ti;
+  const int pos = __builtin_amdgcn_readfirstlane(pos_state);
   const int T = pos + 1;
   const int nstored = max(min(pos, max_ctx), 0);    // cached positions [0, nstored)
   const int nch = (pos + ATT_CH - 1) / ATT_CH;         // V chunks of positions [0, pos)
@@ -2198,7 +2195,7 @@ __device__ __forceinline__ void attn_core_body(const int bx, const int by, const
   const __amdgpu_buffer_rsrc_t vrs = cache_rsrc(vcache, ((nstored + 3) >> 2) * HD * 16);
 
   // ---- loads, in the order they are consumed
-  if constexpr (ANY) {  // a batch of query tokens: each its own row of the table
+  if constexpr (ANY) {
     const int rp = min(max(pos, 0), P.rope_len - 1);
     rcos = P.rope_cos[(size_t)rp * (HD / 2) + (tid & 31)];
     rsin = P.rope_sin[(size_t)rp * (HD / 2) + (tid & 31)];
@@ -2235,8 +2232,7 @@ __device__ __forceinline__ void attn_core_body(const int bx, const int by, const
   }
   __syncthreads();
 
-  // (a batch of query tokens has its K/V stored by a kernel before this one)
-  if (P.store_kv && hx == 0 && tid < HD && pos < max_ctx) {
+  if (hx == 0 && tid < HD && pos < max_ctx) {
     kcache[(size_t)pos * HD + tid] = k_s[tid];
     vcache[vq_index(pos, tid)] = v_s[tid];
   }
@@ -2401,7 +2397,7 @@ __device__ __forceinline__ void attn_core_body(const int bx, const int by, const
   }
   if (tid < HD) {
     acc = __builtin_fmaf(sc[pos], v_s[d], acc);
-    P.out[(size_t)ti * P.out_ld + h * HD + d] = acc;
+    P.out[h * HD + d] = acc;
     if constexpr (TAG) {
       const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane(epoch_state) * 256u + (uint32_t)layer;
       __hip_atomic_store(&P.out_tag[h * HD + d], ((uint64_t)tag << 32) | __float_as_uint(acc), __ATOMIC_RELAXED,
@@ -2414,8 +2410,7 @@ template <int TIER>
 __global__ void __launch_bounds__(256)
     k_attn_core(C2hState* __restrict__ st, float* __restrict__ kv, const float* __restrict__ qg,
                 const float* __restrict__ kg, const float* __restrict__ vg, int dims, int max_ctx, AttnCoreParams P) {
-  attn_core_body<TIER, false>((int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, st, kv, qg, kg, vg, dims, max_ctx,
-                              P);
+  attn_core_body<TIER, false>((int)blockIdx.x, (int)blockIdx.y, st, kv, qg, kg, vg, dims, max_ctx, P);
 }
 template __global__ void k_attn_core<ATT_TIER_32>(C2hState*, float*, const float*, const float*, const float*, int, int,
                                                    AttnCoreParams);
@@ -2445,7 +2440,7 @@ __global__ void __launch_bounds__(256)
   static_assert(row_threads(NB, PRO_QUANT, MODE_RESID) == 256, "both halves run 256-thread workgroups");
   const int n_attn = P.n_attn_wg;
   if ((int)blockIdx.x < n_attn) {
-    attn_core_body<TIER, true>((int)blockIdx.x, 0, 0, st, kv, qg, kg, vg, dims, max_ctx, P);
+    attn_core_body<TIER, true>((int)blockIdx.x, 0, st, kv, qg, kg, vg, dims, max_ctx, P);
     return;
   }
   const uint32_t tag = (uint32_t)st->epoch * 256u + (uint32_t)(dims & 0xff);
@@ -2482,7 +2477,7 @@ __global__ void __launch_bounds__(256)
   }
   const int n_attn = P.n_attn_wg;
   if (b < nq + n_attn) {
-    attn_core_body<TIER, true, true>(b - nq, 0, 0, st, kv, nullptr, nullptr, nullptr, dims, max_ctx, P, qkv_tag);
+    attn_core_body<TIER, true, true>(b - nq, 0, st, kv, nullptr, nullptr, nullptr, dims, max_ctx, P, qkv_tag);
     return;
   }
   const uint32_t tag = (uint32_t)st->epoch * 256u + (uint32_t)(dims & 0xff);
@@ -2518,7 +2513,7 @@ __global__ void __launch_bounds__(256)
   }
   const int n_attn = P.n_attn_wg;
   if (b < nq + n_attn) {
-    attn_core_body<TIER, true, true>(b - nq, 0, 0, st, kv, nullptr, nullptr, nullptr, dims, max_ctx, P, qkv_tag);
+    attn_core_body<TIER, true, true>(b - nq, 0, st, kv, nullptr, nullptr, nullptr, dims, max_ctx, P, qkv_tag);
     return;
   }
   gemv_f_body<PRO_QUANT, MODE_RESID, true, false, true>(b - nq - n_attn, 0, Go, tag);
@@ -2572,8 +2567,8 @@ C2H_ATTN_OPROJ(ATT_TIER_ANY, 3)
 //   what limits), the first ones issued while wave 0 sums the exponentials;
 //   the chains read each chunk from LDS, one barrier per chunk.
 // The scores of every position sit in LDS (P.sc_ld floats,
-// attn_h128_lds_floats(max_ctx)), the V buffers (VCH > 0) after them.
-// Grid (query heads per KV head, KV heads, query tokens); 256 threads.
+// attn_h128_lds_floats of the split), the V buffers (VCH > 0) after them.
+// Grid (query heads per KV head, KV heads); 256 threads.
 template <int VCH>
 __global__ void __launch_bounds__(256) k_attn_h128(AttnCoreParams P) {
   constexpr int VQ = VCH / 4 > 0 ? VCH / 4 : 1;  // V quads per chunk
@@ -2587,26 +2582,24 @@ __global__ void __launch_bounds__(256) k_attn_h128(AttnCoreParams P) {
 
   // the launch's fields in one scalar batch (see k_attn_core)
   asm volatile("" ::"s"(P.q), "s"(P.k), "s"(P.v), "s"(P.q_norm), "s"(P.k_norm), "s"(P.eps), "s"(P.out),
-               "s"(P.q_ld), "s"(P.kv_ld), "s"(P.out_ld), "s"(P.store_kv), "s"(P.kv), "s"(P.rope_cos),
-               "s"(P.rope_sin), "s"(P.rope_len), "s"(P.layer), "s"(P.n_layers), "s"(P.n_kv_heads), "s"(P.max_ctx),
-               "s"(P.scale), "s"(P.state), "s"(P.tok0), "s"(gridDim.x));
+               "s"(P.kv), "s"(P.rope_cos), "s"(P.rope_sin), "s"(P.rope_len), "s"(P.layer), "s"(P.n_layers),
+               "s"(P.n_kv_heads), "s"(P.max_ctx), "s"(P.scale), "s"(P.state), "s"(gridDim.x));
   const int tid = threadIdx.x;
   const int qpkv = (int)gridDim.x;
   const int g = (int)blockIdx.y;
   const int h = g * qpkv + (int)blockIdx.x;
-  const int ti = P.tok0 + (int)blockIdx.z;  // query token of the batch (0 in decode)
   const int e = tid & (HD - 1);
   const int role = tid >> 7;  // 0: this thread holds q_h[e], 1: k_g[e]
   const bool has_q_norm = P.q_norm != nullptr, has_k_norm = P.k_norm != nullptr;
   // ---- loads: q_h / k_g element, v_g element, the head-norm weight, then
   // the position and the RoPE row
-  const float* src = role == 0 ? P.q + (size_t)ti * P.q_ld + h * HD : P.k + (size_t)ti * P.kv_ld + g * HD;
+  const float* src = role == 0 ? P.q + h * HD : P.k + g * HD;
   const float own = src[e];
-  const float vown = P.v[(size_t)ti * P.kv_ld + g * HD + e];
+  const float vown = P.v[g * HD + e];
   const float* nsrc = role == 0 ? P.q_norm : P.k_norm;
   const float nwt = nsrc ? nsrc[e] : 1.0f;
   issue_fence();
-  const int pos = P.state->pos + ti;
+  const int pos = P.state->pos;
   const int T = pos + 1;
   const size_t head_stride = (size_t)kv_slot(P.max_ctx) * HD;
   float* kcache = P.kv + ((size_t)P.layer * P.n_kv_heads + g) * head_stride;
@@ -2649,7 +2642,7 @@ __global__ void __launch_bounds__(256) k_attn_h128(AttnCoreParams P) {
   }
   __syncthreads();
 
-  if (P.store_kv && blockIdx.x == 0 && tid < HD && pos < P.max_ctx) {
+  if (blockIdx.x == 0 && tid < HD && pos < P.max_ctx) {
     kcache[(size_t)pos * HD + tid] = k_s[tid];
     vcache[vq_index(pos, tid, HD)] = v_s[tid];
   }
@@ -2759,7 +2752,7 @@ __global__ void __launch_bounds__(256) k_attn_h128(AttnCoreParams P) {
       float acc = 0.0f;
       if (pos > 0) acc = av_chain_q3<HD>(sc, reinterpret_cast<const f32x4_t*>(vcache), pos, tid, acc);
       acc = __builtin_fmaf(sc[pos], v_s[tid], acc);
-      P.out[(size_t)ti * P.out_ld + h * HD + tid] = acc;
+      P.out[h * HD + tid] = acc;
     }
   } else {
     f32x4_t* vbuf = reinterpret_cast<f32x4_t*>(sc + P.sc_ld);  // [2][VQ][HD]
@@ -2794,7 +2787,7 @@ __global__ void __launch_bounds__(256) k_attn_h128(AttnCoreParams P) {
         acc = av_chain_q3<HD>(sc + c * VCH, vbuf + (c & 1) * VQ * HD, min(VCH, pos - c * VCH), tid, acc);
       }
       acc = __builtin_fmaf(sc[pos], v_s[tid], acc);
-      P.out[(size_t)ti * P.out_ld + h * HD + tid] = acc;
+      P.out[h * HD + tid] = acc;
     }
   }
 }

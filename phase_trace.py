@@ -86,14 +86,14 @@ __device__ __forceinline__ int phase_kind_f() {
 #define PH_AT(k, t) do { if ((threadIdx.x & 63) == 0) ph_s_[threadIdx.x >> 6][k] = (t); } while (0)
 #define PH_A_END do { const bool f_ = h == 0; \
   const bool l_ = h == P.n_heads - 1; \
-  if ((threadIdx.x & 63) == 0 && bz == 0 && (f_ || l_)) \
+  if ((threadIdx.x & 63) == 0 && (f_ || l_)) \
     for (int k_ = 0; k_ < 16; ++k_) \
       g_phase[TIER == ATT_TIER_ANY ? 5 : 4][f_ ? 0 : 1][threadIdx.x >> 6][k_] = ph_s_[threadIdx.x >> 6][k_]; } while (0)
 #define PH_A(k) PH_AT(k, __builtin_amdgcn_s_memtime())
 // k_attn_h128 (no k_attn_core runs at head_dim 128): its stamps take the attention slot
 #define PH_H_END do { const bool f_ = h == 0; \
   const bool l_ = h == (int)(gridDim.x * gridDim.y) - 1; \
-  if ((threadIdx.x & 63) == 0 && blockIdx.z == 0 && (f_ || l_)) \
+  if ((threadIdx.x & 63) == 0 && (f_ || l_)) \
     for (int k_ = 0; k_ < 16; ++k_) \
       g_phase[4][f_ ? 0 : 1][threadIdx.x >> 6][k_] = ph_s_[threadIdx.x >> 6][k_]; } while (0)
 """
@@ -142,8 +142,7 @@ def instrument(kernels: str) -> str:
                    ("  const int tid = threadIdx.x;\n  const int layer = dims & 0xff",
                     "  PH_DECL;\n  const long long ph_entry_ = __builtin_amdgcn_s_memtime();\n"
                     "  const int tid = threadIdx.x;\n  const int layer = dims & 0xff"),
-                   ('"s"(P.scale), "s"(P.store_kv));\n', '"s"(P.scale), "s"(P.store_kv));\n'
-                    '  PH_A(1);\n'),
+                   ('"s"(P.out), "s"(P.scale));\n', '"s"(P.out), "s"(P.scale));\n  PH_A(1);\n'),
                    ("  const int h = g * qpkv + hx;\n", "  const int h = g * qpkv + hx;\n  PH_AT(0, ph_entry_);\n"),
                    ("  const int T = pos + 1;\n", "  asm volatile(\"\" ::\"s\"(pos));\n  PH_A(9);\n  const int T = pos + 1;\n"),
                    ("    __syncthreads();\n    const int p = c0 + tid;\n",
@@ -156,8 +155,8 @@ def instrument(kernels: str) -> str:
                     "      while_summing();\n    }\n    PH_A(14);\n"),
                    ("  qkv_s[bm][tid & 63] = own;\n  __syncthreads();\n",
                     "  PH_A(2);\n  qkv_s[bm][tid & 63] = own;\n  __syncthreads();\n  PH_A(3);\n"),
-                   ("  __syncthreads();\n\n  // (a batch of query tokens",
-                    "  __syncthreads();\n  PH_A(4);\n\n  // (a batch of query tokens"),
+                   ("  if (hx == 0 && tid < HD && pos < max_ctx) {\n",
+                    "  PH_A(4);\n  if (hx == 0 && tid < HD && pos < max_ctx) {\n"),
                    ("  // softmax, then V chunk 0 from registers into LDS buffer 0\n",
                     "  PH_A(5);\n  // softmax, then V chunk 0 from registers into LDS buffer 0\n"),
                    ("    softmax([] {});\n    if (tid < HD && nbat > 0) acc = av_chain_pad(sc, vbuf, nbat, d, acc);\n",
@@ -198,12 +197,12 @@ def instrument(kernels: str) -> str:
                    ("  extern __shared__ __align__(16) unsigned char smem[];\n  float* sc = reinterpret_cast<float*>(smem);\n",
                     "  extern __shared__ __align__(16) unsigned char smem[];\n  float* sc = reinterpret_cast<float*>(smem);\n"
                     "  PH_DECL;\n  const long long ph_entry_ = __builtin_amdgcn_s_memtime();\n"),
-                   ('"s"(P.scale), "s"(P.state), "s"(P.tok0), "s"(gridDim.x));\n',
-                    '"s"(P.scale), "s"(P.state), "s"(P.tok0), "s"(gridDim.x));\n  PH_AT(0, ph_entry_);\n  PH_A(1);\n'),
+                   ('"s"(P.scale), "s"(P.state), "s"(gridDim.x));\n',
+                    '"s"(P.scale), "s"(P.state), "s"(gridDim.x));\n  PH_AT(0, ph_entry_);\n  PH_A(1);\n'),
                    ("  const int T = pos + 1;\n", "  asm volatile(\"\" ::\"s\"(pos));\n  PH_A(9);\n  const int T = pos + 1;\n"),
                    ("  qkv_s[role][e] = own;\n", "  PH_A(2);\n  qkv_s[role][e] = own;\n"),
                    ("  // ---- RoPE: threads 0..63", "  PH_A(3);\n  // ---- RoPE: threads 0..63"),
-                   ("  if (P.store_kv && blockIdx.x == 0 && tid < HD", "  PH_A(4);\n  if (P.store_kv && blockIdx.x == 0 && tid < HD"),
+                   ("  if (blockIdx.x == 0 && tid < HD", "  PH_A(4);\n  if (blockIdx.x == 0 && tid < HD"),
                    ("  // ---- softmax: max (x[0] first", "  PH_A(5);\n  // ---- softmax: max (x[0] first"),
                    ("  if (sc[0] != sc[0]) mx = sc[0];\n  for (int p = tid; p < T; p += 256) sc[p] = (float)exp((double)(sc[p] - mx));\n  if (T <= H128_SUM_DIRECT_N) pad_chain(sc, T);\n  __syncthreads();\n",
                     "  if (sc[0] != sc[0]) mx = sc[0];\n  PH_A(12);\n  for (int p = tid; p < T; p += 256) sc[p] = (float)exp((double)(sc[p] - mx));\n  if (T <= H128_SUM_DIRECT_N) pad_chain(sc, T);\n  __syncthreads();\n  PH_A(13);\n"),
