@@ -427,8 +427,7 @@ def real_formats(tmpdir, im_end, eos, steps: int = 64):
 def qwen3_decode(tmpdir, im_end, eos, steps: int = 64, device_fed_only: bool = False):
     """The Qwen3-1.7B shape (28 layers, hidden 2048, 16/8 heads of 128, FFN
     6144, per-head QK-norm, tied Q8_0 embedding; Q4_K / Q6_K projections),
-    random-init: a 32-token prompt (one forward per token at head_dim 128),
-    then greedy steps timed on the host around synchronous c2h_step calls,
+    random-init: a 32-token prompt (one batched pass), then greedy steps timed on the host around synchronous c2h_step calls,
     as the main line, and device-fed (c2h_time_steps); algorithmic bytes of
     a step at the mean attended position.  device_fed_only: the warm-up and
     timed steps fed on the device only (graph replays without c2h_step, the

@@ -189,7 +189,7 @@ __host__ __device__ inline size_t vq_index(int p, int d, int hd = 64) {
 //   long contexts: k_attn_scores (workgroups over position blocks, one K
 //     row read for all query heads of a group) -> k_attn_softmax (one
 //     workgroup per head, exps in LDS) -> k_attn_av (one workgroup per KV
-//     head and 16-dim slice: two waves run the FMA chains of all the group's
+//     head and 8-dim slice: one wave runs the FMA chains of all the group's
 //     query heads, the others stage the V slice through LDS).
 // At head_dim 128 the forms are k_attn_h128, and k_attn_h128_scores ->
 // k_attn_h128_sav (a workgroup per query head and 16 output dims: softmax, FMA

@@ -525,7 +525,8 @@ __device__ const double kExp2Frac[EXP_TAB] = {
     0x1.b7f76f2fb5e47p+0, 0x1.c199bdd85529cp+0, 0x1.cb720dcef9069p+0, 0x1.d5818dcfba487p+0, 0x1.dfc97337b9b5fp+0,
     0x1.ea4afa2a490dap+0, 0x1.f50765b6e4540p+0};
 
-// f32(exp(f64(t))) of the softmax (tensor/ops.go:327-330) for t <= 0 or NaN:
+// f32(exp(f64(t))) of the softmax (tensor/ops.go:327-330) for t <= 0 or NaN,
+// by the table-driven reduction of P. T. P. Tang (ACM TOMS 15, 1989):
 // exp(t) = 2^e 2^(j/32) e^r with n = round(32 t / ln 2) = 32 e + j and
 // |r| <= ln 2 / 64, in f64 (the two-part ln 2 / 32 keeps r exact to a final
 // rounding; the Taylor sum to r^6 is off by 2^-58), rounded once to f32.
@@ -2805,8 +2806,10 @@ template __global__ void k_attn_h128<H128_VCH>(AttnCoreParams);
 //                   makes the max NaN, tensor/ops.go:321-326), f64 exp, the
 //                   sequential f32 sum (exact speculative form), p = e/sum;
 //   k_attn_av       per output dim the FMA chain over p = 0..pos in order,
-//                   run by wave 0 while waves 1..7 stage V quads and
-//                   probabilities through two LDS chunks.
+//                   run by wave 0 while waves 1..3 stage V quads and
+//                   probabilities through three LDS chunks.
+// They also take prompts late in a session, sixteen tokens a launch, where
+// k_pf_attn would leave the GPU to a few workgroups (pf_attn_split).
 
 // In decode (store_kv) the workgroup whose block holds pos stores RoPE(k)
 // and v at pos; a batch has its K/V stored and its q rotated (k_pf_qk)
@@ -3392,7 +3395,7 @@ template __global__ void k_pf_gemm_q50s<MODE_RESID>(PFGemmFParams);
 // SIMD with two waves or more (4.7 with one).  So nothing else is done per
 // product: a lane is a row, its block's quants floats in registers, and x
 // comes through scalar loads (a token's x is the same for every lane), the
-// next chunk of 4 tokens x 8 elements in flight under the current one.
+// next chunk of 2 tokens x 16 elements in flight under the current one.
 // The form before read x from LDS for every two products, which set its
 // pace; the products as outer products on the FP32 matrix unit, which
 // shares the VALU's time, were slower than the multiplies.  300 tokens, a launch:
@@ -3952,7 +3955,11 @@ __global__ void __launch_bounds__(ATT_SAV_THREADS) k_attn_h128_sav(AttnCoreParam
 // tokens up to ~1,900 positions, fewer beyond (pf_attn_tokens).  512 tokens,
 // 14 heads of 64: 20.2 us (31.9 with the same FMAs on the VALU); 400 tokens, 16
 // heads of 128: 25 us; the six passes of a 3,000-token prompt 121 us on
-// average (beyond 1,024 positions three launches per 16 tokens took 42 us).
+// average (beyond 1,024 positions the long-context launches take 42 us per 16
+// tokens).  Few tokens at head_dim 64 late in a session leave most CUs idle
+// here, a chain over T positions being as long for one token: those, and
+// passes whose blocks fall to one token, run the long-context launches
+// (pf_attn_split).
 // Block order: a block's work grows with its last position, so the grid is
 // one-dimensional and runs the blocks from the last (longest) to the first;
 // the dispatcher hands each freed slot the next block.
@@ -4313,11 +4320,11 @@ __device__ __forceinline__ f32x4_t pf_pair_params_q4k(const PFA& A, int lk) {
 // rows x 1 token.  (Q6_K projections run k_pf_gemm_q6.)
 // Bound by the VALU: 14 instructions per (row, token, pair) of the fold in
 // the reference's order and ~4.5 around them; the SIMDs issue one per 4.3
-// clk (91 % busy).  Four waves per SIMD and conflict-free strides of the
-// parameters get it there: with 64-token tiles, 167 registers and every
-// other LDS cycle a conflict it was one per 5.9 clk.  512 tokens, gate|up of
-// the 0.5B shape 42.4 -> 39 us; 400 tokens of the 1.7B shape: gate|up 113 ->
-// 89, q|k 51 -> 38, o 34.7 -> 28 us.
+// clk (91 % busy).  Four waves per SIMD and strides of the parameters that
+// leave a conflict in every fourth LDS cycle get it there: with 64-token
+// tiles, 157 registers and a conflict in every other it was one per 5.9 clk.
+// 512 tokens, gate|up of the 0.5B shape 42.4 -> 39 us; 400 tokens of the 1.7B
+// shape: gate|up 113 -> 89, q|k 51 -> 38, o 34.7 -> 28 us.
 template <int TYPE, int MODE, int TT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_pf_gemm(PFGemmParams P) {
   static_assert(TYPE == T_Q4_K, "Q6_K prefill projections run k_pf_gemm_q6");

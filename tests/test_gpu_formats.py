@@ -78,8 +78,9 @@ def test_real_formats_greedy_stream(real_tiny):
 
 
 def test_real_formats_batched_prefill(real_tiny):
-    # Q5_0 / Q8_0 projections of a token batch (k_pf_gemm_q50, k_pf_gemm_f;
-    # 37 and 21 tokens: partial 16-token tiles) with the K-quant ffn_down on
+    # Q5_0 / Q8_0 projections of a token batch (k_pf_gemm_q50 for gate|up,
+    # k_pf_gemm_q50s for q|k and o, k_pf_gemm_f for v; 37 and 21 tokens:
+    # partial 16-token tiles) with the K-quant ffn_down on
     # MFMA: KV and normX equal sequential ingest
     gf, ctx, orc, _, _ = open_pair(real_tiny, 256)
     rng = np.random.default_rng(81)
@@ -100,10 +101,10 @@ def test_real_formats_batched_prefill(real_tiny):
 
 
 def test_real_formats_prefill_300_tokens(real_tiny):
-    # 300 tokens from position 0: nineteen 16-token tiles of k_pf_gemm_q50
-    # (the last partial, 12 tokens: both staged halves hold padding), attn_v
-    # through k_pf_gemm_f at 4 tokens per workgroup, and the 8-token blocks
-    # of k_pf_attn up to 300 positions
+    # 300 tokens from position 0: nineteen 16-token tiles of k_pf_gemm_q50's
+    # gate|up (the last partial, 12 tokens), 8-token tiles with a row's blocks
+    # over several waves for q|k and o, attn_v through k_pf_gemm_f at 4 tokens
+    # per workgroup, and the 16-token blocks of k_pf_attn up to 300 positions
     gf, ctx, orc, _, _ = open_pair(real_tiny, 512)
     toks = np.random.default_rng(83).integers(0, 4093, 300).astype(np.int32)
     got = ctx.prefill(toks, 0)

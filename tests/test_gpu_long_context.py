@@ -3,8 +3,9 @@ at 512 / 4096 / 32768 positions (GQA 14/2, head_dim 64), then engine.Forward
 and greedy steps through libc2h.so against the oracle on the same cache.
 
 Past the split length (1024 attended positions by default; C2H_ATT_SPLIT
-moves it) decode and prefill attend with the long-context kernels
-(k_attn_scores -> k_attn_softmax -> k_attn_av); both forms reproduce
+moves it) decode attends with the long-context kernels (k_attn_scores ->
+k_attn_softmax -> k_attn_av), and so do prompts there where those are faster
+than k_pf_attn (few tokens at thousands of positions); both forms reproduce
 engine/forward.go:143-155 bit for bit, so every comparison is exact."""
 import os
 
@@ -121,8 +122,9 @@ def test_long_kernels_cross_the_split(tiny_model_path):
 
 
 def test_long_kernels_prefill(tiny_model_path):
-    # 40 prompt tokens after 300 cached positions: long-form attention in
-    # sub-batches of 16 tokens, KV and normX equal to sequential ingest
+    # 40 prompt tokens after 300 cached positions, past the split that decode
+    # goes by (k_pf_attn takes them: the long-context launches are slower
+    # there), KV and normX equal to sequential ingest
     gf, ctx, orc, im_end, eos = open_pair(tiny_model_path, max_ctx=2048, split=64)
     fill_cache(ctx, orc, 300, seed=33)
     rng = np.random.default_rng(34)

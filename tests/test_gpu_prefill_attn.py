@@ -137,8 +137,9 @@ def test_non_finite_token_leaves_earlier_tokens(model):
         ctx.upload(0, "TOKEN_EMBD", G.Q8_0, s.n_vocab, s.n_embd, raw)
 
 
-# k_pf_gemm_q50: 16 tokens per wave; 8, with the blocks of a row whole, in
-# one round of two or four waves, and (4,864 columns) in five rounds
+# k_pf_gemm_q50: 16 tokens per wave; 8, with the blocks of a row whole, in one
+# round of two or four waves, and (4,864 columns) in five rounds.  5 and 100
+# tokens run k_pf_gemm_q50s for q|k and o, 5 with 4,864 columns k_pf_gemm_f.
 @pytest.mark.parametrize("down", [G.Q6_K, G.Q5_0])
 @pytest.mark.parametrize("n", [5, 100, 150, 260])
 def test_q5_0_prompts(down, n, tmp_path):

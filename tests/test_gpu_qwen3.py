@@ -81,8 +81,9 @@ def test_qwen3_greedy_64_steps(qwen3_tiny_path):
 
 
 def test_qwen3_prefill_past_1024_then_steps(qwen3_tiny_path):
-    # c2h_prefill runs one forward graph per token at head_dim 128; past
-    # 1024 attended positions the softmax sum takes the long exact chain
+    # a prompt in three passes (512, 512 and 76 tokens); the steps after it
+    # attend past the split, and past 1,024 positions their softmax sum takes
+    # the longer exact form
     gf, ctx, orc, im_end, eos = open_pair(qwen3_tiny_path, max_ctx=1200)
     rng = np.random.default_rng(7)
     prompt = rng.integers(0, 4096, 1100).astype(np.int32)

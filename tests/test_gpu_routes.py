@@ -1,6 +1,6 @@
 """Prompts and decode steps take, at each size, the kernels that suit it: the
-time of one against that of work the other route would not keep up with, with
-a wide margin on both sides, and bit for bit what one forward per token leaves."""
+time of one against that of like work, with a bound between what the two
+routes measure, and bit for bit what one forward per token leaves."""
 import time
 
 import numpy as np
